@@ -61,7 +61,8 @@ enum {
 /* Message for the last non-zero return on this thread. */
 const char* ls_last_error(void);
 
-/* ABI version (bumped on any signature change or addition). */
+/* ABI version (bumped when an existing signature changes; entry points may be
+ * added under the same version). */
 int ls_abi_version(void);
 
 /* What the runtime reports of a loaded kernel (hipFuncGetAttributes and
@@ -82,7 +83,7 @@ typedef struct LsKernelResources {
  * "sparse_attention_bounds_fp16" (one launch), "combine_splits",
  * "page_index", "page_index_heads", "page_mass", "page_select",
  * "page_bounds_update", "page_bounds_rebuild", "int8_decode_write",
- * "int8_finalize_blocks".  kv_heads: decode kernels pair the heads of an
+ * "int8_finalize_blocks", "int8_prefill_write".  kv_heads: decode kernels pair the heads of an
  * even count in one workgroup; n_rep: the index kernels are specialised on
  * it.  Needs a current HIP device. */
 int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, int has_res,
@@ -353,6 +354,35 @@ int ls_int8_finalize_blocks(const void* data, const int64_t* data_strides, const
                             float* k_zero, const int64_t* ks_strides, int64_t num_blocks,
                             int kv_heads, int head_dim, int page, int asym, float eps, float qmax,
                             float levels, float offset, int recip, void* stream);
+
+/* ls_int8_finalize_blocks with item i read from row rows[i] (int64) of data
+ * [num_rows, 16, H_kv, 128]; rows outside it are skipped.  (The INT8 cache's
+ * full last pages, straight from the residual.) */
+int ls_int8_finalize_rows(const void* data, const int64_t* data_strides, const int64_t* rows,
+                          int64_t num_rows, const int64_t* ids, int n, void* k_pool,
+                          const int64_t* kv_strides, float* k_scale, float* k_zero,
+                          const int64_t* ks_strides, int64_t num_blocks, int kv_heads,
+                          int head_dim, int page, int asym, float eps, float qmax, float levels,
+                          float offset, int recip, void* stream);
+
+/* A prefill chunk's write: K and V [B, H_kv, tokens, 128] fp16 (strides[3] =
+ * (b, h, token)) at the flat slots [B, tokens] int64, each sequence's in token
+ * order (page after page, starting anywhere in its first page).  V is
+ * quantized per (token, head) into v_pool / v_scale (/ v_zero); the K of every
+ * page but the chunk's last is quantized per (block, head, channel) into
+ * k_pool / k_scale (/ k_zero), the rows of the first page before the chunk
+ * taken from row rows[b] of the fp16 residual k_res [num_res, 16, H_kv, 128];
+ * the last page's K goes to that row, zeros past its end.  All pools
+ * contiguous; slots and rows outside them are skipped.  qmax / levels / offset
+ * are K's, v_* V's.  Replaces Int8PagedKVCache.write of a chunk
+ * (cache/int8_paged_cache.py:432-600, :670-758). */
+int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v,
+                          const int64_t* v_strides, const int64_t* slots, const int64_t* rows,
+                          void* k_pool, float* k_scale, float* k_zero, void* v_pool,
+                          float* v_scale, float* v_zero, void* k_res, int64_t num_blocks,
+                          int64_t num_res, int batch, int kv_heads, int tokens, int head_dim,
+                          int page, int asym, float eps, float qmax, float levels, float offset,
+                          int recip, float v_qmax, float v_levels, float v_offset, void* stream);
 
 /* Block-table gather (the paged cache's read path): out [B, length, H_kv,
  * head_dim] (out_strides[3] = (b, token, head)) gets, for token p of

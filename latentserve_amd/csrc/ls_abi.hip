@@ -255,6 +255,7 @@ int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, i
     else if (k == "page_bounds_rebuild") e = ls::sparse_index_resources(5, n_rep, &r);
     else if (k == "int8_decode_write") e = ls::int8_write_resources(0, &r);
     else if (k == "int8_finalize_blocks") e = ls::int8_write_resources(1, &r);
+    else if (k == "int8_prefill_write") e = ls::int8_write_resources(2, &r);
     else return fail(LS_ERR_INVALID, "unknown kernel '%s'", kernel);
     if (e != hipSuccess) return hip_status(e, "ls_kernel_resources");
     out->regs = r.regs;
@@ -849,11 +850,12 @@ int ls_int8_decode_write(const void* k, const int64_t* k_strides, const void* v,
     return hip_status(ls::launch_decode_write(a, (hipStream_t)stream), "ls_int8_decode_write");
 }
 
-int ls_int8_finalize_blocks(const void* data, const int64_t* data_strides, const int64_t* ids,
-                            int n, void* k_pool, const int64_t* kv_strides, float* k_scale,
-                            float* k_zero, const int64_t* ks_strides, int64_t num_blocks,
-                            int kv_heads, int head_dim, int page, int asym, float eps, float qmax,
-                            float levels, float offset, int recip, void* stream) {
+static int finalize_blocks(const void* data, const int64_t* data_strides, const int64_t* rows,
+                           int64_t num_rows, const int64_t* ids, int n, void* k_pool,
+                           const int64_t* kv_strides, float* k_scale, float* k_zero,
+                           const int64_t* ks_strides, int64_t num_blocks, int kv_heads,
+                           int head_dim, int page, int asym, float eps, float qmax, float levels,
+                           float offset, int recip, void* stream, const char* what) {
     if (!data || !data_strides || !ids || !k_pool || !kv_strides || !k_scale || !ks_strides)
         return fail(LS_ERR_INVALID, "null pointer argument");
     if (asym && !k_zero) return fail(LS_ERR_INVALID, "asymmetric quantization needs k_zero");
@@ -871,6 +873,8 @@ int ls_int8_finalize_blocks(const void* data, const int64_t* data_strides, const
     a.sd_n = data_strides[0];
     a.sd_t = data_strides[1];
     a.sd_h = data_strides[2];
+    a.rows = rows;
+    a.num_rows = num_rows;
     a.ids = ids;
     a.k_pool = k_pool;
     a.sp_b = kv_strides[0];
@@ -883,7 +887,81 @@ int ls_int8_finalize_blocks(const void* data, const int64_t* data_strides, const
     a.num_blocks = num_blocks;
     a.N = n;
     a.H = kv_heads;
-    return hip_status(ls::launch_finalize_k(a, (hipStream_t)stream), "ls_int8_finalize_blocks");
+    return hip_status(ls::launch_finalize_k(a, (hipStream_t)stream), what);
+}
+
+int ls_int8_finalize_blocks(const void* data, const int64_t* data_strides, const int64_t* ids,
+                            int n, void* k_pool, const int64_t* kv_strides, float* k_scale,
+                            float* k_zero, const int64_t* ks_strides, int64_t num_blocks,
+                            int kv_heads, int head_dim, int page, int asym, float eps, float qmax,
+                            float levels, float offset, int recip, void* stream) {
+    return finalize_blocks(data, data_strides, nullptr, 0, ids, n, k_pool, kv_strides, k_scale,
+                           k_zero, ks_strides, num_blocks, kv_heads, head_dim, page, asym, eps,
+                           qmax, levels, offset, recip, stream, "ls_int8_finalize_blocks");
+}
+
+int ls_int8_finalize_rows(const void* data, const int64_t* data_strides, const int64_t* rows,
+                          int64_t num_rows, const int64_t* ids, int n, void* k_pool,
+                          const int64_t* kv_strides, float* k_scale, float* k_zero,
+                          const int64_t* ks_strides, int64_t num_blocks, int kv_heads,
+                          int head_dim, int page, int asym, float eps, float qmax, float levels,
+                          float offset, int recip, void* stream) {
+    if (!rows) return fail(LS_ERR_INVALID, "null pointer argument");
+    if (num_rows < 0) return fail(LS_ERR_INVALID, "num_rows must be >= 0");
+    return finalize_blocks(data, data_strides, rows, num_rows, ids, n, k_pool, kv_strides, k_scale,
+                           k_zero, ks_strides, num_blocks, kv_heads, head_dim, page, asym, eps,
+                           qmax, levels, offset, recip, stream, "ls_int8_finalize_rows");
+}
+
+int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v,
+                          const int64_t* v_strides, const int64_t* slots, const int64_t* rows,
+                          void* k_pool, float* k_scale, float* k_zero, void* v_pool,
+                          float* v_scale, float* v_zero, void* k_res, int64_t num_blocks,
+                          int64_t num_res, int batch, int kv_heads, int tokens, int head_dim,
+                          int page, int asym, float eps, float qmax, float levels, float offset,
+                          int recip, float v_qmax, float v_levels, float v_offset, void* stream) {
+    if (!k || !k_strides || !v || !v_strides || !slots || !rows || !k_pool || !k_scale || !v_pool ||
+        !v_scale || !k_res)
+        return fail(LS_ERR_INVALID, "null pointer argument");
+    if (asym && (!k_zero || !v_zero))
+        return fail(LS_ERR_INVALID, "asymmetric quantization needs k_zero and v_zero");
+    if (head_dim != ls::HEAD_DIM) return fail(LS_ERR_INVALID, "head_dim must be 128, got %d", head_dim);
+    if (page != ls::PAGE) return fail(LS_ERR_INVALID, "page (block_size) must be 16, got %d", page);
+    if (batch < 0 || batch > 65535 || kv_heads < 1 || tokens < 0 || num_blocks < 0 || num_res < 0)
+        return fail(LS_ERR_INVALID, "bad batch, kv_heads, tokens, num_blocks or num_res");
+    if (((int64_t)tokens / ls::PAGE + 3) * kv_heads > (1LL << 31) - 1)
+        return fail(LS_ERR_INVALID, "tokens x heads too large for one write");
+    if (!rows_aligned(k, k_strides, 3, 2, 4) || !rows_aligned(v, v_strides, 3, 2, 16) ||
+        !aligned(v_pool, 8) || !aligned(k_pool, 2) || !aligned(k_res, 4) || !aligned(k_scale, 4) ||
+        !aligned(v_scale, 4))
+        return fail(LS_ERR_INVALID, "k rows must be aligned to channel pairs, v rows to 16 bytes");
+    ls::PrefillWriteParams a;
+    if (int rc = quant_args(asym, eps, qmax, levels, offset, recip, a.qk)) return rc;
+    if (int rc = quant_args(asym, eps, v_qmax, v_levels, v_offset, recip, a.qv)) return rc;
+    if (batch == 0 || tokens == 0) return LS_OK;
+    a.k = k;
+    a.sk_b = k_strides[0];
+    a.sk_h = k_strides[1];
+    a.sk_t = k_strides[2];
+    a.v = v;
+    a.sv_b = v_strides[0];
+    a.sv_h = v_strides[1];
+    a.sv_t = v_strides[2];
+    a.slots = slots;
+    a.rows = rows;
+    a.k_pool = k_pool;
+    a.k_scale = k_scale;
+    a.k_zero = k_zero;
+    a.v_pool = v_pool;
+    a.v_scale = v_scale;
+    a.v_zero = v_zero;
+    a.k_res = k_res;
+    a.num_blocks = num_blocks;
+    a.num_res = num_res;
+    a.B = batch;
+    a.H = kv_heads;
+    a.N = tokens;
+    return hip_status(ls::launch_prefill_write(a, (hipStream_t)stream), "ls_int8_prefill_write");
 }
 
 int ls_paged_gather(const void* pool, int elem_bytes, const int64_t* kv_strides, int num_blocks,

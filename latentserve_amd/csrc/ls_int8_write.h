@@ -30,9 +30,31 @@ struct DecodeWriteParams {
     QuantArgs q;
 };
 
+// One prefill chunk of N tokens for each of B sequences.
+struct PrefillWriteParams {
+    const void* k;                 // fp16 [B, H, N, 128]
+    int64_t sk_b, sk_h, sk_t;
+    const void* v;                 // fp16 [B, H, N, 128]
+    int64_t sv_b, sv_h, sv_t;
+    const int64_t* slots;          // [B, N] flat token slots, a sequence's in order
+    const int64_t* rows;           // [B] residual row of each sequence
+    void* k_pool;                  // int8 [num_blocks, 16, H, 128] contiguous
+    float* k_scale;                // [num_blocks, H, 128]
+    float* k_zero;                 // same (asym)
+    void* v_pool;                  // int8 [num_blocks, 16, H, 128] contiguous
+    float* v_scale;                // [num_blocks, 16, H]
+    float* v_zero;                 // same (asym)
+    void* k_res;                   // fp16 [num_res, 16, H, 128] contiguous
+    int64_t num_blocks, num_res;
+    int B, H, N;
+    QuantArgs qk, qv;              // the same kind (asym, recip)
+};
+
 struct FinalizeParams {
     const void* data;              // fp16 [N, 16, H, 128]
     int64_t sd_n, sd_t, sd_h;
+    const int64_t* rows;           // [N] row of data each item reads (NULL: its own)
+    int64_t num_rows;              // data's rows (with rows)
     const int64_t* ids;            // [N] destination block of each
     void* k_pool;                  // int8 [num_blocks, 16, H, 128]
     int64_t sp_b, sp_t, sp_h;
@@ -45,8 +67,9 @@ struct FinalizeParams {
 };
 
 hipError_t launch_decode_write(const DecodeWriteParams& p, hipStream_t stream);
+hipError_t launch_prefill_write(const PrefillWriteParams& p, hipStream_t stream);
 hipError_t launch_finalize_k(const FinalizeParams& p, hipStream_t stream);
-// what: 0 decode_write, 1 finalize_k
+// what: 0 decode_write, 1 finalize_k, 2 prefill_write
 hipError_t int8_write_resources(int what, KernelResources* r);
 
 }  // namespace ls

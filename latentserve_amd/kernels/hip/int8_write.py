@@ -5,7 +5,8 @@ Mirrors the reference's kernels/cuda/int8_write.py: ``eligible`` (:53-58) and
 quantize and scatter, K's scatter into the fp16 last-page residual), plus
 ``finalize_blocks``, the per-block K quantizer of
 Int8PagedKVCache._finalize_blocks (cache/int8_paged_cache.py:670-699), so a
-completed page is quantized on the GPU too.
+completed page is quantized on the GPU too, and ``prefill_write``, a whole
+prefill chunk's write in one launch.
 
 Codes and scales are bit-exact with the reference's torch ops.  Torch
 divides by a Python number differently on the two devices (GPU: times the
@@ -77,14 +78,19 @@ def decode_write(k, v, slots, res_idx, flat_v, flat_v_scale, flat_v_zero, k_res,
 def finalize_blocks(data: torch.Tensor, ids: torch.Tensor, k_pool: torch.Tensor,
                     k_scale: torch.Tensor, k_zero: Optional[torch.Tensor] = None, *,
                     asym: bool, eps: float, qmax: float, levels: float, offset: float,
-                    exact_division: bool = False) -> None:
+                    exact_division: bool = False, rows: Optional[torch.Tensor] = None) -> None:
     """Quantize data [N, 16, H, D] fp16 into k_pool blocks ids [N] (int64):
     one step per (block, head, channel), written to k_scale [nb, H, D] (and
-    the zero point to k_zero when asym).  Ids outside the pool are skipped."""
+    the zero point to k_zero when asym).  Ids outside the pool are skipped.
+    With rows (int64, one an id), item i is data[rows[i]]."""
     if data.dtype != torch.float16 or data.dim() != 4 or data.shape[1] != PAGE \
             or data.shape[-1] != HEAD_DIM or data.stride(-1) != 1:
         raise ValueError("data must be fp16 [N, 16, H, 128] with unit channel stride")
-    n, _, h, d = data.shape
+    _, _, h, d = data.shape
+    n = data.shape[0] if rows is None else ids.shape[0]
+    if rows is not None and (rows.dtype != torch.int64 or rows.shape != (n,)
+                             or rows.stride(0) != 1):
+        raise ValueError("rows must be a unit-stride int64 tensor, one an id")
     if ids.dtype != torch.int64 or ids.dim() != 1 or ids.shape[0] != n or ids.stride(0) != 1:
         raise ValueError("ids must be a unit-stride int64 [N] tensor")
     if k_pool.dtype != torch.int8 or k_pool.shape[1:] != (PAGE, h, d) or k_pool.stride(-1) != 1:
@@ -96,9 +102,62 @@ def finalize_blocks(data: torch.Tensor, ids: torch.Tensor, k_pool: torch.Tensor,
                  or k_zero.stride() != k_scale.stride() or k_zero.dtype != torch.float32):
         raise ValueError("asymmetric quantization needs k_zero shaped and strided as k_scale")
     P, S = _lib.ptr, _lib.strides
-    rc = _lib.lib().ls_int8_finalize_blocks(
-        P(data), S(data, 3), P(ids), n, P(k_pool), S(k_pool, 3), P(k_scale),
+    src = (P(data), S(data, 3)) if rows is None else (P(data), S(data, 3), P(rows), data.shape[0])
+    L = _lib.lib()
+    rc = (L.ls_int8_finalize_blocks if rows is None else L.ls_int8_finalize_rows)(
+        *src, P(ids), n, P(k_pool), S(k_pool, 3), P(k_scale),
         P(k_zero) if asym else None, S(k_scale, 2), nb, h, d, PAGE, int(bool(asym)), float(eps),
         float(qmax), float(levels), float(offset), 0 if exact_division else 1,
         _lib.stream_of(data.device))
-    _lib.check(rc, "ls_int8_finalize_blocks")
+    _lib.check(rc, "ls_int8_finalize_blocks" if rows is None else "ls_int8_finalize_rows")
+
+
+def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v_zero, k_res, *,
+                  asym: bool, k_quant, v_quant, exact_division: bool = False) -> None:
+    """A chunk's k, v [B, H, n, 128] fp16 at flat slots [B, n] int64 (each
+    sequence's in token order): V quantized into v_pool [nb, 16, H, D] /
+    v_scale [nb, 16, H]; K's complete pages into k_pool / k_scale [nb, H, D],
+    its last page to row rows[b] (int64 [B]) of k_res [R, 16, H, D] (where the
+    rows before the chunk in its first page are).  k_quant, v_quant: (eps,
+    qmax, levels, offset).  One launch."""
+    b, h, n, d = k.shape
+    if not (k.is_cuda and v.is_cuda) or k.dtype != torch.float16 or v.dtype != torch.float16 \
+            or d != HEAD_DIM or v.shape != k.shape:
+        raise ValueError("prefill_write: k and v must be fp16 [B, H, n, 128] GPU tensors")
+    if slots.dtype != torch.int64 or slots.shape != (b, n) or not slots.is_contiguous():
+        raise ValueError("slots must be a contiguous int64 [B, n] tensor")
+    if rows.dtype != torch.int64 or rows.dim() != 1 or rows.shape[0] < b or rows.stride(0) != 1:
+        raise ValueError("rows must be a unit-stride int64 [B] tensor")
+    nb = k_pool.shape[0]
+    for t, name, dt, shape in (
+            (k_pool, "k_pool", torch.int8, (nb, PAGE, h, d)),
+            (v_pool, "v_pool", torch.int8, (nb, PAGE, h, d)),
+            (k_scale, "k_scale", torch.float32, (nb, h, d)),
+            (v_scale, "v_scale", torch.float32, (nb, PAGE, h)),
+            (k_res, "k_res", torch.float16, (k_res.shape[0], PAGE, h, d))):
+        if t.dtype != dt or t.shape != shape:
+            raise ValueError(f"{name} must be {dt} {shape}")
+        _contig(t, name)
+    if asym:
+        for t, name, like in ((k_zero, "k_zero", k_scale), (v_zero, "v_zero", v_scale)):
+            if t is None or t.shape != like.shape or t.dtype != torch.float32:
+                raise ValueError(f"asymmetric quantization needs {name} shaped as its scales")
+            _contig(t, name)
+    k, v = _loadable(k, 4), _loadable(v, 16)
+    P, S = _lib.ptr, _lib.strides
+    eps, qmax, levels, offset = k_quant
+    _, v_qmax, v_levels, v_offset = v_quant
+    rc = _lib.lib().ls_int8_prefill_write(
+        P(k), S(k, 3), P(v), S(v, 3), P(slots), P(rows), P(k_pool), P(k_scale),
+        P(k_zero) if asym else None, P(v_pool), P(v_scale), P(v_zero) if asym else None, P(k_res),
+        nb, k_res.shape[0], b, h, n, d, PAGE, int(bool(asym)), eps, qmax, levels, offset,
+        0 if exact_division else 1, v_qmax, v_levels, v_offset, _lib.stream_of(k.device))
+    _lib.check(rc, "ls_int8_prefill_write")
+
+
+def _loadable(t: torch.Tensor, nbytes: int) -> torch.Tensor:
+    """t, or a contiguous copy where its rows are not unit-stride and aligned
+    to the kernel's loads."""
+    ok = t.stride(-1) == 1 and t.data_ptr() % nbytes == 0 \
+        and all(st * 2 % nbytes == 0 for st in t.stride()[:-1])
+    return t if ok else t.clone(memory_format=torch.contiguous_format)

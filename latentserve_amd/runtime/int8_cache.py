@@ -29,10 +29,10 @@ sequence's last page.
   (the reference's deferred finalize, :514-580).
 * ``write`` of one token (decode) is one ``ls_int8_decode_write`` launch:
   V quantized into the pool, K into the residual row.
-* ``write`` of n > 1 tokens (a prefill chunk) quantizes V the same way; K
-  is assembled page by page (the residual's rows for a page the chunk
-  continues), the pages that are complete and not last are quantized into
-  the pool in one launch, and the new last page goes to the residual.
+* ``write`` of n > 1 tokens (a prefill chunk) is one ``ls_int8_prefill_write``
+  launch: V quantized the same way; K assembled page by page (the residual's
+  rows for a page the chunk continues), the pages that are complete and not
+  last quantized into the pool, the new last page to the residual.
 
 Quantization runs on the HIP kernels only (bit-exact with the reference's
 torch ops, tests/test_gpu_int8_write.py); there is no CPU path.
@@ -89,6 +89,7 @@ class Int8PagedKVCache(_PagedBase):
         self._pooled: List[List[int]] = [[0] * spec.max_batch_size
                                          for _ in range(spec.num_layers)]
         self._starts: List[int] = []
+        self._chunk_rows: Optional[torch.Tensor] = None     # residual row a sequence of a chunk
 
     # ---- API of the reference cache ----------------------------------------
     def enable_deferred_finalize(self) -> None:
@@ -149,12 +150,15 @@ class Int8PagedKVCache(_PagedBase):
         if n == 1:
             extra["res_index"] = [s * bs + p % bs for s, p in zip(self._active, starts)]
         self._publish(n, starts, extra)
+        if n != 1:                       # the chunk's residual rows, as its slots: its own copy
+            self._chunk_rows = torch.tensor(self._active, dtype=torch.long, device=self.device)
 
     def _pool_full_last_pages(self, seqs: Sequence[int]) -> None:
         """Quantize each sequence's full last page from the residual (it is
         about to stop being the last page), in every layer where it is not
         pooled yet."""
         bs = self.block_size
+        sent: dict = {}           # the layers' pages are almost always the same: sent once
         for li in range(self.spec.num_layers):
             rows, ids = [], []
             for s in seqs:
@@ -171,23 +175,25 @@ class Int8PagedKVCache(_PagedBase):
                 ids.append(t.blocks[page])
                 self._pooled[li][s] = page + 1
             if rows:
-                idx = torch.tensor(rows, dtype=torch.long, device=self.device)
-                self._quantize_k(li, self._residual[li].index_select(0, idx),
-                                 torch.tensor(ids, dtype=torch.long, device=self.device))
+                key = (tuple(rows), tuple(ids))
+                if key not in sent:
+                    sent[key] = torch.tensor([rows, ids], dtype=torch.long, device=self.device)
+                self._quantize_k(li, self._residual[li], sent[key][1], sent[key][0])
 
-    def _quantize_k(self, layer: int, data: torch.Tensor, ids: torch.Tensor) -> None:
+    def _quantize_k(self, layer: int, data: torch.Tensor, ids: torch.Tensor,
+                    rows: torch.Tensor) -> None:
         from latentserve_amd.kernels.hip import int8_write as iw
 
         eps, qmax, levels, offset = self.k_quant
         iw.finalize_blocks(data, ids, self.k_pool[layer], self.k_scale_pool[layer],
                            self.k_zero_pool[layer] if self.asymmetric else None,
                            asym=self.asymmetric, eps=eps, qmax=qmax, levels=levels,
-                           offset=offset, exact_division=self.exact_division)
+                           offset=offset, exact_division=self.exact_division, rows=rows)
 
     def _quantize_v_and_residual(self, layer: int, k_rows: torch.Tensor, v_rows: torch.Tensor,
                                  slots: torch.Tensor, res_index: torch.Tensor) -> None:
         """V rows quantized into the pool at flat `slots`; K rows copied to
-        the flattened residual at `res_index` (-1: not copied)."""
+        the flattened residual at `res_index`."""
         from latentserve_amd.kernels.hip import int8_write as iw
 
         h, d = self.spec.num_kv_heads, self.spec.head_dim
@@ -211,32 +217,14 @@ class Int8PagedKVCache(_PagedBase):
             self._quantize_v_and_residual(layer_idx, k, v, slots.view(b),
                                           self.inputs.vec["res_index"][:b])
             return
-        # V of every token, no K copy
-        k_tok = k.transpose(1, 2).reshape(b * n, h, 1, d)
-        v_tok = v.transpose(1, 2).reshape(b * n, h, 1, d)
-        skip = torch.full((b * n,), -1, dtype=torch.long, device=k.device)
-        self._quantize_v_and_residual(layer_idx, k_tok, v_tok, slots.reshape(-1), skip)
-        # K page by page
-        bs = self.block_size
-        res = self._residual[layer_idx]
-        full_data, full_ids = [], []
+        from latentserve_amd.kernels.hip import int8_write as iw
+
+        iw.prefill_write(k, v, slots, self._chunk_rows, self.k_pool[layer_idx],
+                         self.k_scale_pool[layer_idx],
+                         self.k_zero_pool[layer_idx] if self.asymmetric else None,
+                         self.v_pool[layer_idx], self.v_scale_pool[layer_idx],
+                         self.v_zero_pool[layer_idx] if self.asymmetric else None,
+                         self._residual[layer_idx], asym=self.asymmetric, k_quant=self.k_quant,
+                         v_quant=self.v_quant, exact_division=self.exact_division)
         for row, s in enumerate(self._active[:b]):
-            start = self._starts[row]
-            first_page, off = divmod(start, bs)
-            end = start + n
-            last_page = (end - 1) // bs
-            pages = last_page - first_page + 1
-            stage = torch.zeros(pages * bs, h, d, dtype=k.dtype, device=k.device)
-            if off:
-                stage[:off] = res[s, :off]
-            stage[off:off + n] = k[row].transpose(0, 1)
-            stage = stage.view(pages, bs, h, d)
-            blocks = self.tables[s].blocks
-            if pages > 1:
-                full_data.append(stage[:pages - 1])
-                full_ids.extend(blocks[first_page:last_page])
-            res[s] = stage[pages - 1]
-            self._pooled[layer_idx][s] = last_page
-        if full_ids:
-            self._quantize_k(layer_idx, torch.cat(full_data),
-                             torch.tensor(full_ids, dtype=torch.long, device=k.device))
+            self._pooled[layer_idx][s] = (self._starts[row] + n - 1) // self.block_size

@@ -1,0 +1,92 @@
+"""A prefill chunk's K/V write, on an MI355X.
+
+* INT8: after chunks that start and end everywhere in a page, the codes, steps
+  and residual equal the oracle's quantizers (bit for bit), K rows before a
+  chunk in its first page coming from the residual.
+"""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+import oracle
+
+torch = pytest.importorskip("torch")
+
+pytestmark = [
+    pytest.mark.gpu,
+    pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU"),
+]
+
+BS = 16
+
+
+def _layout(x, how):
+    """The same values [B, H, n, D] in other memory."""
+    if how == "token-major":                       # a projection's [B, n, H, D]
+        return x.transpose(1, 2).contiguous().transpose(1, 2)
+    if how == "slice":                             # part of a wider fused row
+        wide = torch.zeros(*x.shape[:-1], x.shape[-1] + 64, dtype=x.dtype, device=x.device)
+        wide[..., 32:32 + x.shape[-1]] = x
+        return wide[..., 32:32 + x.shape[-1]]
+    if how == "misaligned":                        # rows 2 elements off 16 bytes
+        flat = torch.zeros(x.numel() + 2, dtype=x.dtype, device=x.device)
+        flat[2:] = x.reshape(-1)
+        return flat[2:].view(x.shape)
+    if how == "strided":                           # channels not adjacent
+        return x.transpose(2, 3).contiguous().transpose(2, 3)
+    return x.contiguous()
+
+
+LAYOUTS = ("head-major", "token-major", "slice", "misaligned", "strided")
+
+
+@pytest.mark.parametrize("asym", [False, True])
+@pytest.mark.parametrize("layout", LAYOUTS)
+@pytest.mark.parametrize("chunks", [(2, 13, 2, 31, 16, 33), (16, 17, 15, 32), (15, 130, 2),
+                                    (1, 15, 48, 1, 1, 3)])
+@pytest.mark.parametrize("h", [1, 3])
+def test_int8_chunks_equal_the_oracle(asym, layout, chunks, h):
+    from latentserve_amd.runtime.int8_cache import Int8PagedKVCache
+    from latentserve_amd.runtime.kv_cache import KVCacheSpec
+    c = Int8PagedKVCache(KVCacheSpec(num_layers=1, num_kv_heads=h, head_dim=128,
+                                     max_batch_size=4, max_seq_len=256, device="cuda"),
+                         asymmetric=asym)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    slots = [3, 1]
+    c.advance(5, slots=[2])                        # another sequence's page first
+    hist = [[], []]
+    for n in chunks:
+        c.advance(n, slots=slots)
+        k, v = (torch.randn(2, h, n, 128, generator=g, device="cuda").half() for _ in range(2))
+        v[0, 0, 0] = 0                             # a row at the scale's floor
+        if n == 1:                                 # the decode write takes unit-stride rows
+            c.write(0, k, v)
+        else:
+            c.write(0, _layout(k, layout), _layout(v, layout))
+        hist[0].append(k)
+        hist[1].append(v)
+    k_all, v_all = (torch.cat(x, dim=2).transpose(1, 2).cpu().numpy() for x in hist)
+    total = k_all.shape[1]
+    last = (total - 1) // BS
+    for i, s in enumerate(slots):
+        t = c.tables[s]
+        at = np.array(t.slots(0, total))
+        codes, step, zero = oracle.quantize_v(np.ascontiguousarray(v_all[i]), asym=asym,
+                                              recip=True)
+        assert np.array_equal(c.v_pool[0].cpu().numpy().reshape(-1, h, 128)[at], codes)
+        assert np.array_equal(c.v_scale_pool[0].cpu().numpy().reshape(-1, h)[at], step)
+        if asym:
+            assert np.array_equal(c.v_zero_pool[0].cpu().numpy().reshape(-1, h)[at], zero)
+        if last:
+            pages = np.ascontiguousarray(k_all[i, :last * BS]).reshape(last, BS, h, 128)
+            codes, step, zero = oracle.quantize_k(pages, asym=asym, recip=True)
+            blk = t.blocks[:last]
+            assert np.array_equal(c.k_pool[0].cpu().numpy()[blk], codes)
+            assert np.array_equal(c.k_scale_pool[0].cpu().numpy()[blk], step)
+            if asym:
+                assert np.array_equal(c.k_zero_pool[0].cpu().numpy()[blk], zero)
+        res = c.residual(0)[s].cpu().numpy()
+        assert np.array_equal(res[:total - last * BS], k_all[i, last * BS:])
+        assert c.pooled_pages(s) == last
