@@ -384,6 +384,19 @@ int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v
                           int page, int asym, float eps, float qmax, float levels, float offset,
                           int recip, float v_qmax, float v_levels, float v_offset, void* stream);
 
+/* New K and V rows to their slots: k / v [B, H_kv, tokens, head_dim]
+ * (strides[3] = (b, h, token)) of elem_bytes-byte elements to flat slot
+ * slots[b, t] (int64 [B, tokens]) of k_pool / v_pool (shared kv_strides[3]);
+ * slots outside the pool are skipped.  With kmin (and kmax, bound_strides as
+ * ls_page_bounds_rebuild; fp16 pools of fewer than 2^31 blocks), every
+ * block's K bounds are rebuilt behind the write.  Replaces
+ * PagedKVCache.write's scatter and rebuild (cache/paged_cache.py). */
+int ls_paged_write(const void* k, const int64_t* k_strides, const void* v,
+                   const int64_t* v_strides, const int64_t* slots, void* k_pool, void* v_pool,
+                   const int64_t* kv_strides, int64_t num_blocks, int elem_bytes, int batch,
+                   int kv_heads, int tokens, int head_dim, int page, void* kmin, void* kmax,
+                   const int64_t* bound_strides, void* stream);
+
 /* Block-table gather (the paged cache's read path): out [B, length, H_kv,
  * head_dim] (out_strides[3] = (b, token, head)) gets, for token p of
  * sequence b, the pool row of flat slot table[b][p / 16] * 16 + p % 16 when
@@ -396,6 +409,14 @@ int ls_paged_gather(const void* pool, int elem_bytes, const int64_t* kv_strides,
                     const int32_t* block_tables, int64_t bt_stride, int max_pages,
                     const int32_t* seq_lens, void* out, const int64_t* out_strides, int batch,
                     int kv_heads, int head_dim, int page, int length, void* stream);
+
+/* ls_paged_gather of the K and the V pool (shared kv_strides and
+ * out_strides) in one launch. */
+int ls_paged_read(const void* k_pool, const void* v_pool, int elem_bytes,
+                  const int64_t* kv_strides, int num_blocks, const int32_t* block_tables,
+                  int64_t bt_stride, int max_pages, const int32_t* seq_lens, void* k_out,
+                  void* v_out, const int64_t* out_strides, int batch, int kv_heads, int head_dim,
+                  int page, int length, void* stream);
 
 /* ---- fused elementwise ops of the decode step ----
  *

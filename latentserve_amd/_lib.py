@@ -87,6 +87,12 @@ _SIGNATURES = {
     "ls_int8_prefill_write": [
         _VP, _I64P, _VP, _I64P, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _VP, _I64, _I64, _I32,
         _I32, _I32, _I32, _I32, _I32, _F32, _F32, _F32, _F32, _I32, _F32, _F32, _F32, _VP],
+    "ls_paged_write": [
+        _VP, _I64P, _VP, _I64P, _VP, _VP, _VP, _I64P, _I64, _I32, _I32, _I32, _I32, _I32, _I32,
+        _VP, _VP, _I64P, _VP],
+    "ls_paged_read": [
+        _VP, _VP, _I32, _I64P, _I32, _VP, _I64, _I32, _VP, _VP, _VP, _I64P, _I32, _I32, _I32,
+        _I32, _I32, _VP],
     "ls_paged_gather": [
         _VP, _I32, _I64P, _I32, _VP, _I64, _I32, _VP, _VP, _I64P, _I32, _I32, _I32, _I32, _I32,
         _VP],

@@ -964,10 +964,64 @@ int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v
     return hip_status(ls::launch_prefill_write(a, (hipStream_t)stream), "ls_int8_prefill_write");
 }
 
-int ls_paged_gather(const void* pool, int elem_bytes, const int64_t* kv_strides, int num_blocks,
-                    const int32_t* block_tables, int64_t bt_stride, int max_pages,
-                    const int32_t* seq_lens, void* out, const int64_t* out_strides, int batch,
-                    int kv_heads, int head_dim, int page, int length, void* stream) {
+int ls_paged_write(const void* k, const int64_t* k_strides, const void* v,
+                   const int64_t* v_strides, const int64_t* slots, void* k_pool, void* v_pool,
+                   const int64_t* kv_strides, int64_t num_blocks, int elem_bytes, int batch,
+                   int kv_heads, int tokens, int head_dim, int page, void* kmin, void* kmax,
+                   const int64_t* bound_strides, void* stream) {
+    if (!k || !k_strides || !v || !v_strides || !slots || !k_pool || !v_pool || !kv_strides)
+        return fail(LS_ERR_INVALID, "null pointer argument");
+    if (elem_bytes != 1 && elem_bytes != 2 && elem_bytes != 4)
+        return fail(LS_ERR_INVALID, "elem_bytes must be 1, 2 or 4, got %d", elem_bytes);
+    if (page != ls::PAGE) return fail(LS_ERR_INVALID, "page (block_size) must be 16, got %d", page);
+    if (head_dim < 1 || (head_dim * elem_bytes) % 16 != 0)
+        return fail(LS_ERR_INVALID, "a head row must be a multiple of 16 bytes (head_dim %d)",
+                    head_dim);
+    if (batch < 0 || batch > 65535 || kv_heads < 1 || tokens < 0 || num_blocks < 0)
+        return fail(LS_ERR_INVALID, "bad batch, kv_heads, tokens or num_blocks");
+    if ((int64_t)tokens * kv_heads * (head_dim * elem_bytes / 16) > (1LL << 31) - 256)
+        return fail(LS_ERR_INVALID, "tokens x heads too large for one write");
+    const size_t e = (size_t)elem_bytes;
+    if (!rows_aligned(k, k_strides, 3, e, 16) || !rows_aligned(v, v_strides, 3, e, 16) ||
+        !rows_aligned(k_pool, kv_strides, 3, e, 16) || !rows_aligned(v_pool, kv_strides, 3, e, 16))
+        return fail(LS_ERR_INVALID, "k, v and pool rows must be 16-byte aligned");
+    if (batch == 0 || tokens == 0) return LS_OK;
+    ls::PagedWriteParams a;
+    const void* src[2] = {k, v};
+    const int64_t* ss[2] = {k_strides, v_strides};
+    for (int z = 0; z < 2; ++z) {
+        a.src[z] = src[z];
+        a.ss_b[z] = ss[z][0];
+        a.ss_h[z] = ss[z][1];
+        a.ss_t[z] = ss[z][2];
+    }
+    a.slots = slots;
+    a.pool[0] = k_pool;
+    a.pool[1] = v_pool;
+    a.sp_b = kv_strides[0];
+    a.sp_t = kv_strides[1];
+    a.sp_h = kv_strides[2];
+    a.num_blocks = num_blocks;
+    a.elem = elem_bytes;
+    a.row_bytes = head_dim * elem_bytes;
+    a.B = batch;
+    a.H = kv_heads;
+    a.N = tokens;
+    if (kmin && elem_bytes != 2) return fail(LS_ERR_INVALID, "bounds are kept of fp16 pools only");
+    if (kmin && num_blocks > (1LL << 31) - 1) return fail(LS_ERR_INVALID, "too many blocks");
+    if (int rc = hip_status(ls::launch_paged_write(a, (hipStream_t)stream), "ls_paged_write"))
+        return rc;
+    if (!kmin) return LS_OK;
+    return ls_page_bounds_rebuild(k_pool, kv_strides, (int)num_blocks, kmin, kmax, bound_strides,
+                                  kv_heads, head_dim, page, stream);
+}
+
+// One pool (v_pool and v_out NULL) or both.
+static int paged_gather(const void* pool, const void* v_pool, int elem_bytes,
+                        const int64_t* kv_strides, int num_blocks, const int32_t* block_tables,
+                        int64_t bt_stride, int max_pages, const int32_t* seq_lens, void* out,
+                        void* v_out, const int64_t* out_strides, int batch, int kv_heads,
+                        int head_dim, int page, int length, void* stream, const char* what) {
     if (!pool || !kv_strides || !block_tables || !seq_lens || !out || !out_strides)
         return fail(LS_ERR_INVALID, "null pointer argument");
     if (elem_bytes != 1 && elem_bytes != 2 && elem_bytes != 4)
@@ -982,11 +1036,14 @@ int ls_paged_gather(const void* pool, int elem_bytes, const int64_t* kv_strides,
     if ((int64_t)length * kv_heads * (head_dim * elem_bytes / 16) > (1LL << 31) - 256)
         return fail(LS_ERR_INVALID, "length x heads too large for one gather");
     if (!rows_aligned(pool, kv_strides, 3, (size_t)elem_bytes, 16) ||
-        !rows_aligned(out, out_strides, 3, (size_t)elem_bytes, 16))
+        !rows_aligned(out, out_strides, 3, (size_t)elem_bytes, 16) || !aligned(v_pool, 16) ||
+        !aligned(v_out, 16))
         return fail(LS_ERR_INVALID, "pool and out rows must be 16-byte aligned");
     if (batch == 0 || length == 0) return LS_OK;
     ls::GatherParams a;
-    a.pool = pool;
+    a.pool[0] = pool;
+    a.pool[1] = v_pool;
+    a.pools = v_pool ? 2 : 1;
     a.sp_b = kv_strides[0];
     a.sp_t = kv_strides[1];
     a.sp_h = kv_strides[2];
@@ -995,7 +1052,8 @@ int ls_paged_gather(const void* pool, int elem_bytes, const int64_t* kv_strides,
     a.sbt_b = bt_stride;
     a.max_pages = max_pages;
     a.seq_lens = seq_lens;
-    a.out = out;
+    a.out[0] = out;
+    a.out[1] = v_out;
     a.so_b = out_strides[0];
     a.so_t = out_strides[1];
     a.so_h = out_strides[2];
@@ -1004,7 +1062,27 @@ int ls_paged_gather(const void* pool, int elem_bytes, const int64_t* kv_strides,
     a.B = batch;
     a.L = length;
     a.H = kv_heads;
-    return hip_status(ls::launch_gather(a, (hipStream_t)stream), "ls_paged_gather");
+    return hip_status(ls::launch_gather(a, (hipStream_t)stream), what);
+}
+
+int ls_paged_gather(const void* pool, int elem_bytes, const int64_t* kv_strides, int num_blocks,
+                    const int32_t* block_tables, int64_t bt_stride, int max_pages,
+                    const int32_t* seq_lens, void* out, const int64_t* out_strides, int batch,
+                    int kv_heads, int head_dim, int page, int length, void* stream) {
+    return paged_gather(pool, nullptr, elem_bytes, kv_strides, num_blocks, block_tables, bt_stride,
+                        max_pages, seq_lens, out, nullptr, out_strides, batch, kv_heads, head_dim,
+                        page, length, stream, "ls_paged_gather");
+}
+
+int ls_paged_read(const void* k_pool, const void* v_pool, int elem_bytes,
+                  const int64_t* kv_strides, int num_blocks, const int32_t* block_tables,
+                  int64_t bt_stride, int max_pages, const int32_t* seq_lens, void* k_out,
+                  void* v_out, const int64_t* out_strides, int batch, int kv_heads, int head_dim,
+                  int page, int length, void* stream) {
+    if (!v_pool || !v_out) return fail(LS_ERR_INVALID, "null pointer argument");
+    return paged_gather(k_pool, v_pool, elem_bytes, kv_strides, num_blocks, block_tables, bt_stride,
+                        max_pages, seq_lens, k_out, v_out, out_strides, batch, kv_heads, head_dim,
+                        page, length, stream, "ls_paged_read");
 }
 
 int ls_rms_norm(const void* x, int64_t x_stride, const void* residual, int64_t res_stride,

@@ -476,18 +476,24 @@ class PagedKVCache(_PagedBase):
     def write(self, layer_idx: int, k: torch.Tensor, v: torch.Tensor, start_pos: int = 0) -> None:
         """Store k, v [B, H_kv, n, D] at the slots the last advance(n) reserved."""
         b, h, n, d = k.shape
+        from latentserve_amd.kernels.hip import paged_write as pw
+
         flat = self._slots_for_write(b, n).reshape(-1)
-        rows_k = k.transpose(1, 2).reshape(b * n, h, d)
-        rows_v = v.transpose(1, 2).reshape(b * n, h, d)
-        self.k_pool[layer_idx].view(-1, h, d).index_copy_(0, flat, rows_k)
-        self.v_pool[layer_idx].view(-1, h, d).index_copy_(0, flat, rows_v)
-        if self.kmin is not None:
+        k_pool, v_pool = self.k_pool[layer_idx], self.v_pool[layer_idx]
+        bounds = None if self.kmin is None else (self.kmin[layer_idx], self.kmax[layer_idx])
+        # a chunk's bounds are rebuilt over the pool by the same call
+        done = pw.write(k, v, flat, k_pool, v_pool, bounds if n != 1 else None)
+        if not done:                # a CPU cache, or rows the kernel's 16-byte loads cannot take
+            rows_k = k.transpose(1, 2).reshape(b * n, h, d)
+            rows_v = v.transpose(1, 2).reshape(b * n, h, d)
+            k_pool.view(-1, h, d).index_copy_(0, flat, rows_k)
+            v_pool.view(-1, h, d).index_copy_(0, flat, rows_v)
+        if bounds is not None and (n == 1 or not done):
             from latentserve_amd.kernels.hip import paged_sparse as ps
             if n == 1:
-                ps.update_bounds(k[:, :, 0], flat, self.kmin[layer_idx], self.kmax[layer_idx])
+                ps.update_bounds(k[:, :, 0], flat, *bounds)
             else:
-                ps.rebuild_bounds(self.k_pool[layer_idx], self.kmin[layer_idx],
-                                  self.kmax[layer_idx])
+                ps.rebuild_bounds(k_pool, *bounds)
 
     def read(self, layer_idx: int, batch_size: int, length: Optional[int] = None):
         """[B, H_kv, L, D] K and V of the active sequences (the gather read,
