@@ -173,13 +173,16 @@ def check(rc: int, what: str) -> None:
 
 
 def ptr(t: Optional[torch.Tensor]):
-    return None if t is None else _VP(t.data_ptr())
+    return None if t is None else t.data_ptr()
+
+
+_I64N = [None] + [ctypes.c_int64 * n for n in range(1, 5)]
 
 
 def strides(t: Optional[torch.Tensor], n: int):
     if t is None:
         return None
-    return (ctypes.c_int64 * n)(*t.stride()[:n])
+    return _I64N[n](*t.stride()[:n])
 
 
 class KernelResources(ctypes.Structure):
@@ -202,6 +205,12 @@ def kernel_resources(kernel: str, device: Optional[torch.device] = None, kv_head
     return {name: int(getattr(r, name)) for name, _ in KernelResources._fields_}
 
 
-def stream_of(device: torch.device):
+# (torch.cuda.current_stream(device).cuda_stream builds a Stream object for the
+# same handle: 4 us of a launch's host time)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)    # (None: a torch without GPUs)
+
+
+def stream_of(device: torch.device) -> int:
     """torch's current stream on `device` as a hipStream_t."""
-    return _VP(torch.cuda.current_stream(device).cuda_stream)
+    index = device.index
+    return _raw_stream(torch.cuda.current_device() if index is None else index)

@@ -82,7 +82,7 @@ class PackedWeight:
         self.data = torch.empty(nbytes // 2, dtype=torch.float16, device=weight.device)
         rc = _lib.lib().ls_pack_gemm_weight(weight.data_ptr(), weight.stride(0), n, k,
                                             KINDS[kind], head_dim, self.data.data_ptr(),
-                                            torch.cuda.current_stream(weight.device).cuda_stream)
+                                            _lib.stream_of(weight.device))
         _lib.check(rc, "ls_pack_gemm_weight")
         self.shape = (n, k)
         self.kind = kind
@@ -174,7 +174,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] =
         x2.data_ptr(), x2.stride(0) if m > 1 else k, wptr, wstride, packed,
         None if bias is None else bias.data_ptr(), y.data_ptr(),
         y.stride(0) if m > 1 else n, m, n, k, None if ws is None else ws.data_ptr(), need,
-        *nargs, torch.cuda.current_stream(x.device).cuda_stream)
+        *nargs, _lib.stream_of(x.device))
     _lib.check(rc, "ls_decode_gemm")
     y = y.view(*x.shape[:-1], n)
     return y if ro is None else (y, ro)
@@ -226,7 +226,7 @@ def gate_up_silu(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Ten
         x2.data_ptr(), x2.stride(0) if m > 1 else k, wptr, wstride, packed,
         None if bias is None else bias.data_ptr(), y.data_ptr(),
         y.stride(0) if m > 1 else inter, m, inter, k, *nargs,
-        torch.cuda.current_stream(x.device).cuda_stream)
+        _lib.stream_of(x.device))
     _lib.check(rc, "ls_decode_gate_up_silu")
     y = y.view(*x.shape[:-1], inter)
     return y if ro is None else (y, ro)
@@ -279,6 +279,6 @@ def qkv_rope_write(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.T
     rc = _lib.lib().ls_decode_qkv_rope_write(
         x2.data_ptr(), x2.stride(0) if b > 1 else k, wptr, wstride, packed,
         None if bias is None else bias.data_ptr(), k, *args["pre"], b, hq, hk, d, *nargs,
-        torch.cuda.current_stream(x.device).cuda_stream)
+        _lib.stream_of(x.device))
     _lib.check(rc, "ls_decode_qkv_rope_write")
     return args["q_out"] if ro is None else (args["q_out"], ro)

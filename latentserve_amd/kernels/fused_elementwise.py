@@ -79,7 +79,7 @@ def rope_qk_ref(q, k, cos, sin, hq: int, hk: int, d: int):
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    return _lib.stream_of(t.device)
 
 
 def _fp16_gpu(name: str, t: torch.Tensor) -> None:

@@ -128,16 +128,14 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
         raise ValueError("slots must be a contiguous int64 [B, n] tensor")
     if rows.dtype != torch.int64 or rows.dim() != 1 or rows.shape[0] < b or rows.stride(0) != 1:
         raise ValueError("rows must be a unit-stride int64 [B] tensor")
-    nb = k_pool.shape[0]
+    nb, nr = k_pool.shape[0], k_res.shape[0]
+    i8, f32 = torch.int8, torch.float32
     for t, name, dt, shape in (
-            (k_pool, "k_pool", torch.int8, (nb, PAGE, h, d)),
-            (v_pool, "v_pool", torch.int8, (nb, PAGE, h, d)),
-            (k_scale, "k_scale", torch.float32, (nb, h, d)),
-            (v_scale, "v_scale", torch.float32, (nb, PAGE, h)),
-            (k_res, "k_res", torch.float16, (k_res.shape[0], PAGE, h, d))):
-        if t.dtype != dt or t.shape != shape:
-            raise ValueError(f"{name} must be {dt} {shape}")
-        _contig(t, name)
+            (k_pool, "k_pool", i8, (nb, PAGE, h, d)), (v_pool, "v_pool", i8, (nb, PAGE, h, d)),
+            (k_scale, "k_scale", f32, (nb, h, d)), (v_scale, "v_scale", f32, (nb, PAGE, h)),
+            (k_res, "k_res", torch.float16, (nr, PAGE, h, d))):
+        if t.dtype != dt or t.shape != shape or not t.is_contiguous():
+            raise ValueError(f"{name} must be contiguous {dt} {shape}")
     if asym:
         for t, name, like in ((k_zero, "k_zero", k_scale), (v_zero, "v_zero", v_scale)):
             if t is None or t.shape != like.shape or t.dtype != torch.float32:
@@ -150,7 +148,7 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
     rc = _lib.lib().ls_int8_prefill_write(
         P(k), S(k, 3), P(v), S(v, 3), P(slots), P(rows), P(k_pool), P(k_scale),
         P(k_zero) if asym else None, P(v_pool), P(v_scale), P(v_zero) if asym else None, P(k_res),
-        nb, k_res.shape[0], b, h, n, d, PAGE, int(bool(asym)), eps, qmax, levels, offset,
+        nb, nr, b, h, n, d, PAGE, int(bool(asym)), eps, qmax, levels, offset,
         0 if exact_division else 1, v_qmax, v_levels, v_offset, _lib.stream_of(k.device))
     _lib.check(rc, "ls_int8_prefill_write")
 
@@ -158,6 +156,6 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
 def _loadable(t: torch.Tensor, nbytes: int) -> torch.Tensor:
     """t, or a contiguous copy where its rows are not unit-stride and aligned
     to the kernel's loads."""
-    ok = t.stride(-1) == 1 and t.data_ptr() % nbytes == 0 \
-        and all(st * 2 % nbytes == 0 for st in t.stride()[:-1])
+    sb, sh, st, sd = t.stride()
+    ok = sd == 1 and not (t.data_ptr() | 2 * (sb | sh | st)) % nbytes
     return t if ok else t.clone(memory_format=torch.contiguous_format)

@@ -398,12 +398,26 @@ class _PagedBase:
             vals["write_slot"] = [self.tables[s].slot(p) for s, p in zip(seqs, starts)]
             self._chunk_slots = None
         else:
-            self._chunk_slots = torch.tensor(
-                [self.tables[s].slots(p, p + n) for s, p in zip(seqs, starts)],
-                dtype=torch.long, device=self.device).reshape(len(seqs), n)
+            self._chunk_slots = torch.from_numpy(
+                self._token_slots(seqs, starts, n)).to(self.device)
         vals.update(extra or {})
         self.inputs.publish(seqs, self.tables, **vals)
         self._batch = len(seqs)
+
+    def _token_slots(self, seqs: Sequence[int], starts: Sequence[int], n: int) -> np.ndarray:
+        """[len(seqs), n] int64 flat slots of tokens start .. start + n - 1 of
+        each sequence, from its pages (a page at a time: BlockTable.slot
+        a token was 0.8 ms of a pass that writes 4 prompts of 2048 tokens)."""
+        bs = self.block_size
+        out = np.empty((len(seqs), n), dtype=np.int64)
+        if n:
+            offs = np.arange(bs, dtype=np.int64)
+            for row, (s, p) in enumerate(zip(seqs, starts)):
+                first = p // bs
+                blocks = np.asarray(self.tables[s].blocks[first:(p + n - 1) // bs + 1], np.int64)
+                p -= first * bs
+                out[row] = (blocks[:, None] * bs + offs).reshape(-1)[p:p + n]
+        return out
 
     def _need(self, b: Optional[int]) -> int:
         if self._batch == 0:
