@@ -20,8 +20,9 @@ struct GemmParams {
     int64_t ldy;
     int M, N, K;
     int vec_y;           // y 8-byte aligned and ldy % 4 == 0: 8-byte stores
-    float* part;         // fp32 partial sums [splits][M][ldp] when splits > 1
-    unsigned* counters;  // arrivals a tile group, zero on entry and on exit
+    float* part;         // fp32 partial tiles when splits > 1 (1 KiB a split, tile and
+                         // column block)
+    unsigned* counters;  // arrivals a tile, zero on entry and on exit
     int splits;          // workgroups a 16-row tile's K is split over
     int epi;             // GEMM_PLAIN, GEMM_GLU: y[M, N/2] = silu(gate) * up of w =
                          // [gate; up], GEMM_ROPE: the fused q/k/v projection's outputs
@@ -57,15 +58,24 @@ hipError_t launch_pack_gemm_weight(const void* w, int64_t ldw, int N, int K, int
 // Splits of K over workgroups for an [M, N, K] product (1: no workspace).
 int decode_gemm_splits(int M, int N, int K);
 // Workspace of a split product: GEMM_COUNTERS arrival counters (one a
-// tile group; the same bytes for every shape, so counters that one call
+// tile; the same bytes for every shape, so counters that one call
 // leaves at zero are never another call's partial sums), then the fp32
 // partials.
-constexpr int GEMM_COUNTERS = 16384;
+constexpr int GEMM_COUNTERS = 65536;
 constexpr size_t GEMM_PART_OFFSET = GEMM_COUNTERS * sizeof(unsigned);
 // Bytes of workspace the product needs (0 when it is not split).
 size_t decode_gemm_workspace_bytes(int M, int N, int K);
-// Tile groups (arrival counters) of the product.
+// Tiles (arrival counters) of the product.
 int decode_gemm_units(int M, int N, int K);
+
+// A workgroup's waves, and the steps of 32 channels a wave takes at most.
+constexpr int GEMM_WAVES = 8;
+constexpr int GEMM_MAX_SPW = 8;
+// The kernels of one epilogue (ls_gemm_plain.hip, ls_gemm_glu.hip,
+// ls_gemm_rope.hip): at most spw (even) steps a wave, grid (groups, splits).
+hipError_t launch_gemm_plain(const GemmParams& p, int spw, dim3 grid, hipStream_t stream);
+hipError_t launch_gemm_glu(const GemmParams& p, int spw, dim3 grid, hipStream_t stream);
+hipError_t launch_gemm_rope(const GemmParams& p, int spw, dim3 grid, hipStream_t stream);
 
 // p.splits and p.part are set by the caller from the two functions above.
 hipError_t launch_decode_gemm(const GemmParams& p, hipStream_t stream);
