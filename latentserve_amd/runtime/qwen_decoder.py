@@ -8,14 +8,14 @@ surroundings (28 layers, hidden 1536, 12 query / 2 KV heads, MLP 8960,
 vocab 151936, tied embeddings, RoPE theta 1e6, q/k/v biases) so a captured
 decode step can be timed on the reference's full-step configuration.  The
 projections run on the HIP weight-streaming GEMM with packed weights up to
-16 rows (hipBLASLt, through torch, above that, where it is faster); the
-MLP activation is in the gate/up GEMM's epilogue, and RoPE + the K/V store
-+ the query fold (GQAAttention.forward's decode branch,
-model/attention/gqa.py:283-344: q [B, 12, 1, D] folded to [B, 2, 6, D],
-the new K/V written first) in the q/k/v GEMM's.  Everything else is HIP
-as well: the embedding lookup inside the first norm, per layer the fused
-norms (residual add folded in) and the paged decode attention, writing
-straight into the output projection's input.
+64 rows (hipBLASLt, through torch, above that); the MLP activation is in
+the gate/up GEMM's epilogue, RoPE + the K/V store + the query fold
+(GQAAttention.forward's decode branch, model/attention/gqa.py:283-344: q
+[B, 12, 1, D] folded to [B, 2, 6, D], the new K/V written first) in the
+q/k/v GEMM's, and up to 16 rows the norms (residual add folded in) in the
+prologue of the projection behind them.  Everything else is HIP as well:
+the embedding lookup inside the first norm, the norms above 16 rows and the
+paged decode attention, writing straight into the output projection's input.
 """
 
 from __future__ import annotations
@@ -35,10 +35,14 @@ from latentserve_amd.runtime.int8_cache import Int8PagedKVCache
 from latentserve_amd.runtime.kv_cache import KVCacheSpec, PagedKVCache
 
 
-# Rows up to which the projections take the HIP GEMM (measured: at 1 and 16
-# rows it streams the weights 1.3-2.7x faster than hipBLASLt; at 64 rows
-# hipBLASLt is faster).
+# Rows up to which a norm folds into the projection behind it, and up to which
+# packed weights are the ones to hand to the projections one by one (above, the
+# row-major ones take every launch kind).
 HIP_GEMM_MAX_ROWS = 16
+# Rows up to which the decoder's projections run on the HIP GEMM, which streams
+# the weights faster than hipBLASLt (M 16 / 64, us: gate/up 12.8 against 39 /
+# 17.0 against 20.3, down 10.3 against 21 / 15.1 against 25.4).
+HIP_DECODE_MAX_ROWS = dg.MAX_ROWS
 
 
 def _pack(w: torch.Tensor, kind: str, head_dim: int = 128):
@@ -49,7 +53,7 @@ def _pack(w: torch.Tensor, kind: str, head_dim: int = 128):
 def _linear(x: torch.Tensor, w: torch.Tensor, pw=None,
             b: Optional[torch.Tensor] = None) -> torch.Tensor:
     wk = pw if pw is not None else w
-    if x.shape[0] <= HIP_GEMM_MAX_ROWS and dg.supports(x, wk):
+    if x.shape[0] <= HIP_DECODE_MAX_ROWS and dg.supports(x, wk):
         return dg.linear(x, wk, b)
     return F.linear(x, w, b)
 
@@ -57,7 +61,7 @@ def _linear(x: torch.Tensor, w: torch.Tensor, pw=None,
 def _norm_folds(x: torch.Tensor, pw) -> bool:
     """Whether the RMSNorm before the projection with packed weight pw can
     run in its prologue: at most 16 rows and K not split over workgroups."""
-    if pw is None or x.shape[0] > 16 or not dg.supports(x, pw):
+    if pw is None or x.shape[0] > HIP_GEMM_MAX_ROWS or not dg.supports(x, pw):
         return False
     n = pw.shape[0]
     return dg.workspace_bytes(x.shape[0], n, pw.shape[1]) == 0
@@ -65,7 +69,9 @@ def _norm_folds(x: torch.Tensor, pw) -> bool:
 
 def _gate_up_silu(x: torch.Tensor, w: torch.Tensor, pw=None) -> torch.Tensor:
     wk = pw if pw is not None else w
-    if x.shape[0] <= HIP_GEMM_MAX_ROWS and dg.supports(x, wk):
+    if x.shape[0] <= HIP_DECODE_MAX_ROWS and dg.supports(x, wk):
+        if wk is pw and dg.workspace_bytes(x.shape[0], *w.shape):
+            wk = w                                   # K splits: the GEMM, then the activation
         return dg.gate_up_silu(x, wk)                # SiLU in the GEMM's epilogue
     return fe.silu_and_mul(F.linear(x, w))
 
@@ -251,7 +257,9 @@ class QwenDecoder:
                     x, wq, layer.b_qkv, pos, self.rope.cos, self.rope.sin, slots,
                     kdst, vdst, hq, hk, q_out=q, kmin=kmin, kmax=kmax,
                     residual=residual, norm_weight=layer.norm1, eps=eps)
-            elif b <= HIP_GEMM_MAX_ROWS and dg.supports(h, wq):
+            elif b <= HIP_DECODE_MAX_ROWS and dg.supports(h, wq):
+                if wq is layer.p_qkv and dg.workspace_bytes(b, *layer.w_qkv.shape):
+                    wq = layer.w_qkv                 # K splits: the GEMM, then the RoPE write
                 dg.qkv_rope_write(h, wq, layer.b_qkv, pos, self.rope.cos, self.rope.sin,
                                   slots, kdst, vdst, hq, hk, q_out=q, kmin=kmin, kmax=kmax)
             else:
@@ -282,11 +290,13 @@ class QwenDecoder:
                                     softmax_scale=self.scale, out=o,
                                     scoring=layer.attn.sparse_scoring)
             x = _linear(o.view(b, hq * hd), layer.w_o, layer.p_o)
-            # (the gate/up projection keeps its norm launch: over its 1120
-            # workgroups the prologue costs more than the launch it saves)
-            h, residual = fe.fused_add_rms_norm(x, residual, layer.norm2, eps)
-            x = _linear(_gate_up_silu(h, layer.w_gate_up, layer.p_gate_up), layer.w_down,
-                        layer.p_down)
+            if _norm_folds(x, layer.p_gate_up):
+                h, residual = dg.gate_up_silu(x, layer.p_gate_up, residual=residual,
+                                              norm_weight=layer.norm2, eps=eps)
+            else:
+                h, residual = fe.fused_add_rms_norm(x, residual, layer.norm2, eps)
+                h = _gate_up_silu(h, layer.w_gate_up, layer.p_gate_up)
+            x = _linear(h, layer.w_down, layer.p_down)
         if _norm_folds(x, self.p_lm_head):
             logits, _ = dg.linear(x, self.p_lm_head, residual=residual, norm_weight=self.norm,
                                   eps=eps)
