@@ -115,6 +115,7 @@ void fill_common(ls::DecodeParams& a, const void* q, const int64_t* q_strides, c
     if (max_seq_len > 0) {
         int pages = (max_seq_len + ls::PAGE - 1) / ls::PAGE;
         pages = pages < max_pages ? pages : max_pages;
+        a.host_pages = pages;
         a.pages_per_split = (pages + num_splits - 1) / num_splits;
     }
     a.counters = counters;

@@ -69,6 +69,9 @@ struct DecodeParams {
     float* work;                       // [B * S, H] records of NR*128 + 32 floats:
                                        // acc[NR][128], m[16] (natural log), l[16]
     int pages_per_split;               // > 0: dense walk partition given by the host
+    int host_pages;                    // pages of the caller's max_seq_len (0: not given)
+    int groups;                        // a launch of fewer groups than B * the caller's
+                                       // splits: the groups a head group (set at launch)
     int32_t* counters;                 // [B * H * COUNTER_STRIDE], zero at rest, reset by
                                        // the kernel
     _Float16* out;

@@ -593,9 +593,8 @@ struct GroupWork {
 // lane_len: seq_lens[lane] (lane < B), loaded by the caller ahead of its
 // page requests (loads return in order, so a length requested after them
 // would wait for the pages).
-__device__ GroupWork deal_groups(const DecodeParams& a, int w_id, int lane, int lane_len) {
-    const int B = a.B, S = a.num_splits;
-    const int W = B * S;
+__device__ GroupWork deal_groups(const DecodeParams& a, int W, int w_id, int lane, int lane_len) {
+    const int B = a.B, S = W / B;
     auto pages_of_len = [&](int len) {
         int p = len > 0 ? (len + PAGE - 1) / PAGE : 0;
         return p < a.max_pages ? p : a.max_pages;
@@ -669,6 +668,96 @@ __device__ GroupWork deal_groups(const DecodeParams& a, int w_id, int lane, int 
     // pending here would make the small-batch path, which this one joins,
     // wait for every outstanding load before its first page request)
     r.len = __shfl(r.len, src);
+    return r;
+}
+
+// The deal where B * S groups would not be resident at once (DEAL 1): the host
+// gives W groups (at least one a sequence), and a group takes at most t pages,
+// t the smallest share with which the sequences need no more than W groups.
+// Groups past their sum have no work (n = 0) and end at once.  The
+// proportional deal above rounds every share down, and with one or two groups
+// a sequence leaves the long ones as they are.  Up to DEAL_MAX_B sequences
+// (DEAL_LENS a lane, in runs); lens: their lengths, loaded by the caller.
+constexpr int DEAL_LENS = 4;
+constexpr int DEAL_MAX_B = DEAL_LENS * WAVE;
+
+__device__ __forceinline__ int ceil_div_small(int p, int t, float inv_t) {
+    // p < 2^24 and a quotient in the hundreds: the estimate is off by one at most
+    int q = (int)((float)p * inv_t);
+    int r = p - q * t;
+    q += r >= t ? 1 : r < 0 ? -1 : 0;
+    r = p - q * t;
+    return q + (r > 0 ? 1 : 0);
+}
+
+__device__ GroupWork deal_smallest_share(const DecodeParams& a, int W, int w_id, int lane,
+                                         const int (&lens)[DEAL_LENS]) {
+    const int B = a.B, per_lane = (B + WAVE - 1) / WAVE;
+    int p[DEAL_LENS];
+    int sum = 0, most = 1;
+#pragma unroll
+    for (int j = 0; j < DEAL_LENS; ++j) {
+        const bool mine = j < per_lane && lane * per_lane + j < B;
+        int pg = mine && lens[j] > 0 ? (lens[j] + PAGE - 1) / PAGE : 0;
+        pg = pg < a.max_pages ? pg : a.max_pages;
+        p[j] = mine ? pg : -1;
+        sum += pg;
+        most = pg > most ? pg : most;
+    }
+    int T;
+    (void)wave_incl_scan_dpp(sum, lane, T);       // (< 2^31: the host's check)
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const int other = __shfl_xor(most, o);
+        most = other > most ? other : most;
+    }
+    // groups of the lane's sequences at a share of t pages
+    auto groups = [&](int t, int (&n)[DEAL_LENS]) {
+        const float inv = 1.f / (float)t;
+        int c = 0;
+#pragma unroll
+        for (int j = 0; j < DEAL_LENS; ++j) {
+            const int q = ceil_div_small(p[j] > 0 ? p[j] : 1, t, inv);
+            n[j] = p[j] < 0 ? 0 : q;
+            c += n[j];
+        }
+        return c;
+    };
+    int lo = (T + W - 1) / W, hi = __builtin_amdgcn_readfirstlane(most), total;
+    lo = lo < 1 ? 1 : lo;
+    int n[DEAL_LENS];
+    while (lo < hi) {
+        const int t = (lo + hi) >> 1;
+        (void)wave_incl_scan_dpp(groups(t, n), lane, total);
+        if (total <= W)
+            hi = t;
+        else
+            lo = t + 1;
+    }
+    const int c = groups(hi, n);
+    int pos = wave_incl_scan_dpp(c, lane, total) - c;
+    GroupWork r = {0, 0, 0, 0, 0};
+    bool found = false;
+#pragma unroll
+    for (int j = 0; j < DEAL_LENS; ++j) {
+        if (!found && w_id >= pos && w_id < pos + n[j]) {
+            found = true;
+            r.len = lens[j];
+            r.b = lane * per_lane + j;
+            r.s = w_id - pos;
+            r.n = n[j];
+            r.first = pos;
+        }
+        pos += n[j];
+    }
+    const unsigned long long who = __ballot(found);
+    if (!who) return {0, 0, 0, 0, 0};             // no work (the same in every lane)
+    const int src = __builtin_ctzll(who);
+    r.len = __builtin_amdgcn_readlane(r.len, src);
+    r.b = __builtin_amdgcn_readlane(r.b, src);
+    r.s = __builtin_amdgcn_readlane(r.s, src);
+    r.n = __builtin_amdgcn_readlane(r.n, src);
+    r.first = __builtin_amdgcn_readlane(r.first, src);
     return r;
 }
 
@@ -804,7 +893,10 @@ __device__ float score_one(const DecodeParams& a, int b, int h, int len, int p) 
 // 2 a page-subset walk whose lists the group selects from page scores;
 // 3 the same with the scores computed by the launch itself, each group
 // scoring its share of its sequence's pages (score_slice).
-template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int NWT, int HG, int ABL = 0>
+// DEAL 1: a dense walk whose a.groups groups a head group are fewer than B *
+// the caller's splits (deal_smallest_share; a.num_splits is the even split
+// they allow, which equal lengths then get).
+template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int NWT, int HG, int ABL = 0, int DEAL = 0>
 // (two waves a SIMD also for the 4-wave groups of odd head counts: the
 // register budget of the 8-wave groups, 256)
 __global__ __launch_bounds__(WAVE* NWT) __attribute__((amdgpu_waves_per_eu(2)))
@@ -849,12 +941,16 @@ void paged_decode_kernel(const DecodeParams a) {
     // 50.3 -> 49.8 us; the page-subset walks measured slower so, c5 50.0 ->
     // 51.2 us, and keep the dispatch order)
     const int L = blockIdx.x + gridDim.x * blockIdx.y;
-    const int wg = SPARSE ? L : xcd_major(L, gridDim.x * gridDim.y);
-    const int h0 = (wg % gridDim.x % n_hg) * HG;
-    const int split = wg % gridDim.x / n_hg;
-    const int hb = wg / gridDim.x;      // the host grid's sequence (speculation)
-    const int g = lane >> 4, c = lane & 15;
+    const int wg = SPARSE || DEAL ? L : xcd_major(L, gridDim.x * gridDim.y);
     const int S = a.num_splits;
+    // (DEAL 1: the grid is a.groups x n_hg; groups past B x S guess the last
+    // sequence, a split it does not have)
+    const int h0 = DEAL ? wg % n_hg * HG : (wg % gridDim.x % n_hg) * HG;
+    const int guess = DEAL ? wg / n_hg / S : 0;
+    // the host grid's sequence (speculation)
+    const int hb = DEAL ? (guess < a.B ? guess : a.B - 1) : wg / gridDim.x;
+    const int split = DEAL ? wg / n_hg - hb * S : wg % gridDim.x / n_hg;
+    const int g = lane >> 4, c = lane & 15;
     // Each head of the group has its own NWH waves (wave wv serves head hw
     // of the pair as its wl-th wave): a wave holds one head's state and
     // query, and both heads' waves walk the same pages at about the same
@@ -897,7 +993,16 @@ void paged_decode_kernel(const DecodeParams a) {
 
     // The lengths the deal reads (one a lane for batches up to 64).
     int lane_len = 0;
-    if (!SPARSE && a.B <= WAVE) lane_len = a.seq_lens[lane < a.B ? lane : 0];
+    if (!DEAL && !SPARSE && a.B <= WAVE) lane_len = a.seq_lens[lane < a.B ? lane : 0];
+    int lens[DEAL_LENS];
+    if constexpr (DEAL) {
+        const int per_lane = (a.B + WAVE - 1) / WAVE;
+#pragma unroll
+        for (int j = 0; j < DEAL_LENS; ++j) {
+            const int i = lane * per_lane + (j < per_lane ? j : 0);
+            lens[j] = a.seq_lens[i < a.B ? i : a.B - 1];
+        }
+    }
 
     // Query operands of the group's heads: row c, channels 32j+8g..+8.
     // Rows past n_rep repeat row 0: their (finite) scores fill MFMA columns
@@ -964,8 +1069,11 @@ void paged_decode_kernel(const DecodeParams a) {
         gw.n = S;
         gw.first = hb * S;
         gw.len = a.seq_lens[hb];
+    } else if constexpr (DEAL) {
+        gw = deal_smallest_share(a, a.groups, hb * S + split, lane, lens);
+        if (gw.n == 0) return;               // (before any barrier, every wave alike)
     } else {
-        gw = deal_groups(a, hb * S + split, lane, lane_len);
+        gw = deal_groups(a, a.B * S, hb * S + split, lane, lane_len);
     }
     const int b = gw.b;
     const int Sb = gw.n;
@@ -1491,23 +1599,52 @@ extern "C" int ls_diag_read_stamps(void* host, size_t bytes) {
 
 constexpr int NWAVES = 4;
 
+// Groups of NWT waves (HG heads) resident at once on the 256 CUs: one of 8
+// waves a CU, two of 4 (both at two waves a SIMD).
+constexpr int RESIDENT_WAVES = 256 * 8;
+
+// Heads in pairs when the head count allows: both halves of every token row
+// are then read together (INT8 too: c4 37.0 -> 35.8 us).  Each wave holds one
+// head's state, so asymmetric INT8's zero points fit as well.
+template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int ABL, int NWT, int HG>
+static hipError_t launch_heads(const DecodeParams& a, hipStream_t stream) {
+    const int n_hg = a.H / HG;
+    const dim3 block(WAVE * NWT);
+    if constexpr (SPARSE == 0 && ABL == 0) {
+        // More groups than can be resident run a second round, whose groups
+        // start as the first's end: the launch then takes two of the first's
+        // times however little is left (B48, lengths to 1531, 8 heads: 384
+        // groups on 256 CUs).  So a launch gets what is resident, or the
+        // fewest whole rounds that give each sequence a group, and the groups
+        // are dealt by the pages (deal_smallest_share).  Measured (us, before
+        // -> after): fp16 B48, lengths to 1531, 8 heads 46.4 -> 37.2 a layer, the
+        // same in INT8 42.9 -> 34.0, B48 x 800 37.2 -> 29.9, B100 to 1000, 2
+        // heads 27.1 -> 18.2.
+        const int64_t fit = RESIDENT_WAVES / NWT;
+        const int64_t asked = (int64_t)a.B * a.num_splits;
+        if (asked * n_hg > fit && a.B <= DEAL_MAX_B &&
+            (int64_t)a.B * a.max_pages < (1LL << 31)) {
+            const int64_t rounds = ((int64_t)a.B * n_hg + fit - 1) / fit;
+            const int64_t most = fit * rounds / n_hg;      // >= B
+            DecodeParams d = a;
+            d.groups = (int)(most < asked ? most : asked);
+            d.num_splits = d.groups / a.B;
+            d.pages_per_split = (a.host_pages + d.num_splits - 1) / d.num_splits;
+            hipLaunchKernelGGL((paged_decode_kernel<KIND, ASYM, HAS_RES, 0, NWT, HG, 0, 1>),
+                               dim3(d.groups * n_hg), block, 0, stream, d);
+            return hipGetLastError();
+        }
+    }
+    hipLaunchKernelGGL((paged_decode_kernel<KIND, ASYM, HAS_RES, SPARSE, NWT, HG, ABL>),
+                       dim3(a.num_splits * n_hg, a.B), block, 0, stream, a);
+    return hipGetLastError();
+}
+
 template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int ABL = 0>
 static hipError_t launch_t(const DecodeParams& a, hipStream_t stream) {
-    // Heads in pairs when the head count allows: both halves of every token
-    // row are then read together (INT8 too: c4 37.0 -> 35.8 us).  Each wave
-    // holds one head's state, so asymmetric INT8's zero points fit as well.
-    if (a.H % 2 == 0) {
-        dim3 grid(a.num_splits * (a.H / 2), a.B);
-        hipLaunchKernelGGL((paged_decode_kernel<KIND, ASYM, HAS_RES, SPARSE, 2 * NWAVES, 2, ABL>),
-                           grid, dim3(WAVE * NWAVES * 2), 0, stream, a);
-        return hipGetLastError();
-    }
-    {
-        dim3 grid(a.num_splits * a.H, a.B);
-        hipLaunchKernelGGL((paged_decode_kernel<KIND, ASYM, HAS_RES, SPARSE, NWAVES, 1, ABL>),
-                           grid, dim3(WAVE * NWAVES), 0, stream, a);
-    }
-    return hipGetLastError();
+    if (a.H % 2 == 0)
+        return launch_heads<KIND, ASYM, HAS_RES, SPARSE, ABL, 2 * NWAVES, 2>(a, stream);
+    return launch_heads<KIND, ASYM, HAS_RES, SPARSE, ABL, NWAVES, 1>(a, stream);
 }
 
 #ifdef LS_DIAGNOSTICS

@@ -49,17 +49,35 @@ def _cus(device: torch.device) -> int:
 
 
 def choose_splits(batch: int, kv_heads: int, num_pages: int,
-                  device: Optional[torch.device] = None, int8: bool = False) -> int:
+                  device: Optional[torch.device] = None, int8: bool = False,
+                  dealt: bool = True) -> int:
     """Splits per (sequence, KV head) for the MI355X kernel.
 
     Enough (sequence, head, split) units for UNITS_PER_4_CUS per 4 CUs (the
     fp16 or the INT8 walk's), never a split of fewer than MIN_SPLIT_PAGES
     pages.  Fixed by (batch, heads, pages, pool type) alone, so a captured
     graph can pin it per context bucket.
+
+    The groups this makes should all be resident at once (a group serves a
+    pair of heads with 8 waves, or one head of an odd count with 4): the count
+    is rounded down to that where at least 4 splits a sequence remain.  With
+    fewer, rounding down would idle up to half of the chip, so the rounded-up
+    count stands and a dense walk's launch deals what fits by the pages.
+    ``dealt=False``: a walk whose launch does not (the page-subset walks).
     """
     cus = _cus(device) if device is not None and torch.cuda.is_available() else 256
     units = UNITS_PER_4_CUS["int8" if int8 else "fp16"] * cus // 4
     by_cus = -(-units // max(1, batch * kv_heads))
+    pairs = kv_heads % 2 == 0
+    head_groups = max(1, batch) * max(1, kv_heads // 2 if pairs else kv_heads)
+    fit = cus if pairs else 2 * cus
+    if head_groups <= fit:
+        whole = fit // head_groups
+        if by_cus > whole and (whole >= 4 or not dealt):
+            by_cus = whole
+    elif dealt:
+        # whole rounds: the groups that fill the last one
+        by_cus = -(-(-(-head_groups // fit) * fit) // head_groups)
     by_pages = max(1, num_pages // MIN_SPLIT_PAGES)
     return max(1, min(MAX_SPLITS, by_cus, by_pages))
 

@@ -246,7 +246,7 @@ def sparse_decode(q, k_pool, v_pool, block_tables, seq_lens, sel,
         raise ValueError("sel must be an int32 [B, H, K] tensor with unit last stride")
     b, h, n_rep, d = q.shape
     num_sel = sel.shape[-1]
-    splits = num_splits or pdh.choose_splits(b, h, num_sel, q.device)
+    splits = num_splits or pdh.choose_splits(b, h, num_sel, q.device, dealt=False)
     splits = max(1, min(splits, max(1, num_sel), pdh.MAX_SPLITS))
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     buf, work, cnt = pdh._buffers("sparse", b, h, splits, n_rep, q.device)
@@ -305,7 +305,7 @@ def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
         raise ValueError(f"selection supports up to {SELECT_MAX_PAGES} pages, "
                          f"got {block_tables.shape[1]}")
     b, h, n_rep, d = q.shape
-    splits = num_splits or pdh.choose_splits(b, h, k, q.device)
+    splits = num_splits or pdh.choose_splits(b, h, k, q.device, dealt=False)
     splits = max(1, min(splits, max(1, k), pdh.MAX_SPLITS))
     splits = max(splits, -(-k // SELECT_SPLIT_ENTRIES))
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
