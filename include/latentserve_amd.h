@@ -236,8 +236,9 @@ int ls_page_scores(const void* q, const int64_t* q_strides, const void* kmin, co
  * Replaces the index + select + attend steps of sparse_attention
  * (kernels/cuda/paged_sparse.py:222-251; page_index, paged_sparse_fp16.cu:
  * 78-130).  k <= max_pages <= 2048 (COOP_MAX_PAGES), n_rep <= 8
- * (COOP_MAX_NREP), ceil(k / num_splits) <= 1024; longer rows or more query
- * rows a KV head take ls_page_scores + ls_sparse_attention_fp16. */
+ * (COOP_MAX_NREP), ceil(k / num_splits) <= 1024; longer rows take
+ * ls_sparse_attention_bounds_long_fp16, more query rows a KV head
+ * ls_page_scores + ls_sparse_attention_fp16. */
 int ls_sparse_attention_bounds_fp16(const void* q, const int64_t* q_strides,
                                     const void* k_pool, const void* v_pool,
                                     const int64_t* kv_strides, int num_blocks,
@@ -251,12 +252,27 @@ int ls_sparse_attention_bounds_fp16(const void* q, const int64_t* q_strides,
                                     int head_dim, int page, int num_splits, int max_seq_len,
                                     float softmax_scale, void* stream);
 
+/* ls_sparse_attention_bounds_fp16 for rows of up to 8192 pages
+ * (COOP_LONG_MAX_PAGES): the same arguments, score buffer and results. */
+int ls_sparse_attention_bounds_long_fp16(const void* q, const int64_t* q_strides,
+                                         const void* k_pool, const void* v_pool,
+                                         const int64_t* kv_strides, int num_blocks,
+                                         const int32_t* block_tables, int64_t bt_stride,
+                                         int max_pages, const int32_t* seq_lens, const void* kmin,
+                                         const void* kmax, const int64_t* bound_strides,
+                                         float* scores, const int64_t* score_strides, int k,
+                                         float ratio, int recent, void* out,
+                                         const int64_t* out_strides, float* workspace,
+                                         int32_t* counters, int batch, int kv_heads, int n_rep,
+                                         int head_dim, int page, int num_splits, int max_seq_len,
+                                         float softmax_scale, void* stream);
+
 /* Test hook, no counterpart in the reference: how long (ticks of the 100 MHz
  * s_memrealtime clock, 5000 = 50 us by default) a workgroup of
- * ls_sparse_attention_bounds_fp16 waits for the other workgroups' page scores
- * before computing the missing ones itself.  Any value gives the same
- * results (the scores are recomputed bit for bit); 0 forces the fallback.
- * Process-wide; read at each call. */
+ * ls_sparse_attention_bounds_fp16 (or _long_fp16) waits for the other
+ * workgroups' page scores before computing the missing ones itself.  Any
+ * value gives the same results (the scores are recomputed bit for bit); 0
+ * forces the fallback.  Process-wide; read at each call. */
 int ls_set_coop_wait_ticks(uint64_t ticks);
 
 /* Bytes of `workspace` ls_page_scores_mass needs: the per-head logits,

@@ -52,6 +52,10 @@ _SIGNATURES = {
         _VP, _I64P, _VP, _VP, _I64P, _I32, _VP, _I64, _I32, _VP, _VP, _VP, _I64P, _VP, _I64P,
         _I32, _F32, _I32, _VP, _I64P, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F32,
         _VP],
+    "ls_sparse_attention_bounds_long_fp16": [
+        _VP, _I64P, _VP, _VP, _I64P, _I32, _VP, _I64, _I32, _VP, _VP, _VP, _I64P, _VP, _I64P,
+        _I32, _F32, _I32, _VP, _I64P, _VP, _VP, _I32, _I32, _I32, _I32, _I32, _I32, _I32, _F32,
+        _VP],
     "ls_paged_decode_int8": [
         _VP, _I64P, _VP, _VP, _I64P, _I32, _VP, _I64P, _VP, _I64P, _VP, _VP,
         _VP, _I64P, _I32, _VP, _VP, _I64, _I32, _VP, _VP, _I64P,

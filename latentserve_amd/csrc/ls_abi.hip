@@ -467,18 +467,18 @@ int ls_sparse_attention_fp16(const void* q, const int64_t* q_strides, const void
     return hip_status(ls::launch_decode(a, (hipStream_t)stream), "ls_sparse_attention_fp16");
 }
 
-int ls_sparse_attention_bounds_fp16(const void* q, const int64_t* q_strides,
-                                    const void* k_pool, const void* v_pool,
-                                    const int64_t* kv_strides, int num_blocks,
-                                    const int32_t* block_tables, int64_t bt_stride,
-                                    int max_pages, const int32_t* seq_lens, const void* kmin,
-                                    const void* kmax, const int64_t* bound_strides,
-                                    float* scores, const int64_t* score_strides, int k,
-                                    float ratio, int recent, void* out,
-                                    const int64_t* out_strides, float* workspace,
-                                    int32_t* counters, int batch, int kv_heads, int n_rep,
-                                    int head_dim, int page, int num_splits, int max_seq_len,
-                                    float softmax_scale, void* stream) {
+// Both one-launch entries: rows of at most `limit` pages.
+static int sparse_attention_bounds(const char* entry, int limit, const void* q,
+                                   const int64_t* q_strides, const void* k_pool,
+                                   const void* v_pool, const int64_t* kv_strides, int num_blocks,
+                                   const int32_t* block_tables, int64_t bt_stride, int max_pages,
+                                   const int32_t* seq_lens, const void* kmin, const void* kmax,
+                                   const int64_t* bound_strides, float* scores,
+                                   const int64_t* score_strides, int k, float ratio, int recent,
+                                   void* out, const int64_t* out_strides, float* workspace,
+                                   int32_t* counters, int batch, int kv_heads, int n_rep,
+                                   int head_dim, int page, int num_splits, int max_seq_len,
+                                   float softmax_scale, void* stream) {
     if (!kmin || !kmax || !bound_strides) return fail(LS_ERR_INVALID, "needs kmin, kmax");
     if (!rows_aligned(kmin, bound_strides, 2, 2, 16) || !rows_aligned(kmax, bound_strides, 2, 2, 16))
         return fail(LS_ERR_INVALID, "kmin/kmax rows must be 16-byte aligned");
@@ -491,9 +491,9 @@ int ls_sparse_attention_bounds_fp16(const void* q, const int64_t* q_strides,
     if (!scores || !score_strides) return fail(LS_ERR_INVALID, "needs the score buffer");
     if (score_strides[1] < (int64_t)max_pages + 1 || score_strides[0] < kv_heads * score_strides[1])
         return fail(LS_ERR_INVALID, "score rows need max_pages + 1 words (a count after each)");
-    if (max_pages > ls::COOP_MAX_PAGES)
+    if (max_pages > limit)
         return fail(LS_ERR_INVALID, "max_pages must be at most %d, got %d",
-                    ls::COOP_MAX_PAGES, max_pages);
+                    limit, max_pages);
     if (n_rep > ls::COOP_MAX_NREP)
         return fail(LS_ERR_INVALID, "n_rep must be at most %d, got %d", ls::COOP_MAX_NREP, n_rep);
     if (k < 0 || k > max_pages)
@@ -520,8 +520,45 @@ int ls_sparse_attention_bounds_fp16(const void* q, const int64_t* q_strides,
     a.num_sel = k;
     a.ratio = ratio;
     a.recent = recent;
-    return hip_status(ls::launch_decode(a, (hipStream_t)stream),
-                      "ls_sparse_attention_bounds_fp16");
+    return hip_status(ls::launch_decode(a, (hipStream_t)stream), entry);
+}
+
+int ls_sparse_attention_bounds_fp16(const void* q, const int64_t* q_strides, const void* k_pool,
+                                    const void* v_pool, const int64_t* kv_strides, int num_blocks,
+                                    const int32_t* block_tables, int64_t bt_stride, int max_pages,
+                                    const int32_t* seq_lens, const void* kmin, const void* kmax,
+                                    const int64_t* bound_strides, float* scores,
+                                    const int64_t* score_strides, int k, float ratio, int recent,
+                                    void* out, const int64_t* out_strides, float* workspace,
+                                    int32_t* counters, int batch, int kv_heads, int n_rep,
+                                    int head_dim, int page, int num_splits, int max_seq_len,
+                                    float softmax_scale, void* stream) {
+    return sparse_attention_bounds("ls_sparse_attention_bounds_fp16", ls::COOP_MAX_PAGES, q,
+                                   q_strides, k_pool, v_pool, kv_strides, num_blocks, block_tables,
+                                   bt_stride, max_pages, seq_lens, kmin, kmax, bound_strides,
+                                   scores, score_strides, k, ratio, recent, out, out_strides,
+                                   workspace, counters, batch, kv_heads, n_rep, head_dim, page,
+                                   num_splits, max_seq_len, softmax_scale, stream);
+}
+
+int ls_sparse_attention_bounds_long_fp16(const void* q, const int64_t* q_strides,
+                                         const void* k_pool, const void* v_pool,
+                                         const int64_t* kv_strides, int num_blocks,
+                                         const int32_t* block_tables, int64_t bt_stride,
+                                         int max_pages, const int32_t* seq_lens, const void* kmin,
+                                         const void* kmax, const int64_t* bound_strides,
+                                         float* scores, const int64_t* score_strides, int k,
+                                         float ratio, int recent, void* out,
+                                         const int64_t* out_strides, float* workspace,
+                                         int32_t* counters, int batch, int kv_heads, int n_rep,
+                                         int head_dim, int page, int num_splits, int max_seq_len,
+                                         float softmax_scale, void* stream) {
+    return sparse_attention_bounds("ls_sparse_attention_bounds_long_fp16", ls::COOP_LONG_MAX_PAGES,
+                                   q, q_strides, k_pool, v_pool, kv_strides, num_blocks,
+                                   block_tables, bt_stride, max_pages, seq_lens, kmin, kmax,
+                                   bound_strides, scores, score_strides, k, ratio, recent, out,
+                                   out_strides, workspace, counters, batch, kv_heads, n_rep,
+                                   head_dim, page, num_splits, max_seq_len, softmax_scale, stream);
 }
 
 int ls_combine_splits(const float* part_acc, const int64_t* acc_strides, const float* part_m,

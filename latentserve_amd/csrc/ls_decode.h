@@ -14,11 +14,13 @@ enum KvKind { KV_FP16 = 0, KV_INT8 = 1 };
 // table (a split's share of the list must fit).
 constexpr int SELECT_SPLIT_ENTRIES = 1024;
 // The one-launch bounds path (each group scores a share of its sequence's
-// pages, then selects from the whole rows): rows of at most COOP_MAX_PAGES
-// pages (eight keys a thread) and at most COOP_MAX_NREP query rows a KV head
-// (their parts and sign masks stay in registers); larger shapes take the
-// index kernel and the two-launch path.
+// pages, then selects from the whole row): rows of at most COOP_MAX_PAGES
+// pages (COOP_LONG_MAX_PAGES by its entry for long rows: 16 keys a thread, the
+// selection's limit) and at most COOP_MAX_NREP query rows a KV head (their
+// parts and sign masks stay in registers); larger shapes take the index
+// kernel and the two-launch path.
 constexpr int COOP_MAX_PAGES = 2048;
+constexpr int COOP_LONG_MAX_PAGES = 8192;
 constexpr int COOP_MAX_NREP = 8;
 
 // Arrival counters are COUNTER_STRIDE int32 apart (one 128-byte line each):

@@ -780,7 +780,8 @@ __device__ __forceinline__ int claimed_item(int raw) { return __builtin_amdgcn_r
 // are requested together, then their bounds (two dependent round trips a
 // batch of R rounds: the caller picks R so that its share is one batch).
 template <int NWT, int HG, int R>
-__device__ void score_slice(const DecodeParams& a, int b, int h0, int len, int p_lo, int p_hi) {
+__device__ __forceinline__ void score_slice(const DecodeParams& a, int b, int h0, int len,
+                                            int p_lo, int p_hi) {
     const int lane = threadIdx.x % WAVE, wv = threadIdx.x / WAVE;
     const int row = lane >> 4, c0 = (lane & 15) * 8;
     const int np = len > 0 ? (len + PAGE - 1) / PAGE : 0;
@@ -843,7 +844,7 @@ __device__ void score_slice(const DecodeParams& a, int b, int h0, int len, int p
 
 // One page's score computed alone by the calling thread (the same sums in
 // the same order as score_slice), for a score that did not arrive in time.
-__device__ float score_one(const DecodeParams& a, int b, int h, int len, int p) {
+__device__ __forceinline__ float score_one(const DecodeParams& a, int b, int h, int len, int p) {
     const int np = len > 0 ? (len + PAGE - 1) / PAGE : 0;
     if (p >= np) return neg_inf();
     if (p == 0 || p >= np - a.recent) return __builtin_inff();
@@ -893,10 +894,11 @@ __device__ float score_one(const DecodeParams& a, int b, int h, int len, int p) 
 // 2 a page-subset walk whose lists the group selects from page scores;
 // 3 the same with the scores computed by the launch itself, each group
 // scoring its share of its sequence's pages (score_slice).
-// DEAL 1: a dense walk whose a.groups groups a head group are fewer than B *
-// the caller's splits (deal_smallest_share; a.num_splits is the even split
-// they allow, which equal lengths then get).
-template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int NWT, int HG, int ABL = 0, int DEAL = 0>
+// VAR, dense walks: 1 for a launch whose a.groups groups a head group are
+// fewer than B * the caller's splits (deal_smallest_share; a.num_splits is the
+// even split they allow, which equal lengths then get).  Selecting walks: the
+// score keys a thread holds.
+template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int NWT, int HG, int ABL = 0, int VAR = 0>
 // (two waves a SIMD also for the 4-wave groups of odd head counts: the
 // register budget of the 8-wave groups, 256)
 __global__ __launch_bounds__(WAVE* NWT) __attribute__((amdgpu_waves_per_eu(2)))
@@ -909,6 +911,7 @@ void paged_decode_kernel(const DecodeParams a) {
     // ran 42.5 us with one page in flight, 43.7 us with two.
     constexpr int PF_DEPTH = 1;
     constexpr int NB = PF_DEPTH + 1;
+    constexpr int DEAL = SPARSE ? 0 : VAR;
     __shared__ DecodeSmem<NWT, HG, KIND == KV_INT8> sm;
     // fp16: the waves' K slots, one array a buffer: the compiler holds an
     // LDS access back until every direct load that may write its object is
@@ -1161,25 +1164,31 @@ void paged_decode_kernel(const DecodeParams a) {
     auto fill_table = [&]() {
         if (!cached) return;
         if constexpr (SPARSE >= 2) {
-            // Each 256-thread half selects its head's list from the page
-            // scores (the selection kernel's radix select; in LDS the merge
-            // buffer holds only after the walk) and keeps the entries of
-            // this split's range, resolved to blocks.  (A threshold
-            // bisection without LDS atomics measured slower, 25 against 10
-            // us for the selection alone: at one wave a SIMD the select is
-            // bound by its dependent instruction latency, and the bisection
-            // has the longer chain.)
-            static_assert(WAVE * NWT == 256 * HG, "one 256-thread group a head");
+            // The group selects its head's list from the page scores (in
+            // LDS the merge buffer holds only after the walk) and keeps the
+            // entries of this split's range, resolved to blocks.  One head a
+            // group: with the pair of heads in one, each selected by 256
+            // threads, a thread held twice the keys and a launch twice the
+            // splits a row to exchange and merge (us, before -> after, 2 heads: B8
+            // x 32K 43.6 -> 39.0, B16 x 16K 40.7 -> 38.6, B2 x 100K at 25 %,
+            // two launches then, 52.8 -> 33.7; 8 heads, B24 to 5000 at 25 %
+            // 51.8 -> 34.5).  (A threshold bisection without LDS atomics
+            // measured slower, 25 against 10 us for the selection alone: at
+            // one wave a SIMD the select is bound by its dependent
+            // instruction latency, and the bisection has the longer chain.)
+            constexpr int THREADS = WAVE * NWT;
+            static_assert(HG == 1, "one head a selecting group");
             static_assert(CAP >= SELECT_SPLIT_ENTRIES, "a split's entries fit the table");
-            const int hh = threadIdx.x / 256, tid = threadIdx.x % 256;
-            static_assert(sizeof(LinSelectSmem) * HG <= sizeof(sm.acc), "selection fits the merge buffer");
-            LinSelectSmem* ssm = reinterpret_cast<LinSelectSmem*>(&sm.acc[0][0][0][0]);
-            const float* row = a.scores + (int64_t)b * a.ssc_b + (int64_t)(h0 + hh) * a.ssc_h;
+            using Smem = LinSelectSmem<THREADS>;
+            static_assert(sizeof(Smem) <= sizeof(sm.acc), "selection fits the merge buffer");
+            Smem& ssm = *reinterpret_cast<Smem*>(&sm.acc[0][0][0][0]);
+            const int tid = threadIdx.x;
+            const float* row = a.scores + (int64_t)b * a.ssc_b + (int64_t)h0 * a.ssc_h;
             // the selection reports pages only; their blocks are looked up
             // below, one independent load a thread (a load per reported page
             // would chain a thread's round trips)
             auto emit = [&](int pos, int pg) {
-                if (pos >= lo && pos < hi) sm.ent[(hh * 2 + 1) * CAP + pos - lo] = pg;
+                if (pos >= lo && pos < hi) sm.ent[CAP + pos - lo] = pg;
             };
             if constexpr (SPARSE == 3) {
                 // this group's share of the sequence's pages scored, then the
@@ -1224,24 +1233,11 @@ void paged_decode_kernel(const DecodeParams a) {
                         }
                     }
                 };
-                const Coop fix{a, b, h0 + hh, len, Sb, done};
-                // (rows of up to COOP_MAX_PAGES pages: eight keys a thread;
-                // up to 1024, four, half the work a thread: B16 x 16K 40.6 ->
-                // 39.5 us.  In this order: with the four-key branch first,
-                // the eight-key rows ran 0.45 us slower, B8 x 32K 42.7 ->
-                // 43.1 us)
-                if (a.score_pages > 4 * 256)
-                    select_row_lin<8, decltype(emit), 1>(row, a.score_pages, n_list, tid, ssm[hh],
-                                                         ssm[0].vote, emit, fix);
-                else
-                    select_row_lin<4, decltype(emit), 1>(row, a.score_pages, n_list, tid, ssm[hh],
-                                                         ssm[0].vote, emit, fix);
+                const Coop fix{a, b, h0, len, Sb, done};
+                select_row_lin<VAR, THREADS, decltype(emit), 1>(row, a.score_pages, n_list, tid,
+                                                                ssm, ssm.vote, emit, fix);
             } else {
-                if (a.score_pages <= 8 * 256)
-                    select_row_lin<8>(row, a.score_pages, n_list, tid, ssm[hh], ssm[0].vote, emit);
-                else
-                    select_row_lin<32>(row, a.score_pages, n_list, tid, ssm[hh], ssm[0].vote,
-                                       emit);
+                select_row_lin<VAR, THREADS>(row, a.score_pages, n_list, tid, ssm, ssm.vote, emit);
             }
             __syncthreads();
             if (SPARSE == 3 && Sb == 1 && threadIdx.x == 0) {
@@ -1640,6 +1636,38 @@ static hipError_t launch_heads(const DecodeParams& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+// The selecting walks: one head a group of 8 waves, the keys a thread holds by
+// the row's length.  The splits are cut to what is resident at once (the
+// one-launch path's groups wait for each other's scores), where a split's
+// entries still fit the table.
+template <int SPARSE>
+static hipError_t launch_selecting(const DecodeParams& a, hipStream_t stream) {
+    constexpr int NWT = 2 * NWAVES, THREADS = WAVE * NWT;
+    DecodeParams d = a;
+    const int fit = (int)(RESIDENT_WAVES / NWT / ((int64_t)a.B * a.H));
+    const int least = (a.num_sel + SELECT_SPLIT_ENTRIES - 1) / SELECT_SPLIT_ENTRIES;
+    int most = fit > least ? fit : least;
+    most = most > 1 ? most : 1;
+    if (d.num_splits > most) d.num_splits = most;
+    const dim3 grid(d.num_splits * a.H, a.B), block(THREADS);
+    const int keys = (a.score_pages + THREADS - 1) / THREADS;
+    if (keys <= 2)
+        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 2>), grid,
+                           block, 0, stream, d);
+    else if (keys <= 4)
+        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 4>), grid,
+                           block, 0, stream, d);
+    else if (keys <= 8)
+        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 8>), grid,
+                           block, 0, stream, d);
+    else if (keys <= 16)
+        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 16>), grid,
+                           block, 0, stream, d);
+    else
+        return hipErrorInvalidValue;
+    return hipGetLastError();
+}
+
 template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int ABL = 0>
 static hipError_t launch_t(const DecodeParams& a, hipStream_t stream) {
     if (a.H % 2 == 0)
@@ -1670,8 +1698,8 @@ static int ablation() {
 #endif
 
 static hipError_t launch_kernel(const DecodeParams& a, hipStream_t stream) {
-    if (a.scores && a.kmin) return launch_t<KV_FP16, false, false, 3>(a, stream);
-    if (a.scores) return launch_t<KV_FP16, false, false, 2>(a, stream);
+    if (a.scores && a.kmin) return launch_selecting<3>(a, stream);
+    if (a.scores) return launch_selecting<2>(a, stream);
     if (a.sel) return launch_t<KV_FP16, false, false, 1>(a, stream);
 #ifdef LS_DIAGNOSTICS
     if (a.kind == KV_FP16 && ablation() != 0) {
@@ -1712,8 +1740,15 @@ hipError_t decode_resources(int kind, int walk, bool asym, bool has_res, bool pa
         switch (walk) {
             case 0: return resources_t<KV_FP16, false, false, 0>(pair_heads, r);
             case 1: return resources_t<KV_FP16, false, false, 1>(pair_heads, r);
-            case 2: return resources_t<KV_FP16, false, false, 2>(pair_heads, r);
-            case 3: return resources_t<KV_FP16, false, false, 3>(pair_heads, r);
+            // (the selecting walks: the keys of rows of up to 2048 pages)
+            case 2:
+                return func_resources(
+                    paged_decode_kernel<KV_FP16, false, false, 2, 2 * NWAVES, 1, 0, 4>,
+                    2 * NWAVES * WAVE, r);
+            case 3:
+                return func_resources(
+                    paged_decode_kernel<KV_FP16, false, false, 3, 2 * NWAVES, 1, 0, 4>,
+                    2 * NWAVES * WAVE, r);
             default: return hipErrorInvalidValue;
         }
     }

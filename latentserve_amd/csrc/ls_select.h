@@ -1,6 +1,6 @@
-// Top-k page selection over a row of page scores, for a group of 256
-// threads: the selection kernel (one group a row) and the selecting decodes'
-// prologues (one group a head of the workgroup).
+// Top-k page selection over a row of page scores, for a group of 256 or 512
+// threads: the selection kernel (one group of 256 a row) and the selecting
+// decodes' prologues (the workgroup of 512).
 //
 // Two searches.  select_row_k, a radix select (8-bit digits, LDS
 // histograms, up to 4 passes: it stops once the threshold digit's bin is
@@ -54,10 +54,10 @@ struct SelectSmem {
     uint32_t pfx[2][4];                // [and, or][wave]
 };
 
-// Inclusive prefix sum over the 256 threads of a group (tid: the thread's
-// index in its group of 256, whose four waves are whole hardware waves):
-// DPP row shifts within each row of 16 lanes, readlane for the rows, the
-// four waves' totals through LDS with one barrier.  `wsum` alternates
+// Inclusive prefix sum over the threads of a group (tid: the thread's index
+// in its group, whose waves are whole hardware waves): DPP row shifts within
+// each row of 16 lanes, readlane for the rows, the waves' totals through LDS
+// with one barrier.  `wsum` alternates
 // between consecutive calls (a thread may write the next call's totals
 // while another still reads this call's).
 __device__ __forceinline__ uint32_t group_scan(uint32_t v, uint32_t* wsum, int tid) {
@@ -118,16 +118,22 @@ __device__ __attribute__((always_inline)) void select_keys(const float* srow, in
             // a 16-byte aligned row: 16-byte device-coherent loads over a
             // resource of the row's P words (lanes past it read zeros);
             // against one 4-byte load a key, B8 x 32K 45.63 -> 45.10 us
-            static_assert(KPT % 4 == 0, "keys in 16-byte pieces");
+            static_assert(KPT == 2 || KPT % 4 == 0, "keys in 8- or 16-byte pieces");
             const __amdgpu_buffer_rsrc_t rs =
                 __builtin_amdgcn_make_buffer_rsrc((void*)srow, 0, P * 4, 0x00020000);
+            if constexpr (KPT == 2) {
+                const uint64_t v = load_coherent8(rs, i0 * 4, 0);
+                f[0] = __builtin_bit_cast(float, (uint32_t)v);
+                f[1] = __builtin_bit_cast(float, (uint32_t)(v >> 32));
+            } else {
 #pragma unroll
-            for (int j = 0; j < KPT; j += 4) {
-                const f4 v = load_coherent4(rs, (i0 + j) * 4);
-                f[j] = v[0];
-                f[j + 1] = v[1];
-                f[j + 2] = v[2];
-                f[j + 3] = v[3];
+                for (int j = 0; j < KPT; j += 4) {
+                    const f4 v = load_coherent4(rs, (i0 + j) * 4);
+                    f[j] = v[0];
+                    f[j + 1] = v[1];
+                    f[j + 2] = v[2];
+                    f[j + 3] = v[3];
+                }
             }
         } else if (done) {
 #pragma unroll
@@ -135,9 +141,16 @@ __device__ __attribute__((always_inline)) void select_keys(const float* srow, in
                 f[j] = P > 0 ? load_coherent(srow + (i0 + j < last ? i0 + j : last)) : 0.f;
         } else {
             // a writer not seen finishing in time: this thread's scores
-            // computed here, none read from the row
+            // computed here, none read from the row (one at a time, by one
+            // copy of the code)
 #pragma unroll
-            for (int j = 0; j < KPT; ++j) f[j] = j < cnt ? fix(i0 + j) : 0.f;
+            for (int j = 0; j < KPT; ++j) f[j] = 0.f;
+#pragma unroll 1
+            for (int t = 0; t < cnt; ++t) {
+                const float v = fix(i0 + t);
+#pragma unroll
+                for (int j = 0; j < KPT; ++j) f[j] = j == t ? v : f[j];
+            }
         }
         LS_STAMP(4);
     } else {
@@ -379,12 +392,14 @@ __device__ __attribute__((always_inline)) void select_row_k(const float* srow, i
 constexpr int LIN_BINS = 2048;
 constexpr int LIN_LIST = 64;            // a threshold bin this small is ranked directly
 
+// THREADS: the group's (256, or 512 with half the keys and bins a thread).
+template <int THREADS>
 struct LinSelectSmem {
     // [round parity][bin]; past the bins, 32 words that take the adds of
     // non-candidate keys (so every lane adds, without a branch)
     uint32_t hist[2][LIN_BINS + 32];
-    uint32_t red[2][2][4];              // [round parity][min, max][wave]
-    uint32_t wsum[2][4];                // group_scan's wave totals
+    uint32_t red[2][2][THREADS / WAVE]; // [round parity][min, max][wave]
+    uint32_t wsum[2][THREADS / WAVE];   // group_scan's wave totals
     int found[2][4];                    // [round parity] bin, taken, its count, outcome
     int list_n;
     int vote[2];                        // [round parity] some group needs another round
@@ -414,9 +429,9 @@ __device__ __forceinline__ uint32_t wave_extreme(uint32_t v) {
 // COOP and `fix` as select_row_k; every group of the workgroup passes the
 // same barriers (the rounds go on while any group needs another: `vote`,
 // two ints in LDS, is the workgroup's, the same for every group).
-template <int KPT, class Emit, int COOP = 0, class Fix = NoFix>
+template <int KPT, int THREADS, class Emit, int COOP = 0, class Fix = NoFix>
 __device__ __attribute__((always_inline)) void select_row_lin(const float* srow, int P, int n,
-                                                              int tid, LinSelectSmem& sm,
+                                                              int tid, LinSelectSmem<THREADS>& sm,
                                                               int* vote, Emit emit,
                                                               Fix fix = Fix()) {
     // (written without per-key branches: selects and bit masks, one branch
@@ -424,8 +439,9 @@ __device__ __attribute__((always_inline)) void select_row_lin(const float* srow,
     // steps measured several times slower, each phase a chain of short
     // divergent blocks)
     static_assert(KPT <= 32, "a thread's keys fit a 32-bit mask");
-    constexpr int BPT = LIN_BINS / SEL_THREADS;           // bins a thread scans
-    static_assert(BPT == 8, "two 16-byte reads a thread");
+    constexpr int BPT = LIN_BINS / THREADS;               // bins a thread scans
+    static_assert(BPT % 4 == 0, "16-byte reads");
+    constexpr int WAVES = THREADS / WAVE;
     constexpr uint32_t KEY_PINF = 0xFF800000u, KEY_NINF = 0x007FFFFFu;
     enum { OPEN = 0, ALL = 1, NONE = 2, PAGE = 3, LIST = 4 };
     const int i0 = tid * KPT;
@@ -438,8 +454,8 @@ __device__ __attribute__((always_inline)) void select_row_lin(const float* srow,
         vote[0] = 0;
     }
     if (tid < LIN_LIST) sm.list_key[tid] = 0u;
-    *(u4*)&sm.hist[0][tid * BPT] = u4{0u, 0u, 0u, 0u};
-    *(u4*)&sm.hist[0][tid * BPT + 4] = u4{0u, 0u, 0u, 0u};
+#pragma unroll
+    for (int j = 0; j < BPT; j += 4) *(u4*)&sm.hist[0][tid * BPT + j] = u4{0u, 0u, 0u, 0u};
     uint32_t key[KPT];
     select_keys<KPT, COOP>(srow, P, tid, i0, cnt, key, fix);
 
@@ -474,11 +490,12 @@ __device__ __attribute__((always_inline)) void select_row_lin(const float* srow,
         // (the other parity's histogram and vote were last read before this
         // barrier)
         if (tid == 0) vote[par ^ 1] = 0;
-        *(u4*)&sm.hist[par ^ 1][tid * BPT] = u4{0u, 0u, 0u, 0u};
-        *(u4*)&sm.hist[par ^ 1][tid * BPT + 4] = u4{0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int j = 0; j < BPT; j += 4)
+            *(u4*)&sm.hist[par ^ 1][tid * BPT + j] = u4{0u, 0u, 0u, 0u};
         uint32_t fmin = sm.red[par][0][0], fmax = sm.red[par][1][0];
 #pragma unroll
-        for (int w = 1; w < 4; ++w) {
+        for (int w = 1; w < WAVES; ++w) {
             fmin = sm.red[par][0][w] < fmin ? sm.red[par][0][w] : fmin;
             fmax = sm.red[par][1][w] > fmax ? sm.red[par][1][w] : fmax;
         }
@@ -497,17 +514,24 @@ __device__ __attribute__((always_inline)) void select_row_lin(const float* srow,
         }
         __syncthreads();
         if (par == 0) LS_STAMP(14);
-        // this thread's bins, highest first: 2047 - 8 tid - j
-        const u4 b_lo = *(const u4*)&sm.hist[par][LIN_BINS - 8 - tid * BPT];
-        const u4 b_hi = *(const u4*)&sm.hist[par][LIN_BINS - 4 - tid * BPT];
-        const uint32_t c[BPT] = {b_hi.w, b_hi.z, b_hi.y, b_hi.x, b_lo.w, b_lo.z, b_lo.y, b_lo.x};
+        // this thread's bins, highest first: 2047 - BPT tid - j
+        uint32_t c[BPT];
+#pragma unroll
+        for (int j = 0; j < BPT; j += 4) {
+            const u4 b = *(const u4*)&sm.hist[par][LIN_BINS - 4 - j - tid * BPT];
+            c[j] = b.w;
+            c[j + 1] = b.z;
+            c[j + 2] = b.y;
+            c[j + 3] = b.x;
+        }
         uint32_t tot = 0;
 #pragma unroll
         for (int j = 0; j < BPT; ++j) tot += c[j];
         const int scan_par = nscan++ & 1;
         const uint32_t incl = group_scan(tot, sm.wsum[scan_par], tid);
-        const uint32_t total = sm.wsum[scan_par][0] + sm.wsum[scan_par][1] +
-                               sm.wsum[scan_par][2] + sm.wsum[scan_par][3];
+        uint32_t total = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) total += sm.wsum[scan_par][w];
         const uint32_t r = (uint32_t)rem;
         uint32_t acc = incl - tot;
         int fj = -1;
@@ -660,20 +684,21 @@ __device__ __attribute__((always_inline)) void select_row(const float* srow, int
 // select_row_lin with the keys a thread holds fitted to the row length.
 template <class Emit>
 __device__ __attribute__((always_inline)) void select_lin(const float* srow, int P, int n, int tid,
-                                                          LinSelectSmem& sm, Emit emit) {
+                                                          LinSelectSmem<SEL_THREADS>& sm,
+                                                          Emit emit) {
     const int kpt = (P + SEL_THREADS - 1) / SEL_THREADS;
     if (kpt <= 1)
-        select_row_lin<1>(srow, P, n, tid, sm, sm.vote, emit);
+        select_row_lin<1, SEL_THREADS>(srow, P, n, tid, sm, sm.vote, emit);
     else if (kpt <= 2)
-        select_row_lin<2>(srow, P, n, tid, sm, sm.vote, emit);
+        select_row_lin<2, SEL_THREADS>(srow, P, n, tid, sm, sm.vote, emit);
     else if (kpt <= 4)
-        select_row_lin<4>(srow, P, n, tid, sm, sm.vote, emit);
+        select_row_lin<4, SEL_THREADS>(srow, P, n, tid, sm, sm.vote, emit);
     else if (kpt <= 8)
-        select_row_lin<8>(srow, P, n, tid, sm, sm.vote, emit);
+        select_row_lin<8, SEL_THREADS>(srow, P, n, tid, sm, sm.vote, emit);
     else if (kpt <= 16)
-        select_row_lin<16>(srow, P, n, tid, sm, sm.vote, emit);
+        select_row_lin<16, SEL_THREADS>(srow, P, n, tid, sm, sm.vote, emit);
     else
-        select_row_lin<32>(srow, P, n, tid, sm, sm.vote, emit);
+        select_row_lin<32, SEL_THREADS>(srow, P, n, tid, sm, sm.vote, emit);
 }
 
 }  // namespace ls

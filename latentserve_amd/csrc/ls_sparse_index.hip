@@ -217,7 +217,7 @@ __global__ __launch_bounds__(256) void page_select_kernel(SelectParams a) {
     if constexpr (!SORTED) {
         // one threshold (the whole list is the budget): the linear-bin search
         // the selecting decode runs
-        __shared__ LinSelectSmem lsm;
+        __shared__ LinSelectSmem<SEL_THREADS> lsm;
         if (n1 == k) {
             select_lin(srow, a.P, n1, (int)threadIdx.x, lsm, emit);
             return;

@@ -6,13 +6,13 @@ Mirrors the reference's kernels/cuda/paged_sparse.py: ``budget`` (:74-78),
 (:185-219) and ``sparse_attention`` (:222-251), all on HIP kernels.
 
 Per layer per decode step ``sparse_attention`` with bounds scoring is one
-launch (ls_sparse_attention_bounds_fp16): the page-subset decode's
-workgroups score their shares of their sequence's pages, exchange the
-scores, and each selects its own list with the selection kernel's radix
-select (the same lists and partition as index + select + sparse_decode).
-Mass scoring, and bounds scoring of rows longer than COOP_MAX_PAGES or of
-more than COOP_MAX_NREP query rows a KV head, are two launches (the scores,
-then ls_sparse_attention_fp16);
+launch (ls_sparse_attention_bounds_fp16, past COOP_MAX_PAGES pages a row
+ls_sparse_attention_bounds_long_fp16): the page-subset decode's workgroups
+score their shares of their sequence's pages, exchange the scores, and each
+selects its own list by the selection kernel's rule (the same lists and
+partition as index + select + sparse_decode).  Mass scoring, and bounds
+scoring of more than COOP_MAX_NREP query rows a KV head, are two launches
+(the scores, then ls_sparse_attention_fp16);
 ``fused=False`` runs the three (index, select, decode).  Nothing syncs with
 the host, so the step is capturable in a HIP graph.
 """
@@ -263,8 +263,9 @@ def sparse_decode(q, k_pool, v_pool, block_tables, seq_lens, sel,
 
 
 SELECT_SPLIT_ENTRIES = 1024    # list entries a selecting group keeps (a split's share)
-# the one-launch bounds path: rows of at most this many pages, at most this
-# many query rows a KV head (else the index kernel, then the selecting decode)
+# the one-launch bounds path: at most this many query rows a KV head (else the
+# index kernel, then the selecting decode); past this many pages a row, its
+# entry for long rows
 COOP_MAX_PAGES = 2048
 COOP_MAX_NREP = 8
 
@@ -305,15 +306,20 @@ def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
         raise ValueError(f"selection supports up to {SELECT_MAX_PAGES} pages, "
                          f"got {block_tables.shape[1]}")
     b, h, n_rep, d = q.shape
-    splits = num_splits or pdh.choose_splits(b, h, k, q.device, dealt=False)
+    # (a selecting group serves one head: as many groups as a pair of heads makes
+    # elsewhere, so the count is asked for twice the heads)
+    splits = num_splits or pdh.choose_splits(b, 2 * h, k, q.device, dealt=False)
     splits = max(1, min(splits, max(1, k), pdh.MAX_SPLITS))
     splits = max(splits, -(-k // SELECT_SPLIT_ENTRIES))
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     buf, work, cnt = pdh._buffers("sparse", b, h, splits, n_rep, q.device)
     target = buf if out is None else pdh.check_out(out, q)
     P, S = _lib.ptr, _lib.strides
-    if (scoring == "bounds" and block_tables.shape[1] <= COOP_MAX_PAGES
-            and n_rep <= COOP_MAX_NREP):
+    short = block_tables.shape[1] <= COOP_MAX_PAGES
+    # (long rows whose bounds cover another number of blocks than the pools:
+    # the index kernel, which takes the bounds' own count)
+    if (scoring == "bounds" and n_rep <= COOP_MAX_NREP
+            and (short or kmin.shape[0] == k_pool.shape[0])):
         # one launch: the decode's workgroups score the pages themselves,
         # exchanging the scores through a buffer whose count words are all
         # ones at rest
@@ -322,13 +328,14 @@ def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
         # (rows padded to 16 bytes, so a row starts 16-byte aligned)
         ws = scratch("sparse_coop_scores", (b, h, (block_tables.shape[1] + 4) // 4 * 4),
                      torch.int32, q.device, init=-1)
-        rc = _lib.lib().ls_sparse_attention_bounds_fp16(
+        entry = "ls_sparse_attention_bounds_fp16" if short else "ls_sparse_attention_bounds_long_fp16"
+        rc = getattr(_lib.lib(), entry)(
             P(q), S(q, 3), P(k_pool), P(v_pool), S(k_pool, 3), k_pool.shape[0],
             P(block_tables), block_tables.stride(0), block_tables.shape[1], P(seq_lens),
             P(kmin), P(kmax), S(kmin, 2), P(ws), S(ws, 2), k, float(ratio), int(recent),
             P(target), S(target, 3), P(work), P(cnt), b, h, n_rep, d, page,
             splits, 0, float(scale), _lib.stream_of(q.device))
-        _lib.check(rc, "ls_sparse_attention_bounds_fp16")
+        _lib.check(rc, entry)
         return buf[:, :, :n_rep] if out is None else out
     if scoring == "mass":
         scores = page_scores_mass(q, kmin, kmax, block_tables, seq_lens, recent, softmax_scale)

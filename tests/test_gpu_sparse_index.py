@@ -490,3 +490,43 @@ def test_one_launch_path_with_the_fallback_forced(width, lens, splits):
             # the word after every row (the count after each head group's
             # first row; untouched after the others)
             assert bool((buf[:, :, width] == -1).all()), "count words not left all ones"
+
+
+@pytest.mark.parametrize("scoring", ["bounds", "mass"])
+@pytest.mark.parametrize("h_kv,width,lens,splits", [
+    (2, 1023, [1023 * 16, 9], 7),                       # two keys a thread, an odd row
+    (1, 1025, [1025 * 16 - 5, 0], None),                # four
+    (3, 2049, [2049 * 16, 40], 200),                    # eight; more splits than are resident
+    (2, 4097, [4097 * 16 - 1, 33000], None),            # sixteen, the list past one split's table
+    (1, 8192, [8192 * 16], 4),                          # the longest row
+])
+def test_selecting_decode_across_the_row_lengths(h_kv, width, lens, splits, scoring):
+    """The selecting decodes either side of each row length at which a thread
+    takes more score keys (one launch for bounds, two for mass) against index +
+    select + list decode over the same scores; twice, and again with the
+    one-launch path's fallback forced."""
+    from latentserve_amd import _lib
+    q, k, v, t, l, kmin, kmax = index_case(lens, width=width, n_rep=4, h_kv=h_kv, seed=width)
+    args = dev(q, k, v, t, l, kmin, kmax)
+    kw = dict(ratio=0.5, scoring=scoring)
+    want = ps().sparse_attention(*args, fused=False, **kw).float()
+    try:
+        for ticks in (5000, 5000, 0):
+            _lib.lib().ls_set_coop_wait_ticks(ticks)
+            got = ps().sparse_attention(*args, num_splits=splits, **kw).float()
+            torch.cuda.synchronize()
+            assert (got - want).abs().max().item() < 1e-3, ticks
+    finally:
+        _lib.lib().ls_set_coop_wait_ticks(5000)
+
+
+def test_long_rows_with_bounds_of_another_block_count():
+    """Rows past COOP_MAX_PAGES whose bounds hold fewer blocks than the pools:
+    pages of blocks past the bounds are left out, as by index + select."""
+    width = 2100
+    q, k, v, t, l, kmin, kmax = index_case([width * 16], width=width, seed=4)
+    nb = len(kmin) - 300
+    args = dev(q, k, v, t, l, kmin[:nb], kmax[:nb])
+    got = ps().sparse_attention(*args, ratio=0.5).float()
+    want = ps().sparse_attention(*args, ratio=0.5, fused=False).float()
+    assert (got - want).abs().max().item() < 1e-3
