@@ -1261,6 +1261,9 @@ int ls_rope_qk(const void* q, int64_t q_stride, const void* k, int64_t k_stride,
     a.hq = hq;
     a.hk = hk;
     a.d = head_dim;
+    a.vec = (q_stride | k_stride | cos_stride | sin_stride | q_out_stride | k_out_stride) % 8 == 0 &&
+            aligned(q, 16) && aligned(k, 16) && aligned(cos, 16) && aligned(sin, 16) &&
+            aligned(q_out, 16) && aligned(k_out, 16);
     return hip_status(ls::launch_rope_qk(a, (hipStream_t)stream), "ls_rope_qk");
 }
 

@@ -75,6 +75,7 @@ struct RopeParams {
     int hq;
     int hk;
     int d;
+    int vec;                  // every row 16-byte aligned
 };
 
 // One decode token per sequence: q/k/v rows of the fused projection output,

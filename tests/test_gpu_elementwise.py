@@ -122,6 +122,32 @@ def test_rope_qk_broadcast_table():
     assert (qo.cpu().numpy() == want.reshape(b, s, hq * d)).all()
 
 
+@pytest.mark.parametrize("rows,hq,hk,d,shift", [
+    (1, 1, 1, 16, 0),            # one 16-byte piece a half
+    (33, 3, 1, 128, 0),
+    (257, 12, 2, 128, 0),        # the last block partly filled
+    (70, 5, 4, 1024, 0),         # the widest head
+    (9, 2, 1, 24, 0),            # a half that is not whole pieces
+    (9, 12, 2, 128, 1),          # rows not 16-byte aligned
+])
+def test_rope_qk_pieces_are_bit_exact(rows, hq, hk, d, shift):
+    rng = np.random.default_rng(rows + d)
+    width = (hq + hk) * d
+    qkv = rng.standard_normal((1, rows, width)).astype(np.float16)
+    buf = torch.zeros(rows * width + 8, dtype=torch.float16, device="cuda")[shift:shift + rows * width]
+    buf.copy_(g(qkv).view(-1))
+    q, k = buf.view(1, rows, width).split([hq * d, hk * d], dim=-1)
+    ang = rng.uniform(0, 6, (1, 1, rows, d // 2))
+    cos = np.cos(np.concatenate([ang, ang], -1)).astype(np.float16)
+    sin = np.sin(np.concatenate([ang, ang], -1)).astype(np.float16)
+    qo, ko = fe().rope_qk(q, k, g(cos), g(sin), hq, hk, d)
+    torch.cuda.synchronize()
+    want = oracle.rope(qkv.reshape(1, rows, hq + hk, d), cos.reshape(1, rows, 1, d),
+                       sin.reshape(1, rows, 1, d)).reshape(1, rows, width)
+    assert (qo.cpu().numpy() == want[..., :hq * d]).all()
+    assert (ko.cpu().numpy() == want[..., hq * d:]).all()
+
+
 @pytest.mark.parametrize("bounds", [False, True])
 def test_rope_write_decode_matches_the_oracle(bounds):
     rng = np.random.default_rng(5)
