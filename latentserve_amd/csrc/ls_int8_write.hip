@@ -68,16 +68,28 @@ __device__ __forceinline__ int8_t code(float x, const QuantStep& s, const QuantA
     return (int8_t)(int)(u - q.offset);
 }
 
-// One wave per (b, h): grid (ceil(B * H / 4)), 256 threads.
+// One wave per (b, h): grid (ceil(B * H / 4)), 256 threads.  A few kilobytes:
+// bound by the launch and by its chain of memory round trips, so everything it
+// reads is requested at once (the residual row, then K, after V's
+// quantization were two trips more: 4.80 -> 4.71 us between two decode
+// launches of a graph, most of them the launch).
 __global__ __launch_bounds__(256) void decode_write_kernel(DecodeWriteParams a) {
     const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= (int64_t)a.B * a.H) return;
-    const int b = (int)(row / a.H), h = (int)(row % a.H);
+    // (B * H rows of 256 bytes in memory: 32 bits hold it, and a 64-bit
+    // division is a hundred instructions)
+    const unsigned row = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const unsigned H = a.H;
+    const int b = (int)(row / H), h = (int)(row % H);
+    if (b >= a.B) return;
     const int d = 2 * lane;
     const h2 vv = *(const h2*)((const half_t*)a.v + (int64_t)b * a.sv_b + (int64_t)h * a.sv_h + d);
-    const float x0 = (float)vv.x, x1 = (float)vv.y;
+    const h2 kk = *(const h2*)((const half_t*)a.k + (int64_t)b * a.sk_b + (int64_t)h * a.sk_h + d);
     const int64_t slot = a.slots[b];
+    const int64_t ri = a.res_idx[b];
+    issue_here();
+    // K into the fp16 residual: its page is quantized when it completes.
+    if (ri >= 0 && ri < a.num_res) *(h2*)((half_t*)a.k_res + (ri * a.H + h) * HEAD_DIM + d) = kk;
+    const float x0 = (float)vv.x, x1 = (float)vv.y;
     if (slot >= 0 && slot < a.num_slots) {
         float amax = 0.f, lo = 0.f, hi = 0.f;
         if (!a.q.asym) {
@@ -97,11 +109,6 @@ __global__ __launch_bounds__(256) void decode_write_kernel(DecodeWriteParams a) 
             if (a.q.asym) a.flat_v_zero[r] = s.zero;
         }
     }
-    // K into the fp16 residual: its page is quantized when it completes.
-    const int64_t ri = a.res_idx[b];
-    if (ri >= 0 && ri < a.num_res)
-        *(h2*)((half_t*)a.k_res + (ri * a.H + h) * HEAD_DIM + d) =
-            *(const h2*)((const half_t*)a.k + (int64_t)b * a.sk_b + (int64_t)h * a.sk_h + d);
 }
 
 // One page of one head's K quantized: two channels a lane (x[token][e]),
