@@ -104,6 +104,10 @@ struct RopeWriteParams {
     int hq;
     int hk;
     int d;
+    // the projection's epilogue (set at its launch): angles and bias by 8-byte
+    // loads at 32-bit offsets, q and K/V by 8-byte stores
+    int ahead = 0;
+    int vec_out = 0;
 };
 
 hipError_t launch_rms_norm(const NormParams& p, hipStream_t stream);

@@ -24,6 +24,8 @@ struct GemmParams {
                          // column block)
     unsigned* counters;  // arrivals a tile, zero on entry and on exit
     int splits;          // workgroups a 16-row tile's K is split over
+    int chunk_pairs = 0; // pairs of 32-channel steps a wave takes (set at launch), one
+    int chunk_more = 0;  // more for the first chunk_more of them
     int epi;             // GEMM_PLAIN, GEMM_GLU: y[M, N/2] = silu(gate) * up of w =
                          // [gate; up], GEMM_ROPE: the fused q/k/v projection's outputs
                          // rotated and stored as `rope` describes (y unused)

@@ -107,12 +107,16 @@ size_t decode_gemm_workspace_bytes(int M, int N, int K) {
     return GEMM_PART_OFFSET + (size_t)splits * ((N + 15) / 16) * ((M + 15) / 16) * WAVE * sizeof(f4);
 }
 
-hipError_t launch_decode_gemm(const GemmParams& p, hipStream_t stream) {
-    if (p.M == 0 || p.N == 0) return hipSuccess;
+hipError_t launch_decode_gemm(const GemmParams& params, hipStream_t stream) {
+    if (params.M == 0 || params.N == 0) return hipSuccess;
+    GemmParams p = params;
     const int steps = p.K / 32, tiles = (p.N + 15) / 16;
     if (p.splits != gemm_splits(p.N, p.K)) return hipErrorInvalidValue;
-    // steps a wave takes at most, in pairs
-    const int spw = 2 * (((steps + 1) / 2 + p.splits * GEMM_WAVES - 1) / (p.splits * GEMM_WAVES));
+    const int pairs = (steps + 1) / 2, chunks = p.splits * GEMM_WAVES;
+    p.chunk_pairs = pairs / chunks;
+    p.chunk_more = pairs % chunks;
+    // steps a wave takes at most
+    const int spw = 2 * (p.chunk_pairs + (p.chunk_more ? 1 : 0));
     if (spw > GEMM_MAX_SPW || p.M > GEMM_MAX_M) return hipErrorInvalidValue;
     // the norm prologue: a packed weight, one column block, a group covering
     // the whole row
@@ -124,6 +128,12 @@ hipError_t launch_decode_gemm(const GemmParams& p, hipStream_t stream) {
     }
     if (p.epi == GEMM_ROPE) {
         if (p.splits != 1 || p.N % 16 != 0 || p.rope.d % 16 != 0) return hipErrorInvalidValue;
+        RopeWriteParams& w = p.rope;
+        const auto at = [](const void* x) { return (uintptr_t)x; };
+        w.ahead = w.st >= 0 && w.st % 2 == 0 && (int64_t)w.tab_rows * w.st < (1LL << 30) - w.d &&
+                  p.N < (1 << 30) && (at(w.cos) | at(w.sin) | at(p.bias)) % 4 == 0;
+        w.vec_out = (at(w.q_out) | at(w.k_pool) | at(w.v_pool)) % 8 == 0 &&
+                    (w.sq_b | w.sq_h | w.sq_r | w.sp_b | w.sp_t | w.sp_h) % 4 == 0;
         return launch_gemm_rope(p, spw, grid, stream);
     }
     return launch_gemm_plain(p, spw, grid, stream);

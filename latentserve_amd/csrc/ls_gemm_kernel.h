@@ -132,11 +132,16 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
     const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x / WAVE), lane = threadIdx.x % WAVE;
     const int r = lane & 15, g = lane >> 4;
     const int steps = a.K >> 5, tiles = (a.N + 15) / 16, G = gridDim.x;
-    // chunk c of nc, in pairs of steps (128 bytes of a weight row)
-    const int c = blockIdx.y * GEMM_WAVES + wv, nc = a.splits * GEMM_WAVES;
-    const int pairs = (steps + 1) / 2;
-    const int s0 = 2 * (int)((int64_t)pairs * c / nc);
-    const int end = 2 * (int)((int64_t)pairs * (c + 1) / nc);
+    // Chunk c of splits x 8, in pairs of steps (128 bytes of a weight row): the
+    // first chunk_more chunks take a pair more than the others' chunk_pairs.
+    // (By the host: as divisions here, 500 instructions of them, they stood
+    // before the first load: M 16, packed, with the norm 2048 x 1536 8.0 -> 7.5
+    // us, gate/up 13.9 -> 13.4; 1536 x 1536 4.2 -> 3.6.)
+    const auto first_step = [&](int c) {
+        return 2 * (c * a.chunk_pairs + (c < a.chunk_more ? c : a.chunk_more));
+    };
+    const int c = blockIdx.y * GEMM_WAVES + wv;
+    const int s0 = first_step(c), end = first_step(c + 1);
     const int ns = (end < steps ? end : steps) - s0;                          // 0..SPW (host)
 
     // W of a tile.  Packed: a step is 1 KiB in the order the lanes take it.
@@ -221,7 +226,7 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
     // 1.5 us a column block at K 1536.  Groups start at different rows and
     // columns, so that the CUs of an XCD do not ask one L2 channel for the
     // same line together.
-    const int S0 = 2 * (int)((int64_t)pairs * (blockIdx.y * GEMM_WAVES) / nc);
+    const int S0 = first_step(blockIdx.y * GEMM_WAVES);
     u4 xb[SPW][MB];
     auto stage = [&](int first) {
 #pragma unroll
@@ -254,6 +259,13 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
                                          (s0 - S0 + (i < ns ? i : 0)) * 64 + 16 * g);
         }
     };
+    // (the largest kernel has no registers for them and loads them late)
+    constexpr bool AHEAD = EPI == GEMM_ROPE && SPW * MB < GEMM_MAX_SPW * GEMM_MAX_M / 16;
+    RopeAhead ra;
+    if constexpr (AHEAD) {
+        rope_row(a, 16 * wv + r, ra);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     stage(0);
     __builtin_amdgcn_sched_barrier(0);
     // the norm prologue's residual rows and weight: the two rows the wave
@@ -276,7 +288,13 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
     }
 #pragma unroll
     for (int u = 0; u < SETS; ++u) load_w(u, blockIdx.x + u * G);
-    wait_vm_lds<SETS * SPW>();           // X has landed, W is on its way
+    if constexpr (AHEAD) {
+        // (the position is here: only X, the norm's operands and W are after it)
+        wait_vm_lds<ROUND * SPW + (NRM ? 3 * PIECES : 0) + SETS * SPW>();
+        rope_tile(a, blockIdx.x, lane, ra);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    wait_vm_lds<SETS * SPW + (AHEAD ? ROPE_TILE_VM : 0)>();  // X has landed, W is on its way
     if constexpr (NRM) {
         // Every group normalises the rows itself, a wave the two it staged.
         // s = res + x in packed fp16 (the fp32 sum of two fp16 values rounds
@@ -372,8 +390,12 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
             f4 s = pt[wv * WAVE + lane];
 #pragma unroll
             for (int p = 1; p < GEMM_WAVES; ++p) s += pt[(p * MB + wv) * WAVE + lane];
+            if constexpr (EPI == GEMM_ROPE && !AHEAD) {
+                rope_row(a, 16 * wv + r, ra);
+                rope_tile(a, tile, lane, ra);
+            }
             if (EPI != GEMM_PLAIN || a.splits == 1) {
-                finish_tile<EPI>(a, tile, wv, lane, s);
+                finish_tile<EPI>(a, tile, wv, lane, s, ra);
             } else {
                 // write-through (sc1), 1 KiB of its own a wave (by a builtin: a
                 // store in inline asm is not counted by the compiler, whose
@@ -385,6 +407,7 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
                                                        16);
             }
         }
+        if constexpr (AHEAD) rope_tile(a, tile + G, lane, ra);
     };
     // (tiles in pairs, a last odd one after the loop: with an exit inside the
     // pair, the compiler merges it with the loop's own and then waits for
@@ -420,7 +443,7 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
         else
             add_partials<8, MB>(a, t, lane, sum);
 #pragma unroll
-        for (int mb = 0; mb < MB; ++mb) finish_tile<EPI>(a, t, mb, lane, sum[mb]);
+        for (int mb = 0; mb < MB; ++mb) finish_tile<EPI>(a, t, mb, lane, sum[mb], ra);
         // back to zero for the next launch
         if (lane == 0)
             __hip_atomic_store(a.counters + t, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -11,13 +11,6 @@
 
 namespace ls {
 
-// Device-coherent (write-through, sc1) 16-byte store: the workgroup that
-// sums a tile's partials may run on another XCD, whose L2 does not see this
-// one's.
-__device__ __forceinline__ void store_through4(float* p, f4 v) {
-    asm volatile("global_store_dwordx4 %0, %1, off sc1" : : "v"(p), "v"(v) : "memory");
-}
-
 // Stores one lane's four outputs y[m][nc .. nc + 3] (fewer at the right
 // edge of a width-n output).
 __device__ __forceinline__ void store_out(const GemmParams& a, int m, int nc, int n,
@@ -63,23 +56,86 @@ __device__ __forceinline__ int w_row(const GemmParams& a, int tile, int r) {
     return w_row_of<EPI>(a.N, a.rope.d, tile, r, real);
 }
 
+// What the q/k/v epilogue reads of a lane's sequence and tile, requested before
+// the tile's sums are known: late, the bias, the position, the angles it
+// names and the slot were four memory round trips in a chain at the end of the
+// launch (M 48, row-major, 2048 x 1536: 8.84 -> 8.43 us).
+struct RopeAhead {
+    int64_t pos, slot;                   // of the lane's sequence
+    u2 c0, c1, s0, s1;                   // angles of its channels, 4 fp16 each
+    u2 b0, b1;                           // their bias
+};
+
+__device__ __forceinline__ void rope_unpack(u2 v, half_t* o) {
+    const h4 t = as_h4(v.x, v.y);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] = t[e];
+}
+
+// The row's position and slot (once a launch).
+__device__ __forceinline__ void rope_row(const GemmParams& a, int m, RopeAhead& ra) {
+    m = m < a.M ? m : a.M - 1;
+    ra.pos = a.rope.pos[m];
+    ra.slot = a.rope.slots[m];
+}
+
+// The angles and bias of a tile's columns (ROPE_TILE_VM loads), by resources (of no bytes without a
+// bias, or where rope.ahead is unset: the epilogue then loads them): no load
+// under a branch, which would make the walk's loads wait.
+constexpr int ROPE_TILE_VM = 6;
+__device__ __forceinline__ void rope_tile(const GemmParams& a, int tile, int lane, RopeAhead& ra) {
+    const RopeWriteParams& w = a.rope;
+    const int tph = w.d / 16, head = tile / tph, i = 8 * (tile % tph) + 4 * ((lane >> 4) & 1);
+    const int64_t p = ra.pos < 0 ? 0 : (ra.pos >= w.tab_rows ? w.tab_rows - 1 : ra.pos);
+    const int bytes = w.ahead ? 0x7fffffff : 0;
+    const uint32_t at = (uint32_t)((p * w.st + i) * 2);
+    const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc((void*)w.cos, 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)w.sin, 0, bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rb =
+        __builtin_amdgcn_make_buffer_rsrc((void*)a.bias, 0, a.bias && w.ahead ? a.N * 2 : 0, 0x00020000);
+    const uint32_t n0 = (uint32_t)(head * w.d + i) * 2;
+    auto ld = [](__amdgpu_buffer_rsrc_t r, uint32_t off) {
+        return __builtin_bit_cast(u2, __builtin_amdgcn_raw_buffer_load_b64(r, off, 0, 0));
+    };
+    ra.c0 = ld(rc, at);
+    ra.c1 = ld(rc, at + w.d);
+    ra.s0 = ld(rs, at);
+    ra.s1 = ld(rs, at + w.d);
+    ra.b0 = ld(rb, n0);
+    ra.b1 = ld(rb, n0 + w.d);
+}
+
 // The fused q/k/v projection's epilogue for one lane: channels i .. i + 3
 // of head `head` (i < d / 2) and their partners i + d / 2 .. for sequence
 // m, as x0 / x1 (fp16, bias added); rotated and stored as
 // rope_write_decode_kernel stores them (the same rounding, bit-equal).
 __device__ __forceinline__ void rope_store(const RopeWriteParams& a, int m, int head, int i,
-                                           const half_t* x0, const half_t* x1) {
+                                           const half_t* x0, const half_t* x1,
+                                           const RopeAhead& ra) {
     const int hd = a.d / 2;
-    int64_t p = a.pos[m];
-    p = p < 0 ? 0 : (p >= a.tab_rows ? a.tab_rows - 1 : p);
-    const half_t* c = (const half_t*)a.cos + p * a.st;
-    const half_t* s = (const half_t*)a.sin + p * a.st;
+    half_t c0[4], c1[4], s0[4], s1[4];
+    rope_unpack(ra.c0, c0);
+    rope_unpack(ra.c1, c1);
+    rope_unpack(ra.s0, s0);
+    rope_unpack(ra.s1, s1);
+    if (!a.ahead) {
+        const int64_t p = ra.pos < 0 ? 0 : (ra.pos >= a.tab_rows ? a.tab_rows - 1 : ra.pos);
+        const half_t* c = (const half_t*)a.cos + p * a.st;
+        const half_t* s = (const half_t*)a.sin + p * a.st;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            c0[e] = c[i + e];
+            c1[e] = c[i + hd + e];
+            s0[e] = s[i + e];
+            s1[e] = s[i + hd + e];
+        }
+    }
     half_t o0[4], o1[4];
     if (head < a.hq + a.hk) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            o0[e] = rope_h(x0[e], c[i + e], -x1[e], s[i + e]);
-            o1[e] = rope_h(x1[e], c[i + hd + e], x0[e], s[i + hd + e]);
+            o0[e] = rope_h(x0[e], c0[e], -x1[e], s0[e]);
+            o1[e] = rope_h(x1[e], c1[e], x0[e], s1[e]);
         }
     } else {
 #pragma unroll
@@ -94,10 +150,11 @@ __device__ __forceinline__ void rope_store(const RopeWriteParams& a, int m, int 
         dst = (half_t*)a.q_out + (int64_t)m * a.sq_b + (int64_t)(head / n_rep) * a.sq_h +
               (int64_t)(head % n_rep) * a.sq_r;
     } else {
-        const int64_t slot = a.slots[m];
-        if (slot < 0) return;
-        const int64_t blk = slot / a.page, off = slot % a.page;
-        if (blk >= a.num_blocks) return;
+        const int64_t slot = ra.slot;
+        if (slot < 0 || slot >= (int64_t)a.num_blocks * a.page) return;
+        // (a 64-bit division is a hundred instructions)
+        const int64_t blk = slot >> 32 ? slot / a.page : (unsigned)slot / (unsigned)a.page;
+        const int64_t off = slot - blk * a.page;
         const bool isk = head < a.hq + a.hk;
         const int h = isk ? head - a.hq : head - a.hq - a.hk;
         dst = (half_t*)(isk ? a.k_pool : a.v_pool) + blk * a.sp_b + off * a.sp_t +
@@ -123,6 +180,17 @@ __device__ __forceinline__ void rope_store(const RopeWriteParams& a, int m, int 
             }
         }
     }
+    if (a.vec_out) {
+        h4 v0, v1;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            v0[e] = o0[e];
+            v1[e] = o1[e];
+        }
+        *(h4*)(dst + i) = v0;
+        *(h4*)(dst + i + hd) = v1;
+        return;
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         dst[i + e] = o0[e];
@@ -132,9 +200,11 @@ __device__ __forceinline__ void rope_store(const RopeWriteParams& a, int m, int 
 
 // The plain, gate/up and q/k/v epilogues of one 16 x 16 tile whose K is not
 // split over workgroups: lane (r, g) holds the sums of row m = 16 mb + r, tile
-// columns 4g .. 4g + 3 (acc).  All lanes of a wave call it together.
+// columns 4g .. 4g + 3 (acc); ra is read by the q/k/v epilogue only.  All
+// lanes of a wave call it together.
 template <int EPI>
-__device__ __forceinline__ void finish_tile(const GemmParams& a, int tile, int mb, int lane, f4 acc) {
+__device__ __forceinline__ void finish_tile(const GemmParams& a, int tile, int mb, int lane, f4 acc,
+                                            const RopeAhead& ra) {
     const int r = lane & 15, g = lane >> 4, m = 16 * mb + r;
     if (EPI == GEMM_PLAIN) {
         const int nc = 16 * tile + 4 * g;              // this lane's 4 output columns
@@ -173,18 +243,20 @@ __device__ __forceinline__ void finish_tile(const GemmParams& a, int tile, int m
     const int tph = a.rope.d / 16, head = tile / tph, i = 8 * (tile % tph) + 4 * g;
     if (g >= 2 || m >= a.M || head >= a.rope.hq + 2 * a.rope.hk) return;
     const int n0 = head * a.rope.d + i, n1 = n0 + a.rope.d / 2;
-    half_t x0[4], x1[4];
+    half_t b0[4], b1[4], x0[4], x1[4];
+    rope_unpack(ra.b0, b0);
+    rope_unpack(ra.b1, b1);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         float v0 = acc[e], v1 = up[e];
         if (a.bias) {
-            v0 += (float)((const half_t*)a.bias)[n0 + e];
-            v1 += (float)((const half_t*)a.bias)[n1 + e];
+            v0 += (float)(a.rope.ahead ? b0[e] : ((const half_t*)a.bias)[n0 + e]);
+            v1 += (float)(a.rope.ahead ? b1[e] : ((const half_t*)a.bias)[n1 + e]);
         }
         x0[e] = (half_t)v0;
         x1[e] = (half_t)v1;
     }
-    rope_store(a.rope, m, head, i, x0, x1);
+    rope_store(a.rope, m, head, i, x0, x1, ra);
 }
 
 }  // namespace ls
