@@ -1196,11 +1196,10 @@ void paged_decode_kernel(const DecodeParams a) {
                 const int per = (a.score_pages + Sb - 1) / Sb;
                 const int p_lo = gw.s * per;
                 const int p_hi = p_lo + per < a.score_pages ? p_lo + per : a.score_pages;
-                // (batches of 5 rounds: a share of up to 80 pages in one,
-                // the 74-page shares of 14 and 28 splits included, which
-                // batches of 4 had taken in two; one variant only: with
-                // batches of 4, 5 and 8 compiled in, the larger kernel ran
-                // B8 x 32K 0.3 us slower)
+                // (batches of 5 rounds of 32 pages: the 147-page shares of
+                // 2048 pages in 14 splits in one batch, where 4 rounds would
+                // take two; one variant only: with batches of 4, 5 and 8
+                // compiled in, the larger kernel ran B8 x 32K 0.3 us slower)
                 score_slice<NWT, HG, 5>(a, b, h0, len, p_lo, p_hi);
                 LS_STAMP(1);
                 // the group's score stores complete, then it counts itself in
