@@ -239,6 +239,26 @@ __device__ __forceinline__ int xcd_major(int L, int N) {
     return x * q + (x < rem ? x : rem) + L / XCDS;
 }
 
+// The sum over the wave's 64 lanes, in every lane: DPP within rows of 16
+// lanes, the four rows by readlane (six lane exchanges through LDS are a chain
+// of some 800 cycles; this is some 100).
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
+                                             0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+    v = dpp_add<0xB1>(v);                // quad_perm 1, 0, 3, 2
+    v = dpp_add<0x4E>(v);                // quad_perm 2, 3, 0, 1
+    v = dpp_add<0x141>(v);               // half-row mirror
+    v = dpp_add<0x140>(v);               // row mirror
+    const int b = __builtin_bit_cast(int, v);
+    return (__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0)) +
+            __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16))) +
+           (__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)) +
+            __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48)));
+}
+
 // s_waitcnt with vmcnt = n and the other counters left alone (gfx9 encoding).
 constexpr int vmcnt_wait(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 

@@ -59,7 +59,8 @@ __device__ __forceinline__ int w_row(const GemmParams& a, int tile, int r) {
 // What the q/k/v epilogue reads of a lane's sequence and tile, requested before
 // the tile's sums are known: late, the bias, the position, the angles it
 // names and the slot were four memory round trips in a chain at the end of the
-// launch (M 48, row-major, 2048 x 1536: 8.84 -> 8.43 us).
+// launch (M 48, row-major, 2048 x 1536: 8.84 -> 8.43 us; and with no branch an
+// element in the epilogue, M 16, packed, with the norm, 7.24 -> 6.92).
 struct RopeAhead {
     int64_t pos, slot;                   // of the lane's sequence
     u2 c0, c1, s0, s1;                   // angles of its channels, 4 fp16 each
@@ -105,6 +106,27 @@ __device__ __forceinline__ void rope_tile(const GemmParams& a, int tile, int lan
     ra.b1 = ld(rb, n0 + w.d);
 }
 
+// The same without rope.ahead (tables past 32-bit offsets, or off 4 bytes), once
+// the sums are known.
+__device__ __forceinline__ void rope_late(const GemmParams& a, int head, int i, RopeAhead& ra) {
+    const RopeWriteParams& w = a.rope;
+    const int64_t p = ra.pos < 0 ? 0 : (ra.pos >= w.tab_rows ? w.tab_rows - 1 : ra.pos);
+    auto four = [](const void* base, int64_t at) {
+        const uint16_t* x = (const uint16_t*)base + at;
+        return u2{x[0] | (uint32_t)x[1] << 16, x[2] | (uint32_t)x[3] << 16};
+    };
+    const int64_t at = p * w.st + i, n0 = (int64_t)head * w.d + i;
+    const int hd = w.d / 2;
+    ra.c0 = four(w.cos, at);
+    ra.c1 = four(w.cos, at + hd);
+    ra.s0 = four(w.sin, at);
+    ra.s1 = four(w.sin, at + hd);
+    if (a.bias) {
+        ra.b0 = four(a.bias, n0);
+        ra.b1 = four(a.bias, n0 + hd);
+    }
+}
+
 // The fused q/k/v projection's epilogue for one lane: channels i .. i + 3
 // of head `head` (i < d / 2) and their partners i + d / 2 .. for sequence
 // m, as x0 / x1 (fp16, bias added); rotated and stored as
@@ -118,31 +140,14 @@ __device__ __forceinline__ void rope_store(const RopeWriteParams& a, int m, int 
     rope_unpack(ra.c1, c1);
     rope_unpack(ra.s0, s0);
     rope_unpack(ra.s1, s1);
-    if (!a.ahead) {
-        const int64_t p = ra.pos < 0 ? 0 : (ra.pos >= a.tab_rows ? a.tab_rows - 1 : ra.pos);
-        const half_t* c = (const half_t*)a.cos + p * a.st;
-        const half_t* s = (const half_t*)a.sin + p * a.st;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            c0[e] = c[i + e];
-            c1[e] = c[i + hd + e];
-            s0[e] = s[i + e];
-            s1[e] = s[i + hd + e];
-        }
-    }
+    const bool rotated = head < a.hq + a.hk;
     half_t o0[4], o1[4];
-    if (head < a.hq + a.hk) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            o0[e] = rope_h(x0[e], c0[e], -x1[e], s0[e]);
-            o1[e] = rope_h(x1[e], c1[e], x0[e], s1[e]);
-        }
-    } else {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            o0[e] = x0[e];
-            o1[e] = x1[e];
-        }
+    for (int e = 0; e < 4; ++e) {
+        const half_t r0 = rope_h(x0[e], c0[e], -x1[e], s0[e]);
+        const half_t r1 = rope_h(x1[e], c1[e], x0[e], s1[e]);
+        o0[e] = rotated ? r0 : x0[e];
+        o1[e] = rotated ? r1 : x1[e];
     }
     half_t* dst;
     if (head < a.hq) {
@@ -164,19 +169,20 @@ __device__ __forceinline__ void rope_store(const RopeWriteParams& a, int m, int 
             // max are exact)
             half_t* mn = (half_t*)a.kmin + blk * a.sb_b + (int64_t)h * a.sb_h;
             half_t* mx = (half_t*)a.kmax + blk * a.sb_b + (int64_t)h * a.sb_h;
+            half_t n0[4], n1[4], m0[4], m1[4];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                if (off == 0) {
-                    mn[i + e] = o0[e];
-                    mx[i + e] = o0[e];
-                    mn[i + hd + e] = o1[e];
-                    mx[i + hd + e] = o1[e];
-                } else {
-                    mn[i + e] = (half_t)fminf((float)mn[i + e], (float)o0[e]);
-                    mx[i + e] = (half_t)fmaxf((float)mx[i + e], (float)o0[e]);
-                    mn[i + hd + e] = (half_t)fminf((float)mn[i + hd + e], (float)o1[e]);
-                    mx[i + hd + e] = (half_t)fmaxf((float)mx[i + hd + e], (float)o1[e]);
-                }
+                n0[e] = mn[i + e];
+                n1[e] = mn[i + hd + e];
+                m0[e] = mx[i + e];
+                m1[e] = mx[i + hd + e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                mn[i + e] = off ? (half_t)fminf((float)n0[e], (float)o0[e]) : o0[e];
+                mx[i + e] = off ? (half_t)fmaxf((float)m0[e], (float)o0[e]) : o0[e];
+                mn[i + hd + e] = off ? (half_t)fminf((float)n1[e], (float)o1[e]) : o1[e];
+                mx[i + hd + e] = off ? (half_t)fmaxf((float)m1[e], (float)o1[e]) : o1[e];
             }
         }
     }
@@ -242,21 +248,18 @@ __device__ __forceinline__ void finish_tile(const GemmParams& a, int tile, int m
     }
     const int tph = a.rope.d / 16, head = tile / tph, i = 8 * (tile % tph) + 4 * g;
     if (g >= 2 || m >= a.M || head >= a.rope.hq + 2 * a.rope.hk) return;
-    const int n0 = head * a.rope.d + i, n1 = n0 + a.rope.d / 2;
+    RopeAhead rt = ra;
+    if (!a.rope.ahead) rope_late(a, head, i, rt);
     half_t b0[4], b1[4], x0[4], x1[4];
-    rope_unpack(ra.b0, b0);
-    rope_unpack(ra.b1, b1);
+    rope_unpack(rt.b0, b0);
+    rope_unpack(rt.b1, b1);
+    const bool biased = a.bias != nullptr;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        float v0 = acc[e], v1 = up[e];
-        if (a.bias) {
-            v0 += (float)(a.rope.ahead ? b0[e] : ((const half_t*)a.bias)[n0 + e]);
-            v1 += (float)(a.rope.ahead ? b1[e] : ((const half_t*)a.bias)[n1 + e]);
-        }
-        x0[e] = (half_t)v0;
-        x1[e] = (half_t)v1;
+        x0[e] = (half_t)(biased ? acc[e] + (float)b0[e] : acc[e]);
+        x1[e] = (half_t)(biased ? up[e] + (float)b1[e] : up[e]);
     }
-    rope_store(a.rope, m, head, i, x0, x1, ra);
+    rope_store(a.rope, m, head, i, x0, x1, rt);
 }
 
 }  // namespace ls

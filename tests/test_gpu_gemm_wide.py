@@ -131,3 +131,42 @@ def test_weight_rows_far_apart(m):
     far.copy_(w)
     assert torch.equal(dg().linear(x, far, b), dg().linear(x, w, b))
     assert torch.equal(dg().gate_up_silu(x, far), dg().gate_up_silu(x, w))
+
+
+@pytest.mark.parametrize("m,k", [(3, 96), (16, 1536), (40, 1536), (64, 2048)])
+@pytest.mark.parametrize("off", ["table", "bias", "rows", "none"])
+def test_qkv_rope_write_off_the_wide_loads(m, k, off):
+    """The q/k/v epilogue where its early 8-byte loads or its 8-byte stores do
+    not apply (tables or a bias off 4 bytes, an odd table stride; rows of q and
+    the pools off 8 bytes) and where they do, without a bias in between, over
+    pages of 12 tokens: the bits of linear followed by rope_write_decode."""
+    gen = torch.Generator(device="cuda").manual_seed(m + k)
+    hq, hk, d, nb, page = 4, 2, 64, 70, 12
+    n = (hq + 2 * hk) * d
+    x = torch.randn(m, k, device="cuda", generator=gen).half()
+    w = (torch.randn(n, k, device="cuda", generator=gen) * k**-0.5).half()
+    bias = torch.randn(n + 1, device="cuda", generator=gen).half()
+    b = {"bias": bias[1:], "none": bias[:n]}.get(off)
+    wide = torch.randn(2, 50, d + 1, device="cuda", generator=gen).half()
+    cos, sin = (wide[0, :, 1:], wide[1, :, 1:]) if off == "table" else \
+        (wide[0, :, :d].contiguous(), wide[1, :, :d].contiguous())
+    pos = torch.randint(0, 60, (m,), device="cuda", generator=gen)
+    slots = torch.randperm(nb, device="cuda", generator=gen)[:m] * page \
+        + torch.randint(0, page, (m,), device="cuda", generator=gen)
+    slots[0] = nb * page                                 # past the pool: not stored
+    extra = 1 if off == "rows" else 0
+    outs = []
+    for fused in (True, False):
+        g = torch.Generator(device="cuda").manual_seed(7)
+        pools = [torch.randn(nb, page, hk, d + extra, device="cuda", generator=g).half()[..., extra:]
+                 for _ in range(2)]
+        q = torch.zeros(m, hk, hq // hk, d + extra, device="cuda").half()[..., extra:]
+        args = (pos, cos, sin, slots, *pools, hq, hk)
+        if fused:
+            dg().qkv_rope_write(x, w, b, *args, q_out=q)
+        else:
+            fe().rope_write_decode(dg().linear(x, w, b), *args, q_out=q)
+        outs.append((q, *pools))
+    torch.cuda.synchronize()
+    for a, c in zip(*outs):
+        assert torch.equal(a, c)
