@@ -26,6 +26,8 @@ struct GemmParams {
     int splits;          // workgroups a 16-row tile's K is split over
     int chunk_pairs = 0; // pairs of 32-channel steps a wave takes (set at launch), one
     int chunk_more = 0;  // more for the first chunk_more of them
+    int walk = 0;        // tiles a workgroup takes (set at launch), one more for the first
+    int walk_more = 0;   // walk_more of them
     int epi;             // GEMM_PLAIN, GEMM_GLU: y[M, N/2] = silu(gate) * up of w =
                          // [gate; up], GEMM_ROPE: the fused q/k/v projection's outputs
                          // rotated and stored as `rope` describes (y unused)

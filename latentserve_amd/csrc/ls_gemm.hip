@@ -122,6 +122,8 @@ hipError_t launch_decode_gemm(const GemmParams& params, hipStream_t stream) {
     // the whole row
     if (p.norm && (!p.w_packed || p.M > 16 || p.splits != 1)) return hipErrorInvalidValue;
     const dim3 grid(gemm_groups(p.splits, tiles), p.splits);
+    p.walk = tiles / grid.x;
+    p.walk_more = tiles % grid.x;
     if (p.epi == GEMM_GLU) {
         if (p.splits != 1 || p.N % 2 != 0) return hipErrorInvalidValue;
         return launch_gemm_glu(p, spw, grid, stream);
