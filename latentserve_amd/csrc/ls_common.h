@@ -57,14 +57,64 @@ __device__ __forceinline__ float shfl_xor(float v, int mask) {
                                                                    __builtin_bit_cast(int, v)));
 }
 
+// Lane exchanges on the VALU (an exchange through LDS takes the wave some 100
+// cycles, and a page's softmax and a merge's reductions are chains of them: us
+// a launch, LDS -> VALU, B1 x 2048 fp16 9.64 -> 9.40, B16 x 16K INT8 34.0 ->
+// 33.3, asymmetric B5 to 11K 23.0 -> 22.5).
+// swap16 / swap32: a lane's value and that of lane ^ 16 / lane ^ 32, in one
+// order for both lanes.
+struct LanePair {
+    float a, b;
+};
+__device__ __forceinline__ LanePair swap16(float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    const uint32_t x = r[0], y = r[1];
+    return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
+}
+__device__ __forceinline__ LanePair swap32(float v) {
+    const uint32_t u = __builtin_bit_cast(uint32_t, v);
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    const uint32_t x = r[0], y = r[1];
+    return {__builtin_bit_cast(float, x), __builtin_bit_cast(float, y)};
+}
+
 // Max / sum over the four 16-lane groups that share a lane's `lane & 15`.
 __device__ __forceinline__ float group4_max(float v) {
-    v = fmaxf(v, shfl_xor(v, 16));
-    return fmaxf(v, shfl_xor(v, 32));
+    const LanePair p = swap16(v), q = swap32(fmaxf(p.a, p.b));
+    return fmaxf(q.a, q.b);
 }
 __device__ __forceinline__ float group4_sum(float v) {
-    v += shfl_xor(v, 16);
-    return v + shfl_xor(v, 32);
+    const LanePair p = swap16(v), q = swap32(p.a + p.b);
+    return q.a + q.b;
+}
+
+// Max / sum over the lane's half of the wave.
+template <int CTRL>
+__device__ __forceinline__ float dpp_move(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL,
+                                                                  0xF, 0xF, false));
+}
+__device__ __forceinline__ float half_max(float v) {
+    v = fmaxf(v, dpp_move<0xB1>(v));     // quad_perm 1, 0, 3, 2
+    v = fmaxf(v, dpp_move<0x4E>(v));     // quad_perm 2, 3, 0, 1
+    v = fmaxf(v, dpp_move<0x141>(v));    // half-row mirror
+    v = fmaxf(v, dpp_move<0x140>(v));    // row mirror
+    const LanePair p = swap16(v);
+    return fmaxf(p.a, p.b);
+}
+__device__ __forceinline__ float half_sum(float v) {
+    v += dpp_move<0xB1>(v);
+    v += dpp_move<0x4E>(v);
+    v += dpp_move<0x141>(v);
+    v += dpp_move<0x140>(v);
+    const LanePair p = swap16(v);
+    return p.a + p.b;
+}
+// Sum over the wave.
+__device__ __forceinline__ float wave_sum_dpp(float v) {
+    const LanePair p = swap32(half_sum(v));
+    return p.a + p.b;
 }
 
 // Four signed int8 (one dword) -> four fp16, exactly: each byte, offset by
@@ -237,26 +287,6 @@ __device__ __forceinline__ int xcd_major(int L, int N) {
     constexpr int XCDS = 8;
     const int q = N / XCDS, rem = N % XCDS, x = L % XCDS;
     return x * q + (x < rem ? x : rem) + L / XCDS;
-}
-
-// The sum over the wave's 64 lanes, in every lane: DPP within rows of 16
-// lanes, the four rows by readlane (six lane exchanges through LDS are a chain
-// of some 800 cycles; this is some 100).
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    return v + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(
-                                             0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
-}
-__device__ __forceinline__ float wave_sum_dpp(float v) {
-    v = dpp_add<0xB1>(v);                // quad_perm 1, 0, 3, 2
-    v = dpp_add<0x4E>(v);                // quad_perm 2, 3, 0, 1
-    v = dpp_add<0x141>(v);               // half-row mirror
-    v = dpp_add<0x140>(v);               // row mirror
-    const int b = __builtin_bit_cast(int, v);
-    return (__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 0)) +
-            __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 16))) +
-           (__builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 32)) +
-            __builtin_bit_cast(float, __builtin_amdgcn_readlane(b, 48)));
 }
 
 // s_waitcnt with vmcnt = n and the other counters left alone (gfx9 encoding).

@@ -487,17 +487,11 @@ __device__ void combine_records(const float* acc, const float* m, int S, int NR,
                 av[i] = load_coherent4(rs, vo_a, (int)(sp * sa_s * (int64_t)sizeof(float)));
             }
             const float mj = j < n ? __builtin_bit_cast(float, (uint32_t)ml) : neg_inf();
-            float cm = mj;
-#pragma unroll
-            for (int k = 16; k > 0; k >>= 1) cm = fmaxf(cm, shfl_xor(cm, k));
-            cm = fmaxf(cm, mg);                     // the same in the half-wave
+            const float cm = fmaxf(half_max(mj), mg);   // the same in the half-wave
             const bool none = cm == neg_inf();      // nothing valid yet
             const float sc = none ? 1.f : __expf(mg - cm);          // 0 while mg is -inf
             const float wj = none || j >= n ? 0.f : __expf(mj - cm);  // 0 for empty splits
-            float lj = wj * __builtin_bit_cast(float, (uint32_t)(ml >> 32));
-#pragma unroll
-            for (int k = 16; k > 0; k >>= 1) lj += shfl_xor(lj, k);
-            lt = lt * sc + lj;
+            lt = lt * sc + half_sum(wj * __builtin_bit_cast(float, (uint32_t)(ml >> 32)));
             at *= sc;
 #pragma unroll
             for (int i = 0; i < R; ++i) {
