@@ -83,9 +83,9 @@ typedef struct LsKernelResources {
  * "sparse_attention_bounds_fp16" (one launch), "combine_splits",
  * "page_index", "page_index_heads", "page_mass", "page_select",
  * "page_bounds_update", "page_bounds_rebuild", "int8_decode_write",
- * "int8_finalize_blocks", "int8_prefill_write".  kv_heads: decode kernels pair the heads of an
- * even count in one workgroup; n_rep: the index kernels are specialised on
- * it.  Needs a current HIP device. */
+ * "int8_finalize_blocks", "int8_prefill_write".  kv_heads: dense and list
+ * decodes pair the heads of an even count in one workgroup; n_rep: the index
+ * kernels are specialised on it.  Needs a current HIP device. */
 int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, int has_res,
                         LsKernelResources* out);
 
@@ -583,7 +583,7 @@ int ls_decode_gemm(const void* x, int64_t x_stride, const void* w, int64_t w_str
  * partial sums and arrival counters when K is split over workgroups (narrow
  * outputs with long K), 0 otherwise (workspace may then be NULL).  The
  * workspace is 256-byte aligned and zero-filled before its first use; its
- * first 64 KiB hold the counters, which each call leaves at zero again.  Calls that share a workspace
+ * first 256 KiB hold the counters, which each call leaves at zero again.  Calls that share a workspace
  * must be ordered on one stream.  No counterpart in the reference (a cuBLAS
  * call sizes its own). */
 size_t ls_decode_gemm_workspace_bytes(int M, int N, int K);
