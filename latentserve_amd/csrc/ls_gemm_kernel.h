@@ -33,11 +33,11 @@
 // kernel before gave a group of up to 4 waves one to four tiles, with X read
 // again for them, and split K from 512 channels on above 32 rows):
 //                      M 16, packed     M 48, row-major    M 64, row-major
-//   17920 x 1536      15.5 -> 12.8      42.8 -> 14.8       52.8 -> 17.0
-//   1536 x 8960       12.4 -> 10.3      42.7 -> 13.1       53.5 -> 15.1
-//   1536 x 1536        4.9 -> 4.3       12.7 ->  6.3       15.2 ->  7.4
-//   2048 x 5632       10.8 -> 8.9       31.3 -> 11.4       39.1 -> 13.2
-//   151936 x 1536     89.0 -> 80.9  (5.8 TB/s)
+//   17920 x 1536      15.5 -> 12.5      42.8 -> 14.1       52.8 -> 16.7
+//   1536 x 8960       12.4 -> 9.8       42.7 -> 12.8       53.5 -> 14.5
+//   1536 x 1536        4.9 -> 4.0       12.7 ->  6.0       15.2 ->  7.2
+//   2048 x 5632       10.8 -> 8.4
+//   151936 x 1536     89.0 -> 80.8  (5.8 TB/s)
 #pragma once
 
 #include <type_traits>
@@ -143,8 +143,12 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
         return 2 * (c * a.chunk_pairs + (c < a.chunk_more ? c : a.chunk_more));
     };
     const int c = blockIdx.y * GEMM_WAVES + wv;
-    const int s0 = first_step(c), end = first_step(c + 1);
-    const int ns = (end < steps ? end : steps) - s0;                          // 0..SPW (host)
+    const int S0 = first_step(blockIdx.y * GEMM_WAVES);      // the group's first
+    const int begin = first_step(c), end = first_step(c + 1);
+    const int ns = (end < steps ? end : steps) - begin;      // at most SPW (host)
+    // (fewer pairs than waves leave the last chunks empty: they stay at the
+    // group's first step, so that no address is past the row)
+    const int s0 = ns > 0 ? begin : S0;
 
     // W of a tile.  Packed: a step is 1 KiB in the order the lanes take it.
     // Row-major: lane (r, g) needs 16 bytes of row r a step; so that an
@@ -228,7 +232,6 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
     // 1.5 us a column block at K 1536.  Groups start at different rows and
     // columns, so that the CUs of an XCD do not ask one L2 channel for the
     // same line together.
-    const int S0 = first_step(blockIdx.y * GEMM_WAVES);
     u4 xb[SPW][MB];
     auto stage = [&](int first) {
 #pragma unroll

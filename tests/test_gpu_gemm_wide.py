@@ -104,6 +104,18 @@ def test_qkv_rope_write(m, hq, hk, d, k, bounds):
         assert torch.equal(a, c)
 
 
+@pytest.mark.parametrize("k", [32, 64, 96, 448])
+def test_weight_rows_far_apart_with_empty_chunks(k):
+    """Rows past 32-bit offsets and a K of fewer steps than the waves: the waves
+    without a chunk read within the rows (the last row ends the allocation)."""
+    n, ld = 16, (1 << 26) + 8
+    x, w, b = _operands(16, n, k)
+    store = torch.empty((n - 1) * ld + k, dtype=torch.float16, device="cuda")
+    far = store.as_strided((n, k), (ld, 1))
+    far.copy_(w)
+    assert torch.equal(dg().linear(x, far, b), dg().linear(x, w, b))
+
+
 def test_split_product_in_a_graph_replays_exactly():
     x, w, _ = _operands(48, 1536, 8960)
     assert dg().workspace_bytes(48, 1536, 8960) > 0
