@@ -215,6 +215,9 @@ _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)    # (None: a
 
 
 def stream_of(device: torch.device) -> int:
-    """torch's current stream on `device` as a hipStream_t."""
+    """torch's current stream on `device` as a hipStream_t.  Every launch asks
+    for it, and for several entry points this is what refuses CPU tensors."""
+    if device.type != "cuda":
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return _raw_stream(torch.cuda.current_device() if index is None else index)
