@@ -40,6 +40,14 @@ def _contig(t: torch.Tensor, name: str) -> None:
         raise ValueError(f"{name} must be contiguous")
 
 
+def _on_device(first: torch.Tensor, *others: Optional[torch.Tensor]) -> None:
+    dev = first.get_device()
+    for t in others:
+        if t is not None and t.get_device() != dev:
+            raise ValueError(f"all tensors must be on one device, got {first.device} and "
+                             f"{t.device}")
+
+
 def decode_write(k, v, slots, res_idx, flat_v, flat_v_scale, flat_v_zero, k_res, *,
                  asym: bool, eps: float, qmax: float, levels: float, offset: float,
                  exact_division: bool = False) -> None:
@@ -101,6 +109,7 @@ def finalize_blocks(data: torch.Tensor, ids: torch.Tensor, k_pool: torch.Tensor,
     if asym and (k_zero is None or k_zero.shape != k_scale.shape
                  or k_zero.stride() != k_scale.stride() or k_zero.dtype != torch.float32):
         raise ValueError("asymmetric quantization needs k_zero shaped and strided as k_scale")
+    _on_device(data, ids, k_pool, k_scale, k_zero if asym else None, rows)
     P, S = _lib.ptr, _lib.strides
     src = (P(data), S(data, 3)) if rows is None else (P(data), S(data, 3), P(rows), data.shape[0])
     L = _lib.lib()
@@ -121,26 +130,28 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
     rows before the chunk in its first page are).  k_quant, v_quant: (eps,
     qmax, levels, offset).  One launch."""
     b, h, n, d = k.shape
-    if not (k.is_cuda and v.is_cuda) or k.dtype != torch.float16 or v.dtype != torch.float16 \
+    dev = k.get_device()                      # (-1: not on a GPU)
+    if dev < 0 or v.get_device() != dev or k.dtype != torch.float16 or v.dtype != torch.float16 \
             or d != HEAD_DIM or v.shape != k.shape:
         raise ValueError("prefill_write: k and v must be fp16 [B, H, n, 128] GPU tensors")
-    if slots.dtype != torch.int64 or slots.shape != (b, n) or not slots.is_contiguous():
-        raise ValueError("slots must be a contiguous int64 [B, n] tensor")
-    if rows.dtype != torch.int64 or rows.dim() != 1 or rows.shape[0] < b or rows.stride(0) != 1:
-        raise ValueError("rows must be a unit-stride int64 [B] tensor")
+    if slots.dtype != torch.int64 or slots.shape != (b, n) or not slots.is_contiguous() \
+            or slots.get_device() != dev:
+        raise ValueError("slots must be a contiguous int64 [B, n] tensor on k's device")
+    if rows.dtype != torch.int64 or rows.dim() != 1 or rows.shape[0] < b or rows.stride(0) != 1 \
+            or rows.get_device() != dev:
+        raise ValueError("rows must be a unit-stride int64 [B] tensor on k's device")
     nb, nr = k_pool.shape[0], k_res.shape[0]
     i8, f32 = torch.int8, torch.float32
-    for t, name, dt, shape in (
-            (k_pool, "k_pool", i8, (nb, PAGE, h, d)), (v_pool, "v_pool", i8, (nb, PAGE, h, d)),
-            (k_scale, "k_scale", f32, (nb, h, d)), (v_scale, "v_scale", f32, (nb, PAGE, h)),
-            (k_res, "k_res", torch.float16, (nr, PAGE, h, d))):
-        if t.dtype != dt or t.shape != shape or not t.is_contiguous():
-            raise ValueError(f"{name} must be contiguous {dt} {shape}")
+    pools = [(k_pool, "k_pool", i8, (nb, PAGE, h, d)), (v_pool, "v_pool", i8, (nb, PAGE, h, d)),
+             (k_scale, "k_scale", f32, (nb, h, d)), (v_scale, "v_scale", f32, (nb, PAGE, h)),
+             (k_res, "k_res", torch.float16, (nr, PAGE, h, d))]
     if asym:
-        for t, name, like in ((k_zero, "k_zero", k_scale), (v_zero, "v_zero", v_scale)):
-            if t is None or t.shape != like.shape or t.dtype != torch.float32:
-                raise ValueError(f"asymmetric quantization needs {name} shaped as its scales")
-            _contig(t, name)
+        if k_zero is None or v_zero is None:
+            raise ValueError("asymmetric quantization needs k_zero and v_zero")
+        pools += [(k_zero, "k_zero", f32, (nb, h, d)), (v_zero, "v_zero", f32, (nb, PAGE, h))]
+    for t, name, dt, shape in pools:
+        if t.dtype != dt or t.shape != shape or not t.is_contiguous() or t.get_device() != dev:
+            raise ValueError(f"{name} must be contiguous {dt} {shape} on k's device")
     k, v = _loadable(k, 4), _loadable(v, 16)
     P, S = _lib.ptr, _lib.strides
     eps, qmax, levels, offset = k_quant

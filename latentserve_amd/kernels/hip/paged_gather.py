@@ -18,6 +18,12 @@ from latentserve_amd import _lib
 PAGE = 16
 
 
+def _same_device(pool: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tensor) -> None:
+    dev = pool.get_device()
+    if block_tables.get_device() != dev or seq_lens.get_device() != dev:
+        raise ValueError("block tables and sequence lengths must be on the pool's device")
+
+
 def gather(pool: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tensor,
            length: Optional[int] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """pool [nb, 16, H, D] (fp16 / int8 / fp32) -> [B, H, length, D] view.
@@ -29,12 +35,14 @@ def gather(pool: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tenso
     if block_tables.dtype != torch.int32 or seq_lens.dtype != torch.int32 \
             or block_tables.stride(-1) != 1 or seq_lens.stride(-1) != 1:
         raise ValueError("block tables and sequence lengths must be unit-stride int32")
+    _same_device(pool, block_tables, seq_lens)
     nb, _, h, d = pool.shape
     b = block_tables.shape[0]
     length = block_tables.shape[1] * PAGE if length is None else int(length)
     if out is None:
         out = torch.empty(b, length, h, d, dtype=pool.dtype, device=pool.device)
-    elif out.shape != (b, length, h, d) or out.dtype != pool.dtype or out.stride(-1) != 1:
+    elif out.shape != (b, length, h, d) or out.dtype != pool.dtype or out.stride(-1) != 1 \
+            or out.device != pool.device:
         raise ValueError(f"out must be {pool.dtype} [{b}, {length}, {h}, {d}]")
     P, S = _lib.ptr, _lib.strides
     rc = _lib.lib().ls_paged_gather(
@@ -57,6 +65,7 @@ def read(k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Tensor,
     if block_tables.dtype != torch.int32 or seq_lens.dtype != torch.int32 \
             or block_tables.stride(-1) != 1 or seq_lens.stride(-1) != 1:
         raise ValueError("block tables and sequence lengths must be unit-stride int32")
+    _same_device(k_pool, block_tables, seq_lens)
     nb, _, h, d = k_pool.shape
     b = block_tables.shape[0]
     length = block_tables.shape[1] * PAGE if length is None else int(length)

@@ -91,3 +91,64 @@ def test_stream_of_takes_gpu_devices_only(library):
     for device in ("cpu", "meta"):
         with pytest.raises(ValueError):
             _lib.stream_of(torch.device(device))
+
+
+def _mixed_calls():
+    """(entry, the operand left on the CPU) -> a call with every other operand on
+    the GPU."""
+    half = dict(dtype=torch.float16, device="cuda")
+    zeros = torch.zeros
+
+    def gather(name):
+        ops = dict(pool=zeros(NB, 16, H, D, **half), t=_tables()[0].cuda(), l=_tables()[1].cuda())
+        ops[name] = ops[name].cpu()
+        return pg.gather(ops["pool"], ops["t"], ops["l"])
+
+    def read(name):
+        ops = dict(k=zeros(NB, 16, H, D, **half), v=zeros(NB, 16, H, D, **half),
+                   t=_tables()[0].cuda(), l=_tables()[1].cuda())
+        ops[name] = ops[name].cpu()
+        return pg.read(ops["k"], ops["v"], ops["t"], ops["l"])
+
+    def finalize(name):
+        ops = dict(data=zeros(3, 16, H, D, **half), ids=zeros(2, dtype=torch.long, device="cuda"),
+                   rows=zeros(2, dtype=torch.long, device="cuda"),
+                   k_pool=zeros(NB, 16, H, D, dtype=torch.int8, device="cuda"),
+                   k_scale=zeros(NB, H, D, device="cuda"), k_zero=zeros(NB, H, D, device="cuda"))
+        ops[name] = ops[name].cpu()
+        return iw.finalize_blocks(ops["data"], ops["ids"], ops["k_pool"], ops["k_scale"],
+                                  ops["k_zero"], rows=ops["rows"], asym=True, eps=1e-8, qmax=127.0,
+                                  levels=255.0, offset=128.0)
+
+    def prefill(name):
+        ops = dict(k=zeros(B, H, 5, D, **half), v=zeros(B, H, 5, D, **half),
+                   slots=zeros(B, 5, dtype=torch.long, device="cuda"),
+                   rows=zeros(B, dtype=torch.long, device="cuda"),
+                   k_pool=zeros(NB, 16, H, D, dtype=torch.int8, device="cuda"),
+                   k_scale=zeros(NB, H, D, device="cuda"), k_zero=zeros(NB, H, D, device="cuda"),
+                   v_pool=zeros(NB, 16, H, D, dtype=torch.int8, device="cuda"),
+                   v_scale=zeros(NB, 16, H, device="cuda"), v_zero=zeros(NB, 16, H, device="cuda"),
+                   k_res=zeros(B, 16, H, D, **half))
+        if name is not None:
+            ops[name] = ops[name].cpu()
+        quant = (1e-8, 127.0, 255.0, 128.0)
+        return iw.prefill_write(*ops.values(), asym=True, k_quant=quant, v_quant=quant)
+
+    return {(fn, name): (lambda fn=fn, name=name: fn(name)) for fn, names in (
+        (gather, ("pool", "t", "l")), (read, ("k", "t", "l")),
+        (finalize, ("data", "ids", "rows", "k_pool", "k_scale", "k_zero")),
+        (prefill, ("k", "v", "slots", "rows", "k_pool", "k_scale", "k_zero", "v_pool", "v_scale",
+                   "v_zero", "k_res"))) for name in names}, lambda: prefill(None)
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+def test_one_operand_on_the_cpu_is_refused(library):
+    """A CPU operand among GPU ones (the recorder takes the launch's place)."""
+    calls, whole = _mixed_calls()
+    for (fn, name), call in calls.items():
+        with pytest.raises(ValueError):
+            call()
+        assert library.launched == [], (fn.__name__, name)
+    whole()
+    assert library.launched == ["ls_int8_prefill_write"]
