@@ -263,9 +263,9 @@ def sparse_decode(q, k_pool, v_pool, block_tables, seq_lens, sel,
 
 
 SELECT_SPLIT_ENTRIES = 1024    # list entries a selecting group keeps (a split's share)
-# the one-launch bounds path: at most this many query rows a KV head (else the
-# index kernel, then the selecting decode); past this many pages a row, its
-# entry for long rows
+# the one-launch bounds path: bounds of as many blocks as the pools and at most
+# this many query rows a KV head (else the index kernel, then the selecting
+# decode); past this many pages a row, its entry for long rows
 COOP_MAX_PAGES = 2048
 COOP_MAX_NREP = 8
 
@@ -316,10 +316,11 @@ def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
     target = buf if out is None else pdh.check_out(out, q)
     P, S = _lib.ptr, _lib.strides
     short = block_tables.shape[1] <= COOP_MAX_PAGES
-    # (long rows whose bounds cover another number of blocks than the pools:
-    # the index kernel, which takes the bounds' own count)
+    # (bounds that cover another number of blocks than the pools: the index
+    # kernel, which takes the bounds' own count; the one launch has one count
+    # for both, and would read past the end of shorter bounds)
     if (scoring == "bounds" and n_rep <= COOP_MAX_NREP
-            and (short or kmin.shape[0] == k_pool.shape[0])):
+            and kmin.shape[0] == k_pool.shape[0]):
         # one launch: the decode's workgroups score the pages themselves,
         # exchanging the scores through a buffer whose count words are all
         # ones at rest

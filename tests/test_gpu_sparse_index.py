@@ -520,10 +520,11 @@ def test_selecting_decode_across_the_row_lengths(h_kv, width, lens, splits, scor
         _lib.lib().ls_set_coop_wait_ticks(5000)
 
 
-def test_long_rows_with_bounds_of_another_block_count():
-    """Rows past COOP_MAX_PAGES whose bounds hold fewer blocks than the pools:
-    pages of blocks past the bounds are left out, as by index + select."""
-    width = 2100
+@pytest.mark.parametrize("width", [340, 2048, 2100])
+def test_bounds_of_another_block_count(width):
+    """Bounds that hold fewer blocks than the pools, rows either side of
+    COOP_MAX_PAGES: pages of blocks past the bounds are left out, as by index +
+    select."""
     q, k, v, t, l, kmin, kmax = index_case([width * 16], width=width, seed=4)
     nb = len(kmin) - 300
     args = dev(q, k, v, t, l, kmin[:nb], kmax[:nb])
