@@ -325,10 +325,13 @@ def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
         # exchanging the scores through a buffer whose count words are all
         # ones at rest
         _check_bounds(kmin, kmax, q.device)
-        # (each row is followed by one word: the count of its scored shares)
-        # (rows padded to 16 bytes, so a row starts 16-byte aligned)
-        ws = scratch("sparse_coop_scores", (b, h, (block_tables.shape[1] + 4) // 4 * 4),
-                     torch.int32, q.device, init=-1)
+        # (each row is followed by one word: the count of its scored shares; rows
+        # padded to 16 bytes, so a row starts 16-byte aligned.  A buffer a width:
+        # in one of several widths, the word one counts in holds a score of
+        # another)
+        width = block_tables.shape[1]
+        ws = scratch(("sparse_coop_scores", width), (b, h, (width + 4) // 4 * 4), torch.int32,
+                     q.device, init=-1)
         entry = "ls_sparse_attention_bounds_fp16" if short else "ls_sparse_attention_bounds_long_fp16"
         rc = getattr(_lib.lib(), entry)(
             P(q), S(q, 3), P(k_pool), P(v_pool), S(k_pool, 3), k_pool.shape[0],

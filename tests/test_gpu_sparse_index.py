@@ -484,12 +484,31 @@ def test_one_launch_path_with_the_fallback_forced(width, lens, splits):
     sel = ps().index_select(Q, KN, KX, T, L, kk, ratio).cpu().numpy()
     want = oracle.sparse_decode(q, k, v, t, l, sel, ratio=ratio, recent=2)
     assert_close(forced.float().cpu().numpy(), want, ATOL, RTOL, "fallback forced")
+    assert _count_words_at_rest(width)
+
+
+def _count_words_at_rest(width):
+    """The word after every row of the width's score buffers (a row's count of
+    scored shares) is all ones."""
     from latentserve_amd.kernels.gqa import _SCRATCH
-    for key, buf in _SCRATCH.items():
-        if key[0] == "sparse_coop_scores" and buf.shape[2] == (width + 4) // 4 * 4:
-            # the word after every row (the count after each head group's
-            # first row; untouched after the others)
-            assert bool((buf[:, :, width] == -1).all()), "count words not left all ones"
+    bufs = [buf for key, buf in _SCRATCH.items() if key[0] == ("sparse_coop_scores", width)]
+    assert bufs and all(buf.shape[2] == (width + 4) // 4 * 4 for buf in bufs)
+    return all(bool((buf[:, :, width] == -1).all()) for buf in bufs)
+
+
+def test_widths_of_the_same_padding_in_turn():
+    """Rows of 300 to 303 pages are padded alike: calls at each in turn keep their
+    count words apart (a score left in one would make the groups wait the bound
+    out, or take another call's scores for the missing ones)."""
+    width, seen = 300, set()
+    for n in (3, 0, 2, 1, 3, 0):
+        q, k, v, t, l, kmin, kmax = index_case([(width + n) * 16, 77], width=width + n, seed=n)
+        args = dev(q, k, v, t, l, kmin, kmax)
+        got = ps().sparse_attention(*args, ratio=0.5, num_splits=5).float()
+        want = ps().sparse_attention(*args, ratio=0.5, fused=False).float()
+        assert (got - want).abs().max().item() < 1e-3, n
+        seen.add(width + n)
+        assert all(_count_words_at_rest(w) for w in seen), n
 
 
 @pytest.mark.parametrize("scoring", ["bounds", "mass"])

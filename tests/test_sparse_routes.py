@@ -55,3 +55,17 @@ def test_one_launch_only_with_bounds_of_every_pool_block(library, width, bound_b
     else:
         assert names == ["ls_page_scores", "ls_sparse_attention_fp16"]
         assert library.calls[0][1][5] == bound_blocks
+
+
+def test_every_row_width_counts_in_a_buffer_of_its_own(library):
+    """A row's count of scored shares is the word behind its scores, all ones at
+    rest: widths that share a buffer leave scores in each other's counts."""
+    for width in (40, 41, 42, 43, 44):
+        _attend(width)
+    one = "ls_sparse_attention_bounds_fp16"
+    buffers = [args[13] for name, args in library.calls if name == one]
+    assert len(set(buffers)) == 5
+    for width in (40, 43):                      # and the same one again
+        _attend(width)
+    again = [args[13] for name, args in library.calls if name == one][5:]
+    assert again == [buffers[0], buffers[3]]
