@@ -61,8 +61,10 @@ enum {
 /* Message for the last non-zero return on this thread. */
 const char* ls_last_error(void);
 
-/* ABI version (bumped when an existing signature changes; entry points may be
- * added under the same version). */
+/* ABI version (bumped on any signature change or addition, and when what a
+ * caller must provide changes: 20 has the sparse, INT8 chunk, row and paged
+ * read / write entries that 19 lacked, and 256 KiB of counters at the head of
+ * the decode GEMM's workspace, not 64). */
 int ls_abi_version(void);
 
 /* What the runtime reports of a loaded kernel (hipFuncGetAttributes and

@@ -28,7 +28,7 @@ LS_ERR_INVALID = 1
 LS_ERR_HIP = 2
 # The ABI this binding is written for (include/latentserve_amd.h); a library
 # built from other sources is refused rather than called with wrong arguments.
-ABI_VERSION = 19
+ABI_VERSION = 20
 
 # name -> argtypes, mirroring include/latentserve_amd.h
 _SIGNATURES = {
@@ -148,6 +148,12 @@ def lib() -> ctypes.CDLL:
                 f"{LIB_PATH} is not built; run `python -m latentserve_amd.csrc.build` "
                 "(the HIP backend has no fallback)")
         handle = ctypes.CDLL(LIB_PATH)
+        # (before the entry points: a library of another version may lack some)
+        got = handle.ls_abi_version()
+        if got != ABI_VERSION:
+            raise HipLibraryMissing(
+                f"{LIB_PATH} has ABI {got}, this binding expects {ABI_VERSION}: rebuild it with "
+                "`python -m latentserve_amd.csrc.build`")
         for name, argtypes in _SIGNATURES.items():
             fn = getattr(handle, name)
             fn.argtypes = argtypes
@@ -158,11 +164,6 @@ def lib() -> ctypes.CDLL:
                           "ls_argmax_workspace_bytes": ctypes.c_size_t,
                           "ls_page_mass_workspace_bytes": ctypes.c_size_t,
                           "ls_gemm_packed_bytes": ctypes.c_size_t}.get(name, ctypes.c_int)
-        got = handle.ls_abi_version()
-        if got != ABI_VERSION:
-            raise HipLibraryMissing(
-                f"{LIB_PATH} has ABI {got}, this binding expects {ABI_VERSION}: rebuild it with "
-                "`python -m latentserve_amd.csrc.build`")
         _lib = handle
     return _lib
 

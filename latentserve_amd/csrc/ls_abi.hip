@@ -231,7 +231,7 @@ extern "C" {
 
 const char* ls_last_error(void) { return g_err.c_str(); }
 
-int ls_abi_version(void) { return 19; }
+int ls_abi_version(void) { return 20; }
 
 int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, int has_res,
                         LsKernelResources* out) {

@@ -5,6 +5,7 @@ any launch (argument checks need no device)."""
 from __future__ import annotations
 
 import ctypes
+import hashlib
 import os
 import re
 
@@ -38,8 +39,31 @@ def test_python_binding_covers_the_header():
     assert set(declared()) == set(_lib.exported_symbols())
 
 
+# the header's declarations and structs at ABI_VERSION, comments and spacing aside
+DECLARATIONS = (20, "54b543351dcfeb38")
+
+
 def test_abi_version(lib):
-    assert lib.ls_abi_version() == 19
+    """A change of any declaration, or a new one, is a new version: the digest
+    names the version it was taken at."""
+    from latentserve_amd import _lib
+    text = re.sub(r"/\*.*?\*/", "", open(HEADER).read(), flags=re.S)
+    digest = hashlib.sha256(" ".join(text.split()).encode()).hexdigest()[:16]
+    assert (_lib.ABI_VERSION, digest) == DECLARATIONS
+    assert lib.ls_abi_version() == _lib.ABI_VERSION
+
+
+def test_a_library_of_another_version_is_refused_by_its_version(lib, monkeypatch, tmp_path):
+    """Before its entry points are looked up: it may lack some."""
+    import subprocess
+    from latentserve_amd import _lib
+    src, so = tmp_path / "other.c", tmp_path / "other.so"
+    src.write_text("int ls_abi_version(void) { return 1; }\n")
+    subprocess.run(["gcc", "-shared", "-fPIC", "-o", str(so), str(src)], check=True)
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib, "LIB_PATH", str(so))
+    with pytest.raises(_lib.HipLibraryMissing, match="ABI 1"):
+        _lib.lib()
 
 
 def test_workspace_size(lib):
