@@ -64,7 +64,8 @@ const char* ls_last_error(void);
 /* ABI version (bumped on any signature change or addition, and when what a
  * caller must provide changes: 20 has the sparse, INT8 chunk, row and paged
  * read / write entries that 19 lacked, and 256 KiB of counters at the head of
- * the decode GEMM's workspace, not 64). */
+ * the decode GEMM's workspace, not 64; 21 has ls_int8_prefill_write's
+ * v_eps). */
 int ls_abi_version(void);
 
 /* What the runtime reports of a loaded kernel (hipFuncGetAttributes and
@@ -391,8 +392,8 @@ int ls_int8_finalize_rows(const void* data, const int64_t* data_strides, const i
  * k_pool / k_scale (/ k_zero), the rows of the first page before the chunk
  * taken from row rows[b] of the fp16 residual k_res [num_res, 16, H_kv, 128];
  * the last page's K goes to that row, zeros past its end.  All pools
- * contiguous; slots and rows outside them are skipped.  qmax / levels / offset
- * are K's, v_* V's.  Replaces Int8PagedKVCache.write of a chunk
+ * contiguous; slots and rows outside them are skipped.  eps / qmax / levels /
+ * offset are K's, v_* V's.  Replaces Int8PagedKVCache.write of a chunk
  * (cache/int8_paged_cache.py:432-600, :670-758). */
 int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v,
                           const int64_t* v_strides, const int64_t* slots, const int64_t* rows,
@@ -400,7 +401,8 @@ int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v
                           float* v_scale, float* v_zero, void* k_res, int64_t num_blocks,
                           int64_t num_res, int batch, int kv_heads, int tokens, int head_dim,
                           int page, int asym, float eps, float qmax, float levels, float offset,
-                          int recip, float v_qmax, float v_levels, float v_offset, void* stream);
+                          int recip, float v_eps, float v_qmax, float v_levels, float v_offset,
+                          void* stream);
 
 /* New K and V rows to their slots: k / v [B, H_kv, tokens, head_dim]
  * (strides[3] = (b, h, token)) of elem_bytes-byte elements to flat slot

@@ -231,7 +231,7 @@ extern "C" {
 
 const char* ls_last_error(void) { return g_err.c_str(); }
 
-int ls_abi_version(void) { return 20; }
+int ls_abi_version(void) { return 21; }
 
 int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, int has_res,
                         LsKernelResources* out) {
@@ -957,7 +957,8 @@ int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v
                           float* v_scale, float* v_zero, void* k_res, int64_t num_blocks,
                           int64_t num_res, int batch, int kv_heads, int tokens, int head_dim,
                           int page, int asym, float eps, float qmax, float levels, float offset,
-                          int recip, float v_qmax, float v_levels, float v_offset, void* stream) {
+                          int recip, float v_eps, float v_qmax, float v_levels, float v_offset,
+                          void* stream) {
     if (!k || !k_strides || !v || !v_strides || !slots || !rows || !k_pool || !k_scale || !v_pool ||
         !v_scale || !k_res)
         return fail(LS_ERR_INVALID, "null pointer argument");
@@ -975,7 +976,7 @@ int ls_int8_prefill_write(const void* k, const int64_t* k_strides, const void* v
         return fail(LS_ERR_INVALID, "k rows must be aligned to channel pairs, v rows to 16 bytes");
     ls::PrefillWriteParams a;
     if (int rc = quant_args(asym, eps, qmax, levels, offset, recip, a.qk)) return rc;
-    if (int rc = quant_args(asym, eps, v_qmax, v_levels, v_offset, recip, a.qv)) return rc;
+    if (int rc = quant_args(asym, v_eps, v_qmax, v_levels, v_offset, recip, a.qv)) return rc;
     if (batch == 0 || tokens == 0) return LS_OK;
     a.k = k;
     a.sk_b = k_strides[0];

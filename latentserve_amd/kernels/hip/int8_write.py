@@ -155,12 +155,12 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
     k, v = _loadable(k, 4), _loadable(v, 16)
     P, S = _lib.ptr, _lib.strides
     eps, qmax, levels, offset = k_quant
-    _, v_qmax, v_levels, v_offset = v_quant
+    v_eps, v_qmax, v_levels, v_offset = v_quant
     rc = _lib.lib().ls_int8_prefill_write(
         P(k), S(k, 3), P(v), S(v, 3), P(slots), P(rows), P(k_pool), P(k_scale),
         P(k_zero) if asym else None, P(v_pool), P(v_scale), P(v_zero) if asym else None, P(k_res),
         nb, nr, b, h, n, d, PAGE, int(bool(asym)), eps, qmax, levels, offset,
-        0 if exact_division else 1, v_qmax, v_levels, v_offset, _lib.stream_of(k.device))
+        0 if exact_division else 1, v_eps, v_qmax, v_levels, v_offset, _lib.stream_of(k.device))
     _lib.check(rc, "ls_int8_prefill_write")
 
 

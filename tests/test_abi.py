@@ -40,7 +40,7 @@ def test_python_binding_covers_the_header():
 
 
 # the header's declarations and structs at ABI_VERSION, comments and spacing aside
-DECLARATIONS = (20, "54b543351dcfeb38")
+DECLARATIONS = (21, "6a2c84314c59d0ec")
 
 
 def test_abi_version(lib):
@@ -134,3 +134,17 @@ def test_kernel_resources_rejects_unknown_names_and_bad_shapes(lib):
     assert lib.ls_kernel_resources(b"page_index", 2, 17, 0, 0, ctypes.byref(r)) == 1
     assert lib.ls_kernel_resources(b"page_index", 2, 6, 0, 0, None) == 1
 
+
+
+def _call_prefill_write(lib, batch=0, eps=1e-8, v_eps=1e-8, v_qmax=127.0):
+    st = _strides(4096, 2048, 128)
+    return lib.ls_int8_prefill_write(1024, st, 2048, st, 4096, 64, 1 << 12, 1 << 13, None, 1 << 14,
+                                     1 << 15, None, 1 << 16, 10, 4, batch, 2, 16, 128, 16, 0, eps,
+                                     127.0, 255.0, 128.0, 1, v_eps, v_qmax, 255.0, 128.0, None)
+
+
+@pytest.mark.parametrize("over", [dict(eps=-1.0), dict(v_eps=-1.0), dict(v_qmax=0.0)])
+def test_prefill_write_checks_both_quantizers(lib, over):
+    assert _call_prefill_write(lib) == 0
+    assert _call_prefill_write(lib, **over) == 1
+    assert "quantizer constants" in lib.ls_last_error().decode()

@@ -123,3 +123,34 @@ def test_int8_chunks_equal_the_oracle(asym, layout, chunks, h):
         res = c.residual(0)[s].cpu().numpy()
         assert np.array_equal(res[:total - last * BS], k_all[i, last * BS:])
         assert c.pooled_pages(s) == last
+
+
+@pytest.mark.parametrize("asym", [False, True])
+def test_int8_chunk_takes_ks_and_vs_own_eps(asym):
+    """K's and V's quantizer constants apart, eps included: rows below V's floor
+    but above K's, and the other way round."""
+    from latentserve_amd.kernels.hip import int8_write as iw
+    h, n, nb = 2, 40, 5
+    g = torch.Generator(device="cuda").manual_seed(9)
+    k, v = ((torch.randn(1, h, n, 128, generator=g, device="cuda") * 0.01).half()
+            for _ in range(2))
+    pool = lambda *shape, dtype=torch.float32: torch.zeros(*shape, dtype=dtype, device="cuda")
+    kp, vp = (pool(nb, BS, h, 128, dtype=torch.int8) for _ in range(2))
+    ks, kz, vs, vz = pool(nb, h, 128), pool(nb, h, 128), pool(nb, BS, h), pool(nb, BS, h)
+    for k_eps, v_eps in ((1e-8, 0.5), (0.5, 1e-8)):
+        iw.prefill_write(k, v, torch.arange(n, device="cuda").view(1, n),
+                         torch.zeros(1, dtype=torch.long, device="cuda"), kp, ks, kz, vp, vs, vz,
+                         pool(1, BS, h, 128, dtype=torch.float16), asym=asym,
+                         k_quant=(k_eps, 127.0, 255.0, 128.0), v_quant=(v_eps, 7.0, 15.0, 8.0))
+        rows = np.ascontiguousarray(v[0].transpose(0, 1).cpu().numpy())
+        codes, step, zero = oracle.quantize_v(rows, asym=asym, eps=v_eps, bits=4, recip=True)
+        assert np.array_equal(vp.view(-1, h, 128)[:n].cpu().numpy(), codes)
+        assert np.array_equal(vs.view(-1, h)[:n].cpu().numpy(), step)
+        pages = np.ascontiguousarray(k[0].transpose(0, 1)[:2 * BS].cpu().numpy())
+        codes, step, kzero = oracle.quantize_k(pages.reshape(2, BS, h, 128), asym=asym, eps=k_eps,
+                                               recip=True)
+        assert np.array_equal(kp[:2].cpu().numpy(), codes)
+        assert np.array_equal(ks[:2].cpu().numpy(), step)
+        if asym:
+            assert np.array_equal(vz.view(-1, h)[:n].cpu().numpy(), zero)
+            assert np.array_equal(kz[:2].cpu().numpy(), kzero)
