@@ -803,9 +803,10 @@ int ls_page_bounds_update(const void* k_new, const int64_t* kn_strides, const in
     return hip_status(ls::launch_bounds_update(a, (hipStream_t)stream), "ls_page_bounds_update");
 }
 
-int ls_page_bounds_rebuild(const void* k_pool, const int64_t* kv_strides, int num_blocks,
-                           void* kmin, void* kmax, const int64_t* bound_strides, int kv_heads,
-                           int head_dim, int page, void* stream) {
+// The argument checks of a bounds rebuild.
+static int check_bounds_rebuild(const void* k_pool, const int64_t* kv_strides, int64_t num_blocks,
+                                const void* kmin, const void* kmax, const int64_t* bound_strides,
+                                int kv_heads, int head_dim, int page) {
     if (!k_pool || !kv_strides || !kmin || !kmax || !bound_strides)
         return fail(LS_ERR_INVALID, "null pointer argument");
     if (head_dim != ls::HEAD_DIM) return fail(LS_ERR_INVALID, "head_dim must be 128, got %d", head_dim);
@@ -814,6 +815,15 @@ int ls_page_bounds_rebuild(const void* k_pool, const int64_t* kv_strides, int nu
     if (!rows_aligned(k_pool, kv_strides, 3, 2, 16) || !rows_aligned(kmin, bound_strides, 2, 2, 16) ||
         !rows_aligned(kmax, bound_strides, 2, 2, 16))
         return fail(LS_ERR_INVALID, "k_pool, kmin and kmax rows must be 16-byte aligned");
+    return LS_OK;
+}
+
+int ls_page_bounds_rebuild(const void* k_pool, const int64_t* kv_strides, int num_blocks,
+                           void* kmin, void* kmax, const int64_t* bound_strides, int kv_heads,
+                           int head_dim, int page, void* stream) {
+    if (int rc = check_bounds_rebuild(k_pool, kv_strides, num_blocks, kmin, kmax, bound_strides,
+                                      kv_heads, head_dim, page))
+        return rc;
     ls::BoundsParams a;
     a.src = k_pool;
     a.s0 = kv_strides[0];
@@ -1024,6 +1034,14 @@ int ls_paged_write(const void* k, const int64_t* k_strides, const void* v,
     if (!rows_aligned(k, k_strides, 3, e, 16) || !rows_aligned(v, v_strides, 3, e, 16) ||
         !rows_aligned(k_pool, kv_strides, 3, e, 16) || !rows_aligned(v_pool, kv_strides, 3, e, 16))
         return fail(LS_ERR_INVALID, "k, v and pool rows must be 16-byte aligned");
+    // (the bounds' too, before anything is stored)
+    if (kmin) {
+        if (elem_bytes != 2) return fail(LS_ERR_INVALID, "bounds are kept of fp16 pools only");
+        if (num_blocks > (1LL << 31) - 1) return fail(LS_ERR_INVALID, "too many blocks");
+        if (int rc = check_bounds_rebuild(k_pool, kv_strides, num_blocks, kmin, kmax, bound_strides,
+                                          kv_heads, head_dim, page))
+            return rc;
+    }
     if (batch == 0 || tokens == 0) return LS_OK;
     ls::PagedWriteParams a;
     const void* src[2] = {k, v};
@@ -1046,8 +1064,6 @@ int ls_paged_write(const void* k, const int64_t* k_strides, const void* v,
     a.B = batch;
     a.H = kv_heads;
     a.N = tokens;
-    if (kmin && elem_bytes != 2) return fail(LS_ERR_INVALID, "bounds are kept of fp16 pools only");
-    if (kmin && num_blocks > (1LL << 31) - 1) return fail(LS_ERR_INVALID, "too many blocks");
     if (int rc = hip_status(ls::launch_paged_write(a, (hipStream_t)stream), "ls_paged_write"))
         return rc;
     if (!kmin) return LS_OK;

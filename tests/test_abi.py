@@ -148,3 +148,27 @@ def test_prefill_write_checks_both_quantizers(lib, over):
     assert _call_prefill_write(lib) == 0
     assert _call_prefill_write(lib, **over) == 1
     assert "quantizer constants" in lib.ls_last_error().decode()
+
+
+@pytest.mark.parametrize("over,needle", [
+    (dict(kmax=None), "null"),
+    (dict(bst=None), "null"),
+    (dict(kmin=1 << 18 | 8), "aligned"),
+    (dict(bst=_strides(256, 127)), "aligned"),
+    (dict(d=64), "head_dim"),
+    (dict(elem=4), "fp16"),
+    (dict(nb=1 << 31), "blocks"),
+])
+@pytest.mark.parametrize("tokens", [0, 5])
+def test_paged_write_checks_its_bounds_before_anything_is_stored(lib, tokens, over, needle):
+    """Bad bounds refuse the whole call: nothing is launched (there is no device
+    here, and a launch would report that instead), whatever the token count."""
+    st = _strides(4096, 256, 128)
+
+    def call(elem=2, d=128, nb=10, kmin=1 << 18, kmax=1 << 19, bst=_strides(256, 128), tokens=0):
+        return lib.ls_paged_write(1024, st, 2048, st, 4096, 1 << 16, 1 << 17, st, nb, elem, 2, 2,
+                                  tokens, d, 16, kmin, kmax, bst, None)
+
+    assert call() == 0
+    assert call(tokens=tokens, **over) == 1
+    assert needle in lib.ls_last_error().decode()
