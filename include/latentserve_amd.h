@@ -86,9 +86,14 @@ typedef struct LsKernelResources {
  * "sparse_attention_bounds_fp16" (one launch), "combine_splits",
  * "page_index", "page_index_heads", "page_mass", "page_select",
  * "page_bounds_update", "page_bounds_rebuild", "int8_decode_write",
- * "int8_finalize_blocks", "int8_prefill_write".  kv_heads: dense and list
- * decodes pair the heads of an even count in one workgroup; n_rep: the index
- * kernels are specialised on it.  Needs a current HIP device. */
+ * "int8_finalize_blocks", "int8_prefill_write".  The dense
+ * decodes with "_dealt" behind the name are the launches of more workgroups
+ * than are resident at once; the selecting decodes hold four score keys a
+ * thread (rows of 1025 to 2048 pages), with "_keys2", "_keys8" or "_keys16"
+ * behind the name two, eight or sixteen (to 1024, 4096 and 8192).  kv_heads:
+ * dense and list decodes pair the heads of an even count in one workgroup;
+ * n_rep: the index kernels are specialised on it.  Needs a current HIP
+ * device. */
 int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, int has_res,
                         LsKernelResources* out);
 

@@ -240,13 +240,36 @@ int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, i
         return fail(LS_ERR_INVALID, "bad kv_heads (%d) or n_rep (%d)", kv_heads, n_rep);
     const std::string k = kernel;
     const bool pair = kv_heads % 2 == 0;
+    // the decode walks: name (+ variant), kind, walk, variant
+    static const struct {
+        const char *name, *variant;
+        int kind, walk, var;
+    } walks[] = {
+        {"paged_decode_fp16", "", ls::KV_FP16, 0, 0},
+        {"paged_decode_fp16", "_dealt", ls::KV_FP16, 0, 1},
+        {"paged_decode_int8", "", ls::KV_INT8, 0, 0},
+        {"paged_decode_int8", "_dealt", ls::KV_INT8, 0, 1},
+        {"paged_sparse_fp16", "", ls::KV_FP16, 1, 0},
+        {"sparse_attention_fp16", "", ls::KV_FP16, 2, 4},
+        {"sparse_attention_fp16", "_keys2", ls::KV_FP16, 2, 2},
+        {"sparse_attention_fp16", "_keys8", ls::KV_FP16, 2, 8},
+        {"sparse_attention_fp16", "_keys16", ls::KV_FP16, 2, 16},
+        {"sparse_attention_bounds_fp16", "", ls::KV_FP16, 3, 4},
+        {"sparse_attention_bounds_fp16", "_keys2", ls::KV_FP16, 3, 2},
+        {"sparse_attention_bounds_fp16", "_keys8", ls::KV_FP16, 3, 8},
+        {"sparse_attention_bounds_fp16", "_keys16", ls::KV_FP16, 3, 16},
+    };
     ls::KernelResources r{};
-    hipError_t e;
-    if (k == "paged_decode_fp16") e = ls::decode_resources(ls::KV_FP16, 0, false, false, pair, &r);
-    else if (k == "paged_decode_int8") e = ls::decode_resources(ls::KV_INT8, 0, asym, has_res, pair, &r);
-    else if (k == "paged_sparse_fp16") e = ls::decode_resources(ls::KV_FP16, 1, false, false, pair, &r);
-    else if (k == "sparse_attention_fp16") e = ls::decode_resources(ls::KV_FP16, 2, false, false, pair, &r);
-    else if (k == "sparse_attention_bounds_fp16") e = ls::decode_resources(ls::KV_FP16, 3, false, false, pair, &r);
+    hipError_t e = hipErrorInvalidValue;
+    bool found = false;
+    for (const auto& w : walks)
+        if (k == std::string(w.name) + w.variant) {
+            const bool i8 = w.kind == ls::KV_INT8;
+            e = ls::decode_resources(w.kind, w.walk, w.var, i8 && asym, i8 && has_res, pair, &r);
+            found = true;
+        }
+    if (found)
+        ;
     else if (k == "combine_splits") e = ls::combine_resources(&r);
     else if (k == "page_index") e = ls::sparse_index_resources(0, n_rep, &r);
     else if (k == "page_index_heads") e = ls::sparse_index_resources(1, n_rep, &r);

@@ -106,10 +106,12 @@ constexpr int NOALLOC_COUNTERS = 1 << 16;
 hipError_t noalloc_scratch(hipStream_t stream, float** work, int32_t** counters);
 hipError_t launch_combine(const CombineParams& p, hipStream_t stream);
 // The kernel a decode launch runs: walk 0 dense, 1 a given list, 2 selecting
-// from given scores, 3 scoring and selecting itself; `pair_heads` an even
-// head count; INT8 with `asym` / `has_res`.  combine: ls_combine_splits's.
-hipError_t decode_resources(int kind, int walk, bool asym, bool has_res, bool pair_heads,
-                            KernelResources* r);
+// from given scores, 3 scoring and selecting itself; `var` the kernel's VAR (walk
+// 0: 1 where the groups are dealt; walks 2 and 3: a thread's keys, 2 to 16);
+// `pair_heads` an even head count; INT8 with `asym` / `has_res`.  combine:
+// ls_combine_splits's.
+hipError_t decode_resources(int kind, int walk, int var, bool asym, bool has_res,
+                            bool pair_heads, KernelResources* r);
 hipError_t combine_resources(KernelResources* r);
 #ifdef LS_DIAGNOSTICS
 // Page-compute probe (measurement only): groups x 8 waves, each applying one

@@ -1718,38 +1718,49 @@ static hipError_t launch_kernel(const DecodeParams& a, hipStream_t stream) {
     return launch_t<KV_INT8, false, false, 0>(a, stream);
 }
 
-template <int KIND, bool ASYM, bool HAS_RES, int SPARSE>
+template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int VAR = 0>
 static hipError_t resources_t(bool pair_heads, KernelResources* r) {
     if (pair_heads)
-        return func_resources(paged_decode_kernel<KIND, ASYM, HAS_RES, SPARSE, 2 * NWAVES, 2>,
-                              WAVE * NWAVES * 2, r);
-    return func_resources(paged_decode_kernel<KIND, ASYM, HAS_RES, SPARSE, NWAVES, 1>,
+        return func_resources(
+            paged_decode_kernel<KIND, ASYM, HAS_RES, SPARSE, 2 * NWAVES, 2, 0, VAR>,
+            WAVE * NWAVES * 2, r);
+    return func_resources(paged_decode_kernel<KIND, ASYM, HAS_RES, SPARSE, NWAVES, 1, 0, VAR>,
                           WAVE * NWAVES, r);
 }
 
-hipError_t decode_resources(int kind, int walk, bool asym, bool has_res, bool pair_heads,
-                            KernelResources* r) {
-    if (kind == KV_FP16) {
-        switch (walk) {
-            case 0: return resources_t<KV_FP16, false, false, 0>(pair_heads, r);
-            case 1: return resources_t<KV_FP16, false, false, 1>(pair_heads, r);
-            // (the selecting walks: the keys of rows of up to 2048 pages)
-            case 2:
-                return func_resources(
-                    paged_decode_kernel<KV_FP16, false, false, 2, 2 * NWAVES, 1, 0, 4>,
-                    2 * NWAVES * WAVE, r);
-            case 3:
-                return func_resources(
-                    paged_decode_kernel<KV_FP16, false, false, 3, 2 * NWAVES, 1, 0, 4>,
-                    2 * NWAVES * WAVE, r);
-            default: return hipErrorInvalidValue;
-        }
+template <int VAR>
+static hipError_t dense_resources(int kind, bool asym, bool has_res, bool pair_heads,
+                                  KernelResources* r) {
+    if (kind == KV_FP16) return resources_t<KV_FP16, false, false, 0, VAR>(pair_heads, r);
+    if (asym && has_res) return resources_t<KV_INT8, true, true, 0, VAR>(pair_heads, r);
+    if (asym) return resources_t<KV_INT8, true, false, 0, VAR>(pair_heads, r);
+    if (has_res) return resources_t<KV_INT8, false, true, 0, VAR>(pair_heads, r);
+    return resources_t<KV_INT8, false, false, 0, VAR>(pair_heads, r);
+}
+
+template <int SPARSE, int KEYS>
+static hipError_t selecting_resources(KernelResources* r) {
+    return func_resources(
+        paged_decode_kernel<KV_FP16, false, false, SPARSE, 2 * NWAVES, 1, 0, KEYS>,
+        2 * NWAVES * WAVE, r);
+}
+
+hipError_t decode_resources(int kind, int walk, int var, bool asym, bool has_res,
+                            bool pair_heads, KernelResources* r) {
+    if (walk == 0)
+        return var == 0   ? dense_resources<0>(kind, asym, has_res, pair_heads, r)
+               : var == 1 ? dense_resources<1>(kind, asym, has_res, pair_heads, r)
+                          : hipErrorInvalidValue;
+    if (kind != KV_FP16) return hipErrorInvalidValue;
+    if (walk == 1) return resources_t<KV_FP16, false, false, 1>(pair_heads, r);
+    if (walk != 2 && walk != 3) return hipErrorInvalidValue;
+    switch (var) {
+        case 2: return walk == 2 ? selecting_resources<2, 2>(r) : selecting_resources<3, 2>(r);
+        case 4: return walk == 2 ? selecting_resources<2, 4>(r) : selecting_resources<3, 4>(r);
+        case 8: return walk == 2 ? selecting_resources<2, 8>(r) : selecting_resources<3, 8>(r);
+        case 16: return walk == 2 ? selecting_resources<2, 16>(r) : selecting_resources<3, 16>(r);
+        default: return hipErrorInvalidValue;
     }
-    if (walk != 0) return hipErrorInvalidValue;
-    if (asym && has_res) return resources_t<KV_INT8, true, true, 0>(pair_heads, r);
-    if (asym) return resources_t<KV_INT8, true, false, 0>(pair_heads, r);
-    if (has_res) return resources_t<KV_INT8, false, true, 0>(pair_heads, r);
-    return resources_t<KV_INT8, false, false, 0>(pair_heads, r);
 }
 
 hipError_t combine_resources(KernelResources* r) { return func_resources(combine_kernel<4>, 256, r); }

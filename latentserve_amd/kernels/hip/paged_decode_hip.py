@@ -250,7 +250,8 @@ def paged_decode_cuda(q, k_pool, v_pool, block_tables, seq_lens, max_seq_len: in
 def kernel_resources(device: Optional[torch.device] = None, head_dim: int = HEAD_DIM,
                      n_rep: int = 6, page: int = PAGE, variant: str = "fp16",
                      asym: bool = False, has_res: bool = False,
-                     min_blocks: Optional[int] = None, kv_heads: int = 2) -> dict:
+                     min_blocks: Optional[int] = None, kv_heads: int = 2,
+                     dealt: bool = False) -> dict:
     """Registers, private (spill) memory and LDS of the loaded decode kernel
     that a launch with these properties runs, as the HIP runtime reports
     them (kernels/cuda/paged_decode_cuda.py:163-186, which asks the CUDA
@@ -258,7 +259,8 @@ def kernel_resources(device: Optional[torch.device] = None, head_dim: int = HEAD
     spills), ``shared_bytes``, plus ``threads`` (a workgroup) and
     ``groups_per_cu`` (occupancy).  ``min_blocks`` has no effect here (see
     paged_decode_cuda); ``kv_heads`` chooses the paired-head kernel (even)
-    or the one-head kernel (odd).
+    or the one-head kernel (odd); ``dealt`` the kernel of a launch of more
+    workgroups than are resident at once.
     """
     del min_blocks
     if head_dim != HEAD_DIM or page != PAGE or not 1 <= n_rep <= MAX_NREP:
@@ -267,7 +269,7 @@ def kernel_resources(device: Optional[torch.device] = None, head_dim: int = HEAD
     names = {"fp16": "paged_decode_fp16", "int8": "paged_decode_int8"}
     if variant not in names:
         raise ValueError(f"variant must be 'fp16' or 'int8', got {variant!r}")
-    return _lib.kernel_resources(names[variant], device, kv_heads=kv_heads, n_rep=n_rep,
+    return _lib.kernel_resources(names[variant] + ("_dealt" if dealt else ""), device, kv_heads=kv_heads, n_rep=n_rep,
                                  asym=asym, has_res=has_res)
 
 

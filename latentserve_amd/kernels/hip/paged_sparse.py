@@ -58,8 +58,11 @@ def kernel_resources(device: Optional[torch.device] = None, n_rep: int = 6,
     kernel, by name (kernels/cuda/paged_sparse.py:254-265; the reference's
     four names plus this build's selection and one-launch kernels)."""
     names = ("page_bounds_update", "page_index", "page_index_heads", "paged_sparse_fp16",
-             "page_mass", "page_select", "page_bounds_rebuild", "sparse_attention_fp16",
-             "sparse_attention_bounds_fp16")
+             "page_mass", "page_select", "page_bounds_rebuild")
+    # the selecting decodes: four score keys a thread, or (by the row's length)
+    # two, eight or sixteen
+    names += tuple(f"{n}{keys}" for n in ("sparse_attention_fp16", "sparse_attention_bounds_fp16")
+                   for keys in ("", "_keys2", "_keys8", "_keys16"))
     return {n: _lib.kernel_resources(n, device, kv_heads=kv_heads, n_rep=n_rep) for n in names}
 
 

@@ -130,6 +130,8 @@ def test_kernel_resources_rejects_unknown_names_and_bad_shapes(lib):
     r = _lib.KernelResources()
     assert lib.ls_kernel_resources(b"no_such_kernel", 2, 6, 0, 0, ctypes.byref(r)) == 1
     assert "unknown kernel" in lib.ls_last_error().decode()
+    for name in (b"paged_sparse_fp16_dealt", b"sparse_attention_fp16_keys4", b"paged_decode_fp16_keys2"):
+        assert lib.ls_kernel_resources(name, 2, 6, 0, 0, ctypes.byref(r)) == 1
     assert lib.ls_kernel_resources(b"paged_decode_fp16", 0, 6, 0, 0, ctypes.byref(r)) == 1
     assert lib.ls_kernel_resources(b"page_index", 2, 17, 0, 0, ctypes.byref(r)) == 1
     assert lib.ls_kernel_resources(b"page_index", 2, 6, 0, 0, None) == 1

@@ -354,14 +354,17 @@ def test_kernel_resources_report_no_spills():
     seen = {}
     for variant, asym, res in (("fp16", False, False), ("int8", False, False),
                                ("int8", False, True), ("int8", True, False), ("int8", True, True)):
-        for heads in (2, 3):
+        for heads, dealt in ((2, False), (3, False), (2, True), (3, True)):
             r = pdh.kernel_resources(variant=variant, asym=asym, has_res=res, kv_heads=heads,
-                                     min_blocks=12)
-            seen[(variant, asym, res, heads)] = r
+                                     min_blocks=12, dealt=dealt)
+            seen[(variant, asym, res, heads, dealt)] = r
             assert r["local_bytes"] == 0, (variant, asym, res, heads, r)
             assert r["groups_per_cu"] >= 1 and r["threads"] == (512 if heads == 2 else 256), r
             assert r["regs"] <= 256 and r["shared_bytes"] <= 160 * 1024, r
-    for name, r in ps.kernel_resources().items():
+    sparse = ps.kernel_resources()
+    for walk in ("sparse_attention_fp16", "sparse_attention_bounds_fp16"):
+        assert {walk + keys for keys in ("", "_keys2", "_keys8", "_keys16")} <= set(sparse)
+    for name, r in sparse.items():
         assert r["local_bytes"] == 0, (name, r)
         assert r["groups_per_cu"] >= 1, (name, r)
     print(seen)
