@@ -1631,13 +1631,14 @@ static hipError_t launch_heads(const DecodeParams& a, hipStream_t stream) {
 
 // The selecting walks: one head a group of 8 waves, the keys a thread holds by
 // the row's length.  The splits are cut to what is resident at once (the
-// one-launch path's groups wait for each other's scores), where a split's
-// entries still fit the table.
+// one-launch path's groups wait for each other's scores), in the two-launch path
+// to two rounds of it, where a split's entries still fit the table.
 template <int SPARSE>
 static hipError_t launch_selecting(const DecodeParams& a, hipStream_t stream) {
     constexpr int NWT = 2 * NWAVES, THREADS = WAVE * NWT;
     DecodeParams d = a;
-    const int fit = (int)(RESIDENT_WAVES / NWT / ((int64_t)a.B * a.H));
+    constexpr int ROUNDS = SPARSE == 2 ? 2 : 1;
+    const int fit = (int)(ROUNDS * RESIDENT_WAVES / NWT / ((int64_t)a.B * a.H));
     const int least = (a.num_sel + SELECT_SPLIT_ENTRIES - 1) / SELECT_SPLIT_ENTRIES;
     int most = fit > least ? fit : least;
     most = most > 1 ? most : 1;

@@ -11,8 +11,8 @@ ls_sparse_attention_bounds_long_fp16): the page-subset decode's workgroups
 score their shares of their sequence's pages, exchange the scores, and each
 selects its own list by the selection kernel's rule (the same lists and
 partition as index + select + sparse_decode).  Mass scoring, and bounds
-scoring of more than COOP_MAX_NREP query rows a KV head, are two launches
-(the scores, then ls_sparse_attention_fp16);
+scoring of more than COOP_MAX_NREP query rows a KV head or of many long rows
+(_one_launch), are two launches (the scores, then ls_sparse_attention_fp16);
 ``fused=False`` runs the three (index, select, decode).  Nothing syncs with
 the host, so the step is capturable in a HIP graph.
 """
@@ -271,6 +271,40 @@ SELECT_SPLIT_ENTRIES = 1024    # list entries a selecting group keeps (a split's
 # decode); past this many pages a row, its entry for long rows
 COOP_MAX_PAGES = 2048
 COOP_MAX_NREP = 8
+# A selecting group a CU.  In one launch a row's scores are the work of its own
+# groups, 160 pages in one batch of loads; in two the index kernel spreads every
+# row over the chip, which a short row's groups would leave idle.  So one launch
+# up to a batch a group, and up to COOP_MAX_PAGES where the rows are few enough
+# that the launch it saves counts.  (us, ratio 0.25, full / ragged lengths, one
+# launch -> two: B18 x 4 heads to 8000 28.2 / 23.6 -> 27.2 / 22.4, B17 x 8 to
+# 5000 34.0 / 31.6 -> 30.2 / 27.2, to 32000 176 / 134 -> 142 / 99, B32 x 8 to
+# 16000 121 / 89 -> 116 / 82, B8 x 8 to 100K 190 / 127 -> 180 / 109; under a
+# batch, B16 x 8 to 1500 15.6 / 14.4 -> 17.0 / 16.1, B24 x 8 to 2500 22.8 / 20.5 ->
+# 23.3 / 20.4, B32 x 8 to 2500 25.2 / 21.4 -> 26.5 / 21.7.)
+SELECT_GROUPS = 256
+SCORE_BATCH = 160
+FEW_ROWS = 64
+# In two launches the groups need not be resident together: where the whole groups
+# a row that are leave CUs idle (129 to 170 rows: one, on up to half of them), two
+# rounds of an odd count fill them, from this many selected pages a group on (us,
+# full / ragged lengths, B17 x 8 heads, one -> three groups: 125 pages 43.1 /
+# 37.6 -> 47.5 / 36.0, 250 79.5 / 68.0 -> 75.9 / 60.5, 500 142 / 99 -> 136 / 71;
+# B12 x 8, two -> five: 625 pages 118 / 97 -> 121 / 86).
+TWO_ROUNDS_MIN_PAGES = 160
+
+
+def _one_launch(rows: int, width: int) -> bool:
+    """Whether the groups of `rows` (sequence, KV head) rows of `width` pages score
+    the pages themselves."""
+    share = -(-width // max(1, SELECT_GROUPS // max(1, rows)))
+    return share <= SCORE_BATCH or (rows <= FEW_ROWS and width <= COOP_MAX_PAGES)
+
+
+def _two_rounds(rows: int, k: int) -> int:
+    """Splits of the two-launch path's lists of k pages in two rounds of groups, 0
+    where one round is as good."""
+    fit, two = (n * SELECT_GROUPS // max(1, rows) for n in (1, 2))
+    return two if 1 <= fit < 4 and two > 2 * fit and k >= TWO_ROUNDS_MIN_PAGES * fit else 0
 
 
 def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
@@ -282,8 +316,8 @@ def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
     """Index, select, attend. The list width k follows `max_seq_len` (the
     context) when given, else the table's width; each sequence then attends
     its own budget for its current length.  Fused, bounds scoring is one
-    launch (the decode's workgroups score, select and attend) and mass
-    scoring two (the scores, then a decode that selects); ``fused=False``
+    launch (the decode's workgroups score, select and attend), or two as mass
+    scoring (the scores, then a decode that selects); ``fused=False``
     runs index, select and decode as three."""
     if scoring not in ("bounds", "mass"):
         raise ValueError(f"unknown scoring {scoring!r} (bounds or mass)")
@@ -313,17 +347,20 @@ def sparse_attention(q, k_pool, v_pool, block_tables, seq_lens, kmin, kmax,
     # elsewhere, so the count is asked for twice the heads)
     splits = num_splits or pdh.choose_splits(b, 2 * h, k, q.device, dealt=False)
     splits = max(1, min(splits, max(1, k), pdh.MAX_SPLITS))
+    # (bounds that cover another number of blocks than the pools: the index
+    # kernel, which takes the bounds' own count; the one launch has one count
+    # for both, and would read past the end of shorter bounds)
+    one = (scoring == "bounds" and n_rep <= COOP_MAX_NREP and kmin.shape[0] == k_pool.shape[0]
+           and _one_launch(b * h, block_tables.shape[1]))
+    if not num_splits and not one:
+        splits = max(splits, _two_rounds(b * h, k))
     splits = max(splits, -(-k // SELECT_SPLIT_ENTRIES))
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     buf, work, cnt = pdh._buffers("sparse", b, h, splits, n_rep, q.device)
     target = buf if out is None else pdh.check_out(out, q)
     P, S = _lib.ptr, _lib.strides
     short = block_tables.shape[1] <= COOP_MAX_PAGES
-    # (bounds that cover another number of blocks than the pools: the index
-    # kernel, which takes the bounds' own count; the one launch has one count
-    # for both, and would read past the end of shorter bounds)
-    if (scoring == "bounds" and n_rep <= COOP_MAX_NREP
-            and kmin.shape[0] == k_pool.shape[0]):
+    if one:
         # one launch: the decode's workgroups score the pages themselves,
         # exchanging the scores through a buffer whose count words are all
         # ones at rest
