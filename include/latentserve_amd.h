@@ -90,7 +90,8 @@ typedef struct LsKernelResources {
  * decodes with "_dealt" behind the name are the launches of more workgroups
  * than are resident at once; the selecting decodes hold four score keys a
  * thread (rows of 1025 to 2048 pages), with "_keys2", "_keys8" or "_keys16"
- * behind the name two, eight or sixteen (to 1024, 4096 and 8192).  kv_heads:
+ * behind the name two, eight or sixteen (to 1024, 4096 and 8192), with "_4waves"
+ * the form of many short rows.  kv_heads:
  * dense and list decodes pair the heads of an even count in one workgroup;
  * n_rep: the index kernels are specialised on it.  Needs a current HIP
  * device. */

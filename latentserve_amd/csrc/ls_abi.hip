@@ -251,10 +251,12 @@ int ls_kernel_resources(const char* kernel, int kv_heads, int n_rep, int asym, i
         {"paged_decode_int8", "_dealt", ls::KV_INT8, 0, 1},
         {"paged_sparse_fp16", "", ls::KV_FP16, 1, 0},
         {"sparse_attention_fp16", "", ls::KV_FP16, 2, 4},
+        {"sparse_attention_fp16", "_4waves", ls::KV_FP16, 2, 1},
         {"sparse_attention_fp16", "_keys2", ls::KV_FP16, 2, 2},
         {"sparse_attention_fp16", "_keys8", ls::KV_FP16, 2, 8},
         {"sparse_attention_fp16", "_keys16", ls::KV_FP16, 2, 16},
         {"sparse_attention_bounds_fp16", "", ls::KV_FP16, 3, 4},
+        {"sparse_attention_bounds_fp16", "_4waves", ls::KV_FP16, 3, 1},
         {"sparse_attention_bounds_fp16", "_keys2", ls::KV_FP16, 3, 2},
         {"sparse_attention_bounds_fp16", "_keys8", ls::KV_FP16, 3, 8},
         {"sparse_attention_bounds_fp16", "_keys16", ls::KV_FP16, 3, 16},

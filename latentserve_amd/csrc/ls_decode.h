@@ -107,7 +107,7 @@ hipError_t noalloc_scratch(hipStream_t stream, float** work, int32_t** counters)
 hipError_t launch_combine(const CombineParams& p, hipStream_t stream);
 // The kernel a decode launch runs: walk 0 dense, 1 a given list, 2 selecting
 // from given scores, 3 scoring and selecting itself; `var` the kernel's VAR (walk
-// 0: 1 where the groups are dealt; walks 2 and 3: a thread's keys, 2 to 16);
+// 0: 1 where the groups are dealt; walks 2 and 3: a thread's keys, 2 to 16, or 1: the groups of 4 waves);
 // `pair_heads` an even head count; INT8 with `asym` / `has_res`.  combine:
 // ls_combine_splits's.
 hipError_t decode_resources(int kind, int walk, int var, bool asym, bool has_res,

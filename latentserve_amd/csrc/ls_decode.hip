@@ -1629,6 +1629,23 @@ static hipError_t launch_heads(const DecodeParams& a, hipStream_t stream) {
     return hipGetLastError();
 }
 
+template <int SPARSE, int NWT, int KEYS>
+static hipError_t launch_keys(const DecodeParams& a, hipStream_t stream) {
+    hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, KEYS>),
+                       dim3(a.num_splits * a.H, a.B), dim3(WAVE * NWT), 0, stream, a);
+    return hipGetLastError();
+}
+
+// Rows (in pages) of more (sequence, KV head) rows than CUs up to which a group
+// is of 4 waves, two a CU: a group's selection is a chain of latencies, and two
+// chains share the CU where one left it idle.  Longer rows keep 8 waves, which
+// balance ragged lengths better.  (us, full / ragged lengths, 8 -> 4 waves, one
+// launch: B64 x 8 heads to 600 tokens 24.1 / 22.4 -> 16.0 / 13.5, to 1500 34.8 /
+// 29.7 -> 27.5 / 21.8, B128 x 8 to 600 46.1 / 42.5 -> 29.8 / 26.2; two launches:
+// B64 x 8 to 5000 78.1 / 55.6 -> 74.0 / 53.3, B40 x 8 to 5000 63.2 / 41.8 -> 57.7 /
+// 37.4, to 8000 95.7 / 57.2 -> 86.4 / 68.7, to 16000 168 / 100 -> 163 / 126.)
+constexpr int SMALL_GROUP_PAGES = 320;
+
 // The selecting walks: one head a group of 8 waves, the keys a thread holds by
 // the row's length.  The splits are cut to what is resident at once (the
 // one-launch path's groups wait for each other's scores), in the two-launch path
@@ -1636,30 +1653,23 @@ static hipError_t launch_heads(const DecodeParams& a, hipStream_t stream) {
 template <int SPARSE>
 static hipError_t launch_selecting(const DecodeParams& a, hipStream_t stream) {
     constexpr int NWT = 2 * NWAVES, THREADS = WAVE * NWT;
-    DecodeParams d = a;
     constexpr int ROUNDS = SPARSE == 2 ? 2 : 1;
-    const int fit = (int)(ROUNDS * RESIDENT_WAVES / NWT / ((int64_t)a.B * a.H));
+    DecodeParams d = a;
+    const int64_t rows = (int64_t)a.B * a.H, resident = RESIDENT_WAVES / NWT;
+    const int fit = (int)(ROUNDS * resident / rows);
     const int least = (a.num_sel + SELECT_SPLIT_ENTRIES - 1) / SELECT_SPLIT_ENTRIES;
     int most = fit > least ? fit : least;
     most = most > 1 ? most : 1;
     if (d.num_splits > most) d.num_splits = most;
-    const dim3 grid(d.num_splits * a.H, a.B), block(THREADS);
+    static_assert(SMALL_GROUP_PAGES <= 2 * WAVE * NWAVES, "two keys a thread");
+    if (rows > resident && a.score_pages <= SMALL_GROUP_PAGES && d.num_splits == 1)
+        return launch_keys<SPARSE, NWAVES, 2>(d, stream);
     const int keys = (a.score_pages + THREADS - 1) / THREADS;
-    if (keys <= 2)
-        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 2>), grid,
-                           block, 0, stream, d);
-    else if (keys <= 4)
-        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 4>), grid,
-                           block, 0, stream, d);
-    else if (keys <= 8)
-        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 8>), grid,
-                           block, 0, stream, d);
-    else if (keys <= 16)
-        hipLaunchKernelGGL((paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, 16>), grid,
-                           block, 0, stream, d);
-    else
-        return hipErrorInvalidValue;
-    return hipGetLastError();
+    if (keys <= 2) return launch_keys<SPARSE, NWT, 2>(d, stream);
+    if (keys <= 4) return launch_keys<SPARSE, NWT, 4>(d, stream);
+    if (keys <= 8) return launch_keys<SPARSE, NWT, 8>(d, stream);
+    if (keys <= 16) return launch_keys<SPARSE, NWT, 16>(d, stream);
+    return hipErrorInvalidValue;
 }
 
 template <int KIND, bool ASYM, bool HAS_RES, int SPARSE, int ABL = 0>
@@ -1739,11 +1749,10 @@ static hipError_t dense_resources(int kind, bool asym, bool has_res, bool pair_h
     return resources_t<KV_INT8, false, false, 0, VAR>(pair_heads, r);
 }
 
-template <int SPARSE, int KEYS>
+template <int SPARSE, int KEYS, int NWT = 2 * NWAVES>
 static hipError_t selecting_resources(KernelResources* r) {
-    return func_resources(
-        paged_decode_kernel<KV_FP16, false, false, SPARSE, 2 * NWAVES, 1, 0, KEYS>,
-        2 * NWAVES * WAVE, r);
+    return func_resources(paged_decode_kernel<KV_FP16, false, false, SPARSE, NWT, 1, 0, KEYS>,
+                          NWT * WAVE, r);
 }
 
 hipError_t decode_resources(int kind, int walk, int var, bool asym, bool has_res,
@@ -1756,6 +1765,7 @@ hipError_t decode_resources(int kind, int walk, int var, bool asym, bool has_res
     if (walk == 1) return resources_t<KV_FP16, false, false, 1>(pair_heads, r);
     if (walk != 2 && walk != 3) return hipErrorInvalidValue;
     switch (var) {
+        case 1: return walk == 2 ? selecting_resources<2, 2, NWAVES>(r) : selecting_resources<3, 2, NWAVES>(r);
         case 2: return walk == 2 ? selecting_resources<2, 2>(r) : selecting_resources<3, 2>(r);
         case 4: return walk == 2 ? selecting_resources<2, 4>(r) : selecting_resources<3, 4>(r);
         case 8: return walk == 2 ? selecting_resources<2, 8>(r) : selecting_resources<3, 8>(r);

@@ -60,9 +60,9 @@ def kernel_resources(device: Optional[torch.device] = None, n_rep: int = 6,
     names = ("page_bounds_update", "page_index", "page_index_heads", "paged_sparse_fp16",
              "page_mass", "page_select", "page_bounds_rebuild")
     # the selecting decodes: four score keys a thread, or (by the row's length)
-    # two, eight or sixteen
+    # two, eight or sixteen; the 4-wave form of many short rows
     names += tuple(f"{n}{keys}" for n in ("sparse_attention_fp16", "sparse_attention_bounds_fp16")
-                   for keys in ("", "_keys2", "_keys8", "_keys16"))
+                   for keys in ("", "_4waves", "_keys2", "_keys8", "_keys16"))
     return {n: _lib.kernel_resources(n, device, kv_heads=kv_heads, n_rep=n_rep) for n in names}
 
 

@@ -363,7 +363,7 @@ def test_kernel_resources_report_no_spills():
             assert r["regs"] <= 256 and r["shared_bytes"] <= 160 * 1024, r
     sparse = ps.kernel_resources()
     for walk in ("sparse_attention_fp16", "sparse_attention_bounds_fp16"):
-        assert {walk + keys for keys in ("", "_keys2", "_keys8", "_keys16")} <= set(sparse)
+        assert {walk + keys for keys in ("", "_4waves", "_keys2", "_keys8", "_keys16")} <= set(sparse)
     for name, r in sparse.items():
         assert r["local_bytes"] == 0, (name, r)
         assert r["groups_per_cu"] >= 1, (name, r)

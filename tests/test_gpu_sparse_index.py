@@ -550,3 +550,28 @@ def test_bounds_of_another_block_count(width):
     got = ps().sparse_attention(*args, ratio=0.5).float()
     want = ps().sparse_attention(*args, ratio=0.5, fused=False).float()
     assert (got - want).abs().max().item() < 1e-3
+
+
+@pytest.mark.parametrize("scoring", ["bounds", "mass"])
+@pytest.mark.parametrize("b,h,n_rep,width,ratio", [
+    (257, 1, 6, 1, 0.5), (129, 2, 6, 160, 0.25), (129, 2, 8, 161, 0.25), (33, 8, 1, 320, 0.5),
+    (33, 8, 6, 321, 0.5), (256, 1, 6, 320, 0.25), (64, 8, 6, 257, 0.5), (173, 3, 6, 63, 1.0),
+    (17, 8, 6, 640, 0.25), (13, 5, 6, 481, 0.9), (24, 4, 2, 700, 0.5),
+])
+def test_batches_of_many_rows(scoring, b, h, n_rep, width, ratio):
+    """More rows than CUs (4-wave groups up to 320 pages, one launch up to 160) and
+    rows that two rounds of groups serve, at the edges of those rules, ragged
+    with an empty sequence: equal to index + select + list decode."""
+    g = torch.Generator(device="cuda").manual_seed(b + width)
+    draw = lambda *shape: torch.randn(*shape, generator=g, device="cuda").half()
+    nb = 700
+    k, v, q = draw(nb, 16, h, 128), draw(nb, 16, h, 128), draw(b, h, n_rep, 128)
+    kmin, kmax = k.amin(1), k.amax(1)
+    t = torch.stack([torch.randperm(nb, generator=g, device="cuda")[:width] for _ in range(b)]).int()
+    l = torch.randint(1, 16 * width + 1, (b,), generator=g, device="cuda").int()
+    l[0], l[1] = 16 * width, 0
+    kw = dict(ratio=ratio, scoring=scoring)
+    for rep in range(2):
+        got = ps().sparse_attention(q, k, v, t, l, kmin, kmax, **kw).float().clone()
+        want = ps().sparse_attention(q, k, v, t, l, kmin, kmax, fused=False, **kw).float()
+        assert (got - want).abs().max().item() < 1e-3, rep
