@@ -61,7 +61,7 @@ def _cus(device: torch.device) -> int:
 
 def choose_splits(batch: int, kv_heads: int, num_pages: int,
                   device: Optional[torch.device] = None, int8: bool = False,
-                  dealt: bool = True) -> int:
+                  dealt: bool = True, round_pages: Optional[int] = None) -> int:
     """Splits per (sequence, KV head) for the MI355X kernel.
 
     Enough (sequence, head, split) units for UNITS_PER_4_CUS per 4 CUs (the
@@ -74,7 +74,9 @@ def choose_splits(batch: int, kv_heads: int, num_pages: int,
     is rounded down to that where at least 4 splits a sequence remain.  With
     fewer, rounding down would idle up to half of the chip, so the rounded-up
     count stands and a dense walk's launch deals what fits by the pages.
-    ``dealt=False``: a walk whose launch does not (the page-subset walks).
+    ``dealt=False``: a walk whose launch does not (the page-subset walks); with
+    ``round_pages``, splits of more pages than that are of two rounds of groups,
+    not of one.
     """
     cus = _cus(device) if device is not None and torch.cuda.is_available() else 256
     units = UNITS_PER_4_CUS["int8" if int8 else "fp16"] * cus // 4
@@ -85,7 +87,8 @@ def choose_splits(batch: int, kv_heads: int, num_pages: int,
     if head_groups <= fit:
         whole = fit // head_groups
         if by_cus > whole and (whole >= 4 or not dealt):
-            by_cus = whole
+            long = round_pages is not None and num_pages > round_pages * whole
+            by_cus = 2 * fit // head_groups if long else whole
     elif dealt and batch <= DEAL_MAX_BATCH and num_pages >= DEAL_MIN_PAGES:
         # whole rounds: the groups that fill the last one
         by_cus = -(-(-(-head_groups // fit) * fit) // head_groups)

@@ -227,6 +227,17 @@ def budgets(seq_lens: torch.Tensor, ratio: float, recent: int = 2, page: int = 1
     return torch.minimum(n, pages).to(torch.int32)
 
 
+# Pages a split of the list walk up to which its groups are one round: over equal
+# lengths one is the fastest, over ragged ones a long sequence's few groups run
+# on alone, and two rounds of smaller groups lose little to either.  (us, full /
+# ragged lengths, one round -> two, with a first round and a few groups more, the
+# count by the CUs alone, in parentheses: B17 x 8 heads, 500 pages 89 / 54 -> 94 /
+# 44 (122 / 48), B40 x 8, 250 pages 106 / 83 -> 109 / 67 (128 / 70), B70 x 4, 125
+# pages 52 / 44 -> 55 / 40 (68 / 40); 63 pages a split and fewer: B17 x 8, 188 pages
+# 37 / 29 -> 42 / 29 (51 / 29), B40 x 8, 63 pages 30 / 24 -> 36 / 26 (41 / 27).)
+LIST_ROUND_PAGES = 64
+
+
 def sparse_decode(q, k_pool, v_pool, block_tables, seq_lens, sel,
                   num_splits: Optional[int] = None,
                   softmax_scale: Optional[float] = None,
@@ -249,7 +260,8 @@ def sparse_decode(q, k_pool, v_pool, block_tables, seq_lens, sel,
         raise ValueError("sel must be an int32 [B, H, K] tensor with unit last stride")
     b, h, n_rep, d = q.shape
     num_sel = sel.shape[-1]
-    splits = num_splits or pdh.choose_splits(b, h, num_sel, q.device, dealt=False)
+    splits = num_splits or pdh.choose_splits(b, h, num_sel, q.device, dealt=False,
+                                             round_pages=LIST_ROUND_PAGES)
     splits = max(1, min(splits, max(1, num_sel), pdh.MAX_SPLITS))
     scale = softmax_scale if softmax_scale is not None else 1.0 / math.sqrt(d)
     buf, work, cnt = pdh._buffers("sparse", b, h, splits, n_rep, q.device)

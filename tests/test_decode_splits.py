@@ -31,3 +31,28 @@ def test_more_groups_than_are_resident(int8, heads):
                 assert got == _plain(batch, heads, pages, int8), (batch, pages)
             else:                                # whole rounds, no more than one split added
                 assert got == -(-(-(-groups // fit) * fit) // groups) <= 2, (batch, pages)
+
+
+@pytest.mark.parametrize("batch,heads,pages,one,two", [
+    (13, 8, 256, 4, 9), (17, 8, 192, 3, 7), (22, 8, 128, 2, 5), (33, 8, 64, 1, 3), (50, 8, 64, 1, 2),
+    (129, 1, 192, 3, 7),
+])
+def test_list_walks_of_long_splits_take_two_rounds(batch, heads, pages, one, two):
+    """The page-subset walk's launch deals nothing: where whole rounds round the
+    count down, a long sequence's few groups would run on alone."""
+    from latentserve_amd.kernels.hip import paged_sparse as ps
+
+    def count(n, **kw):
+        return pdh.choose_splits(batch, heads, n, None, dealt=False, **kw)
+
+    assert ps.LIST_ROUND_PAGES == 64
+    assert count(pages, round_pages=64) == count(pages) == one
+    assert count(pages + 1, round_pages=64) == two
+    assert count(pages + 1) == one                     # selecting walks: one round
+
+
+@pytest.mark.parametrize("batch,heads", [(1, 2), (8, 2), (16, 8), (65, 8), (200, 4)])
+def test_list_walks_elsewhere_as_without_the_rule(batch, heads):
+    for pages in (1, 60, 500, 8192):
+        assert pdh.choose_splits(batch, heads, pages, None, dealt=False, round_pages=64) == \
+            pdh.choose_splits(batch, heads, pages, None, dealt=False)
