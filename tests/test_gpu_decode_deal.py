@@ -76,3 +76,23 @@ def test_chosen_splits_are_resident_or_dealt():
                 assert s <= 4 or groups * s <= fit, (b, h, s)
                 s = pdh.choose_splits(b, h, 4096, torch.device("cuda", 0), int8=int8, dealt=False)
                 assert s == 1 or groups * s <= fit, (b, h, s)
+
+
+@pytest.mark.parametrize("over", [0, 1, 2, 3, 40])
+@pytest.mark.parametrize("b,h,splits", [(2, 2, 5), (3, 3, 5), (60, 8, 2)])
+def test_host_partition_over_the_even_one(b, h, splits, over):
+    """A host length whose shares are that many pages over even ones (the host's
+    partition up to two, even shares past it), equal lengths, full and ragged
+    last pages, undealt and dealt groups."""
+    from latentserve_amd.kernels.hip import paged_decode_hip as pdh
+    for tokens in (50 * 16, 50 * 16 - 3, 47 * 16 + 1):
+        max_len = (10 + over) * 16 * splits if splits == 5 else (25 + over) * 16 * splits
+        case = paged_case([tokens] * b, h_kv=h, n_rep=4, seed=b + over, width=max_len // 16 if b < 9 else None)
+        got = pdh.paged_decode_hip(*_gpu(case), max_len, num_splits=splits)
+        assert_close(got.float().cpu().numpy(), oracle.paged_decode(*case), 2e-3, 1e-2,
+                     f"{b} {h} {splits} {tokens} {max_len}")
+        case, extra = int8_case([tokens] * b, asym=False, h_kv=h, n_rep=4, seed=b + over)
+        dev = {n: _gpu([x])[0] for n, x in extra.items()}
+        got = pdh.paged_decode_hip(*_gpu(case), max_len, num_splits=splits, **dev)
+        assert_close(got.float().cpu().numpy(), oracle.paged_decode(*case, **extra), 2e-3, 1e-2,
+                     f"int8 {b} {h} {splits} {tokens} {max_len}")
