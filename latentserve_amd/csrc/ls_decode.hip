@@ -884,6 +884,20 @@ __device__ __forceinline__ float score_one(const DecodeParams& a, int b, int h, 
     return bst;
 }
 
+// INT8, dealt: workgroup L of n (dispatched to XCD L % 8) -> its place in the order
+// [unit][head group], the n_hg head groups of a unit on one XCD (its whole eights
+// of units; the rest in order).  A token's V scales of all heads are a few dozen
+// adjacent bytes, so head groups on different XCDs each bring the same lines (us,
+// in the launch's order -> so, ragged lengths, 8 heads: B250 to 1000 88.9 -> 84.0,
+// B72 to 1000 33.7 -> 31.3, B200 to 500 45.8 -> 42.3, asymmetric 53.1 -> 48.7; 4
+// heads, B250 to 3000 117.4 -> 115.4; fp16, without scales, 1 % slower at full
+// lengths).
+__device__ __forceinline__ int xcd_heads(int L, int n, int n_hg) {
+    if (L >= n / (8 * n_hg) * (8 * n_hg)) return L;
+    const int i = L / 8;
+    return (i / n_hg * 8 + L % 8) * n_hg + i % n_hg;
+}
+
 // SPARSE: 0 the dense walk; 1 a page-subset walk over the caller's lists;
 // 2 a page-subset walk whose lists the group selects from page scores;
 // 3 the same with the scores computed by the launch itself, each group
@@ -938,7 +952,9 @@ void paged_decode_kernel(const DecodeParams a) {
     // 50.3 -> 49.8 us; the page-subset walks measured slower so, c5 50.0 ->
     // 51.2 us, and keep the dispatch order)
     const int L = blockIdx.x + gridDim.x * blockIdx.y;
-    const int wg = SPARSE || DEAL ? L : xcd_major(L, gridDim.x * gridDim.y);
+    const int wg = DEAL && KIND == KV_INT8 ? xcd_heads(L, gridDim.x, n_hg)
+                   : SPARSE || DEAL        ? L
+                                           : xcd_major(L, gridDim.x * gridDim.y);
     const int S = a.num_splits;
     // (DEAL 1: the grid is a.groups x n_hg; groups past B x S guess the last
     // sequence, a split it does not have)
