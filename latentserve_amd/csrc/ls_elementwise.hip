@@ -160,6 +160,12 @@ __global__ __launch_bounds__(NORM_THREADS) void rms_norm_any_kernel(NormParams a
     }
 }
 
+// NT: the result stored past the caches (4099 rows of 8960, 220 MB, 36.7 -> 34.8
+// us; the loads so as well, 36.4).  Only of whole 128-byte lines, since a line
+// written in parts by two waves so costs two writes (300 rows of 1544 2.71 -> 3.06
+// us, plain 2.71), and from 2 MB on: less stays in the caches for the product
+// behind it (64 rows of 1024 2.23 -> 2.30; 300 rows of 8960, 5.4 MB, 4.66 -> 4.37).
+template <bool NT>
 __global__ __launch_bounds__(256) void silu_mul_vec_kernel(SiluParams a) {
     const int64_t row = blockIdx.y;
     const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
@@ -170,9 +176,11 @@ __global__ __launch_bounds__(256) void silu_mul_vec_kernel(SiluParams a) {
     unpack8(*(const u4*)(gu + a.inter + i), u);
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = silu_mul_h(g[e], u[e]);
-    // (nontemporal: 4099 rows of 8960, 220 MB, 36.7 -> 34.8 us; the loads so
-    // as well, 36.4)
-    __builtin_nontemporal_store(pack8(o), (u4*)((half_t*)a.out + row * a.so + i));
+    u4* dst = (u4*)((half_t*)a.out + row * a.so + i);
+    if (NT)
+        __builtin_nontemporal_store(pack8(o), dst);
+    else
+        *dst = pack8(o);
 }
 
 __global__ __launch_bounds__(256) void silu_mul_any_kernel(SiluParams a) {
@@ -447,8 +455,12 @@ hipError_t launch_silu_and_mul(const SiluParams& p, hipStream_t stream) {
     if (p.rows == 0 || p.inter == 0) return hipSuccess;
     if (p.vec) {
         const int per = 256 * 8;
-        hipLaunchKernelGGL(silu_mul_vec_kernel, dim3((p.inter + per - 1) / per, p.rows), dim3(256),
-                           0, stream, p);
+        const dim3 grid((p.inter + per - 1) / per, p.rows);
+        const bool lines = (((uintptr_t)p.out | (uint64_t)p.so * 2 | (uint64_t)p.inter * 2) & 127) == 0;
+        if (lines && (int64_t)p.rows * p.inter * 2 >= (2 << 20))
+            hipLaunchKernelGGL(silu_mul_vec_kernel<true>, grid, dim3(256), 0, stream, p);
+        else
+            hipLaunchKernelGGL(silu_mul_vec_kernel<false>, grid, dim3(256), 0, stream, p);
     } else {
         hipLaunchKernelGGL(silu_mul_any_kernel, dim3((p.inter + 255) / 256, p.rows), dim3(256), 0,
                            stream, p);

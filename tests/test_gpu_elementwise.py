@@ -90,6 +90,22 @@ def test_silu_and_mul(inter):
     assert d.max() <= 2 and (d == 0).mean() > 0.99
 
 
+@pytest.mark.parametrize("rows,inter,shift", [(128, 8192, 0), (127, 8192, 0), (300, 3584, 0),
+                                              (300, 3592, 0), (300, 3584, 8), (1, 64, 0)])
+def test_silu_and_mul_stores(rows, inter, shift):
+    """Results stored past the caches (whole 128-byte lines, from 2 MB on) and
+    plainly, into a buffer that starts on a line and one that does not."""
+    rng = np.random.default_rng(rows + inter)
+    gu = (rng.standard_normal((rows, 2 * inter)) * 3).astype(np.float16)
+    buf = torch.full((rows * inter + 128,), 7.0, dtype=torch.float16, device="cuda")
+    out = buf[64 + shift:64 + shift + rows * inter].view(rows, inter)
+    fe().silu_and_mul(g(gu), out=out)
+    torch.cuda.synchronize()
+    d = ulps(out.cpu().numpy(), oracle.silu_and_mul(gu))
+    assert d.max() <= 2 and (d == 0).mean() > 0.99      # as above
+    assert bool((buf[:64 + shift] == 7).all()) and bool((buf[64 + shift + rows * inter:] == 7).all())
+
+
 def test_rope_qk_on_a_strided_slice_is_bit_exact():
     """q and k arrive as slices of the fused q/k/v output, their rows strided
     by the whole projection width."""
