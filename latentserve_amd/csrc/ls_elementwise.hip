@@ -195,7 +195,11 @@ __global__ __launch_bounds__(256) void silu_mul_any_kernel(SiluParams a) {
 // their pairs d/2 further.  Bandwidth-bound from about 1000 rows: 4099 rows of
 // 14 heads of 128 (32 MB) 16.2 us as two-byte loads, one pair a thread (the
 // kernel below, for other widths and alignments) -> 6.8 us.  (Two heads a
-// thread, the angles read once for both, 7.0 us; four 8.8.)
+// thread, the angles read once for both, 7.0 us; four 8.8.)  Of few heads a
+// thread's eight pairs are the longer chain (us, the kernel below -> this one,
+// rows x heads: 16 x 14 2.19 -> 2.37, 33 x 40 2.31 -> 2.42, 130 x 14 2.37 -> 2.45;
+// 64 x 40 2.47 -> 2.45, 300 x 14 2.86 -> 2.54), so it takes ROPE_VEC_HEADS.
+constexpr int ROPE_VEC_HEADS = 2400;
 __global__ __launch_bounds__(256) void rope_qk_vec_kernel(RopeParams a) {
     const int hd = a.d / 2, pieces = hd / 8, heads = a.hq + a.hk;
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -471,7 +475,8 @@ hipError_t launch_silu_and_mul(const SiluParams& p, hipStream_t stream) {
 hipError_t launch_rope_qk(const RopeParams& p, hipStream_t stream) {
     if (p.rows == 0) return hipSuccess;
     const int64_t blocks = ((int64_t)p.rows * (p.hq + p.hk) * (p.d / 16) + 255) / 256;
-    if (p.vec && p.d % 16 == 0 && blocks <= 0x7fffffff)
+    if (p.vec && p.d % 16 == 0 && (int64_t)p.rows * (p.hq + p.hk) >= ROPE_VEC_HEADS &&
+        blocks <= 0x7fffffff)
         hipLaunchKernelGGL(rope_qk_vec_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, p);
     else
         hipLaunchKernelGGL(rope_qk_kernel, dim3(p.rows, p.hq + p.hk), dim3(p.d / 2), 0, stream, p);

@@ -145,6 +145,9 @@ def test_rope_qk_broadcast_table():
     (70, 5, 4, 1024, 0),         # the widest head
     (9, 2, 1, 24, 0),            # a half that is not whole pieces
     (9, 12, 2, 128, 1),          # rows not 16-byte aligned
+    (1199, 1, 1, 16, 0), (1200, 1, 1, 16, 0),      # either side of the pieces' fewest heads
+    (801, 2, 1, 128, 0), (300, 5, 4, 1024, 0), (601, 3, 1, 32, 0),
+    (300, 6, 4, 24, 0), (200, 12, 2, 128, 1),
 ])
 def test_rope_qk_pieces_are_bit_exact(rows, hq, hk, d, shift):
     rng = np.random.default_rng(rows + d)
