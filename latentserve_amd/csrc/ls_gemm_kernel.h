@@ -477,7 +477,14 @@ __global__ __launch_bounds__(GEMM_WAVES* WAVE) void decode_gemm_kernel(GemmParam
 template <int MB, int EPI, bool PW, bool NRM = false>
 void launch_spw(const GemmParams& p, int spw, dim3 grid, hipStream_t stream) {
     const dim3 block(GEMM_WAVES * WAVE);
-    if (spw <= 4)
+    // (K up to 512: a group stages no more of X than it has.  us, four steps ->
+    // two: 1000 x 96 at M 64 4.93 -> 3.77, 16384 x 256 at M 64 8.46 -> 7.01, 4096 x
+    // 512 at M 64 5.56 -> 4.46.  The other epilogues, whose K is a hidden size,
+    // have no such form.)
+    constexpr int FEW = EPI == GEMM_PLAIN && !NRM ? 2 : 4;
+    if (FEW == 2 && spw <= 2)
+        hipLaunchKernelGGL((decode_gemm_kernel<FEW, MB, EPI, PW, NRM, false>), grid, block, 0, stream, p);
+    else if (spw <= 4)
         hipLaunchKernelGGL((decode_gemm_kernel<4, MB, EPI, PW, NRM, false>), grid, block, 0, stream, p);
     else if (spw <= 6)
         hipLaunchKernelGGL((decode_gemm_kernel<6, MB, EPI, PW, NRM, false>), grid, block, 0, stream, p);

@@ -36,7 +36,7 @@ def _operands(m, n, k):
 @pytest.mark.parametrize("m", [1, 16, 17, 32, 33, 48, 49, 64])
 @pytest.mark.parametrize("n,k", [(16, 32), (5, 96), (100, 1024), (4100, 288), (8200, 1120),
                                  (12300, 1536), (300, 2048), (50, 2080), (1536, 8960),
-                                 (2000, 4864)])
+                                 (2000, 4864), (40, 480), (5000, 512), (47, 544)])
 def test_product(m, n, k):
     x, w, b = _operands(m, n, k)
     want = x.double() @ w.double().t() + b.double()
