@@ -288,14 +288,17 @@ COOP_MAX_NREP = 8
 # row over the chip, which a short row's groups would leave idle.  So one launch
 # up to a batch a group, and up to COOP_MAX_PAGES where the rows are few enough
 # that the launch it saves counts.  (us, ratio 0.25, full / ragged lengths, one
-# launch -> two: B18 x 4 heads to 8000 28.2 / 23.6 -> 27.2 / 22.4, B17 x 8 to
+# launch -> two: B12 x 8 heads to 8000 34.1 / 29.6 -> 32.4 / 27.2, B17 x 8 to
 # 5000 34.0 / 31.6 -> 30.2 / 27.2, to 32000 176 / 134 -> 142 / 99, B32 x 8 to
 # 16000 121 / 89 -> 116 / 82, B8 x 8 to 100K 190 / 127 -> 180 / 109; under a
 # batch, B16 x 8 to 1500 15.6 / 14.4 -> 17.0 / 16.1, B24 x 8 to 2500 22.8 / 20.5 ->
 # 23.3 / 20.4, B32 x 8 to 2500 25.2 / 21.4 -> 26.5 / 21.7.)
+# The second launch is 12 us of host work, which calls outside a graph spend: only
+# with pages enough in all rows to take longer than that on the GPU.
 SELECT_GROUPS = 256
 SCORE_BATCH = 160
 FEW_ROWS = 64
+TWO_LAUNCH_MIN_PAGES = 40000
 # In two launches the groups need not be resident together: where the whole groups
 # a row that are leave CUs idle (129 to 170 rows: one, on up to half of them), two
 # rounds of an odd count fill them, from this many selected pages a group on (us,
@@ -309,7 +312,8 @@ def _one_launch(rows: int, width: int) -> bool:
     """Whether the groups of `rows` (sequence, KV head) rows of `width` pages score
     the pages themselves."""
     share = -(-width // max(1, SELECT_GROUPS // max(1, rows)))
-    return share <= SCORE_BATCH or (rows <= FEW_ROWS and width <= COOP_MAX_PAGES)
+    return (share <= SCORE_BATCH or rows * width < TWO_LAUNCH_MIN_PAGES
+            or (rows <= FEW_ROWS and width <= COOP_MAX_PAGES))
 
 
 def _two_rounds(rows: int, k: int) -> int:

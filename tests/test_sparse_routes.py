@@ -75,9 +75,10 @@ def test_every_row_width_counts_in_a_buffer_of_its_own(library):
 @pytest.mark.parametrize("batch,heads,width,one", [
     (2, 2, 2048, True), (2, 2, 8192, True),           # 64 groups a row: 128 pages each
     (8, 8, 2048, True), (8, 8, 2049, False),          # 64 rows, four groups each
-    (13, 5, 480, True), (13, 5, 481, False),          # 65 rows, three groups each
+    (13, 5, 480, True), (13, 5, 616, False),          # 65 rows, three groups each
+    (13, 5, 615, True), (17, 8, 294, True),           # under 40000 pages in all
     (16, 8, 320, True), (16, 8, 321, False),
-    (17, 8, 160, True), (17, 8, 161, False),          # a group a row
+    (17, 8, 160, True), (17, 8, 295, False),          # a group a row
     (33, 8, 160, True), (33, 8, 161, False), (200, 8, 161, False),
     (25, 6, 6250, False),                             # more than a group a row needed
 ])
