@@ -76,7 +76,7 @@ def choose_splits(batch: int, kv_heads: int, num_pages: int,
     count stands and a dense walk's launch deals what fits by the pages.
     ``dealt=False``: a walk whose launch does not (the page-subset walks); with
     ``round_pages``, splits of more pages than that are of two rounds of groups,
-    not of one.
+    not of one, where those are an odd count.
     """
     cus = _cus(device) if device is not None and torch.cuda.is_available() else 256
     units = UNITS_PER_4_CUS["int8" if int8 else "fp16"] * cus // 4
@@ -87,8 +87,9 @@ def choose_splits(batch: int, kv_heads: int, num_pages: int,
     if head_groups <= fit:
         whole = fit // head_groups
         if by_cus > whole and (whole >= 4 or not dealt):
+            two = 2 * fit // head_groups
             long = round_pages is not None and num_pages > round_pages * whole
-            by_cus = 2 * fit // head_groups if long else whole
+            by_cus = two if long and two > 2 * whole else whole
     elif dealt and batch <= DEAL_MAX_BATCH and num_pages >= DEAL_MIN_PAGES:
         # whole rounds: the groups that fill the last one
         by_cus = -(-(-(-head_groups // fit) * fit) // head_groups)

@@ -230,12 +230,12 @@ def budgets(seq_lens: torch.Tensor, ratio: float, recent: int = 2, page: int = 1
 # Pages a split of the list walk up to which its groups are one round: over equal
 # lengths one is the fastest, over ragged ones a long sequence's few groups run
 # on alone, and two rounds of smaller groups lose little to either.  (us, full /
-# ragged lengths, one round -> two, with a first round and a few groups more, the
-# count by the CUs alone, in parentheses: B17 x 8 heads, 500 pages 89 / 54 -> 94 /
-# 44 (122 / 48), B40 x 8, 250 pages 106 / 83 -> 109 / 67 (128 / 70), B70 x 4, 125
-# pages 52 / 44 -> 55 / 40 (68 / 40); 63 pages a split and fewer: B17 x 8, 188 pages
-# 37 / 29 -> 42 / 29 (51 / 29), B40 x 8, 63 pages 30 / 24 -> 36 / 26 (41 / 27).)
-LIST_ROUND_PAGES = 64
+# ragged lengths, one round -> two, with the count by the CUs alone, a round and a
+# few groups more, in parentheses: B17 x 8 heads, 500 pages 94 / 56 -> 99 / 45 (126 /
+# 49), B40 x 8, 250 pages 114 / 88 -> 115 / 69 (135 / 72), B70 x 4, 125 pages 55 /
+# 47 -> 58 / 40 (69 / 40); 79 to 83 pages a split: B33 x 8 34 / 29 -> 39 / 28 (47 /
+# 30), B17 x 8 49 / 40 -> 53 / 40 (67 / 36).)
+LIST_ROUND_PAGES = 96
 
 
 def sparse_decode(q, k_pool, v_pool, block_tables, seq_lens, sel,
