@@ -35,9 +35,9 @@ from latentserve_amd.runtime.int8_cache import Int8PagedKVCache
 from latentserve_amd.runtime.kv_cache import KVCacheSpec, PagedKVCache
 
 
-# Rows up to which a norm folds into the projection behind it, and up to which
-# packed weights are the ones to hand to the projections one by one (above, the
-# row-major ones take every launch kind).
+# Rows up to which a norm folds into the projection behind it: the GEMM's norm
+# prologue takes one column block of 16 rows.  (What a packed weight cannot do,
+# gate/up and q/k/v with K split over workgroups, it cannot do at any row count.)
 HIP_GEMM_MAX_ROWS = 16
 # Rows up to which the decoder's projections run on the HIP GEMM, which streams
 # the weights faster than hipBLASLt (M 16 / 64, us: gate/up 12.8 against 39 /
