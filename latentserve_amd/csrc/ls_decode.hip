@@ -1131,10 +1131,10 @@ void paged_decode_kernel(const DecodeParams a) {
     // time, dealt groups too.  us, fp16 / INT8, before -> with even shares: B26 x
     // 4 heads, lengths to 30000 180 / 149 -> 130 / 100, B16 x 2 of 8K tokens at a
     // host's length of 16K 32.7 / 25.9 -> 25.8 / 19.4.)
-    const int even = (num_pages + S - 1) / S;
+    // (pages_per_split <= ceil(num_pages / S) + 2, without the division)
     const bool spec_ok = host_split && b == hb && Sb == S && gw.s == split &&
                          num_pages <= S * a.pages_per_split &&
-                         (S == 1 || a.pages_per_split <= even + 2);
+                         (S == 1 || num_pages > S * (a.pages_per_split - 3));
     int lo, hi;
     if (spec_ok) {
         lo = spec_lo;
