@@ -215,10 +215,17 @@ def kernel_resources(kernel: str, device: Optional[torch.device] = None, kv_head
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)    # (None: a torch without GPUs)
 
 
+# GPU device -> its index: one lookup a launch (the string of `device.type` costs
+# more than the stream's own, 218 ns against 99).
+_GPU_INDEX = {torch.device("cuda", i): i for i in range(128)}
+
+
 def stream_of(device: torch.device) -> int:
     """torch's current stream on `device` as a hipStream_t.  Every launch asks
     for it, and for several entry points this is what refuses CPU tensors."""
-    if device.type != "cuda":
-        raise ValueError(f"Expected a cuda device, but got: {device}")
-    index = device.index
-    return _raw_stream(torch.cuda.current_device() if index is None else index)
+    index = _GPU_INDEX.get(device)
+    if index is None:
+        if device.type != "cuda":
+            raise ValueError(f"Expected a cuda device, but got: {device}")
+        index = torch.cuda.current_device()
+    return _raw_stream(index)

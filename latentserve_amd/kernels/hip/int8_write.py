@@ -129,15 +129,16 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
     its last page to row rows[b] (int64 [B]) of k_res [R, 16, H, D] (where the
     rows before the chunk in its first page are).  k_quant, v_quant: (eps,
     qmax, levels, offset).  One launch."""
-    b, h, n, d = k.shape
+    shape = k.shape
+    b, h, n, d = shape
     dev = k.get_device()                      # (-1: not on a GPU)
     if dev < 0 or v.get_device() != dev or k.dtype != torch.float16 or v.dtype != torch.float16 \
-            or d != HEAD_DIM or v.shape != k.shape:
+            or d != HEAD_DIM or v.shape != shape:
         raise ValueError("prefill_write: k and v must be fp16 [B, H, n, 128] GPU tensors")
     if slots.dtype != torch.int64 or slots.shape != (b, n) or not slots.is_contiguous() \
             or slots.get_device() != dev:
         raise ValueError("slots must be a contiguous int64 [B, n] tensor on k's device")
-    if rows.dtype != torch.int64 or rows.dim() != 1 or rows.shape[0] < b or rows.stride(0) != 1 \
+    if rows.dtype != torch.int64 or rows.dim() != 1 or rows.numel() < b or rows.stride() != (1,) \
             or rows.get_device() != dev:
         raise ValueError("rows must be a unit-stride int64 [B] tensor on k's device")
     nb, nr = k_pool.shape[0], k_res.shape[0]
@@ -153,12 +154,14 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
         if t.dtype != dt or t.shape != shape or not t.is_contiguous() or t.get_device() != dev:
             raise ValueError(f"{name} must be contiguous {dt} {shape} on k's device")
     k, v = _loadable(k, 4), _loadable(v, 16)
-    P, S = _lib.ptr, _lib.strides
+    S = _lib.strides
     eps, qmax, levels, offset = k_quant
     v_eps, v_qmax, v_levels, v_offset = v_quant
     rc = _lib.lib().ls_int8_prefill_write(
-        P(k), S(k, 3), P(v), S(v, 3), P(slots), P(rows), P(k_pool), P(k_scale),
-        P(k_zero) if asym else None, P(v_pool), P(v_scale), P(v_zero) if asym else None, P(k_res),
+        k.data_ptr(), S(k, 3), v.data_ptr(), S(v, 3), slots.data_ptr(), rows.data_ptr(),
+        k_pool.data_ptr(), k_scale.data_ptr(), k_zero.data_ptr() if asym else None,
+        v_pool.data_ptr(), v_scale.data_ptr(), v_zero.data_ptr() if asym else None,
+        k_res.data_ptr(),
         nb, nr, b, h, n, d, PAGE, int(bool(asym)), eps, qmax, levels, offset,
         0 if exact_division else 1, v_eps, v_qmax, v_levels, v_offset, _lib.stream_of(k.device))
     _lib.check(rc, "ls_int8_prefill_write")

@@ -18,12 +18,6 @@ from latentserve_amd import _lib
 PAGE = 16
 
 
-def _same_device(pool: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tensor) -> None:
-    dev = pool.get_device()
-    if block_tables.get_device() != dev or seq_lens.get_device() != dev:
-        raise ValueError("block tables and sequence lengths must be on the pool's device")
-
-
 def gather(pool: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tensor,
            length: Optional[int] = None, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """pool [nb, 16, H, D] (fp16 / int8 / fp32) -> [B, H, length, D] view.
@@ -35,7 +29,9 @@ def gather(pool: torch.Tensor, block_tables: torch.Tensor, seq_lens: torch.Tenso
     if block_tables.dtype != torch.int32 or seq_lens.dtype != torch.int32 \
             or block_tables.stride(-1) != 1 or seq_lens.stride(-1) != 1:
         raise ValueError("block tables and sequence lengths must be unit-stride int32")
-    _same_device(pool, block_tables, seq_lens)
+    dev = pool.get_device()
+    if block_tables.get_device() != dev or seq_lens.get_device() != dev:
+        raise ValueError("block tables and sequence lengths must be on the pool's device")
     nb, _, h, d = pool.shape
     b = block_tables.shape[0]
     length = block_tables.shape[1] * PAGE if length is None else int(length)
@@ -57,24 +53,26 @@ def read(k_pool: torch.Tensor, v_pool: torch.Tensor, block_tables: torch.Tensor,
          seq_lens: torch.Tensor, length: Optional[int] = None):
     """(k, v) [B, H, L, D] for one layer: PagedKVCache.read's result.  One
     launch where the pools are alike (a K and a V pool of one cache)."""
+    dev = k_pool.get_device()
     if k_pool.dim() != 4 or k_pool.shape != v_pool.shape or k_pool.stride() != v_pool.stride() \
-            or k_pool.dtype != v_pool.dtype or k_pool.device != v_pool.device \
+            or k_pool.dtype != v_pool.dtype or v_pool.get_device() != dev \
             or k_pool.shape[1] != PAGE or k_pool.stride(-1) != 1:
         return (gather(k_pool, block_tables, seq_lens, length),
                 gather(v_pool, block_tables, seq_lens, length))
     if block_tables.dtype != torch.int32 or seq_lens.dtype != torch.int32 \
             or block_tables.stride(-1) != 1 or seq_lens.stride(-1) != 1:
         raise ValueError("block tables and sequence lengths must be unit-stride int32")
-    _same_device(k_pool, block_tables, seq_lens)
+    if block_tables.get_device() != dev or seq_lens.get_device() != dev:
+        raise ValueError("block tables and sequence lengths must be on the pools' device")
     nb, _, h, d = k_pool.shape
     b = block_tables.shape[0]
     length = block_tables.shape[1] * PAGE if length is None else int(length)
-    k, v = (torch.empty(b, length, h, d, dtype=k_pool.dtype, device=k_pool.device)
-            for _ in range(2))
+    device = k_pool.device
+    k, v = (torch.empty(b, length, h, d, dtype=k_pool.dtype, device=device) for _ in range(2))
     P, S = _lib.ptr, _lib.strides
     rc = _lib.lib().ls_paged_read(
         P(k_pool), P(v_pool), k_pool.element_size(), S(k_pool, 3), nb, P(block_tables),
         block_tables.stride(0), block_tables.shape[1], P(seq_lens), P(k), P(v), S(k, 3), b, h, d,
-        PAGE, length, _lib.stream_of(k_pool.device))
+        PAGE, length, _lib.stream_of(device))
     _lib.check(rc, "ls_paged_read")
     return k.permute(0, 2, 1, 3), v.permute(0, 2, 1, 3)
