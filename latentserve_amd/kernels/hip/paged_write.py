@@ -26,8 +26,8 @@ def write(k: torch.Tensor, v: torch.Tensor, slots: torch.Tensor, k_pool: torch.T
 
     False, with nothing done, where the kernel does not apply: CPU tensors,
     another type than the pools', rows that do not start on 16 bytes or whose
-    channels are not adjacent, gradients to record, or rows that lie in the
-    pools themselves (the order of the kernel's reads and stores is not
+    channels are not adjacent, gradients to record, or rows whose span
+    meets the pools (the order of the kernel's reads and stores is not
     defined)."""
     shape, pshape = k.shape, k_pool.shape
     b, h, n, d = shape
@@ -35,6 +35,10 @@ def write(k: torch.Tensor, v: torch.Tensor, slots: torch.Tensor, k_pool: torch.T
     ks, vs, ps = k.stride(), v.stride(), k_pool.stride()
     kp, vp, kpp, vpp = k.data_ptr(), v.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr()
     pool_bytes = k_pool.numel() * size
+    # (the bytes that k and v span, gaps between their rows included)
+    k_end = kp + ((b - 1) * ks[0] + (h - 1) * ks[1] + (n - 1) * ks[2] + d) * size
+    v_end = vp + ((b - 1) * vs[0] + (h - 1) * vs[1] + (n - 1) * vs[2] + d) * size
+    k_pool_end, v_pool_end = kpp + pool_bytes, vpp + pool_bytes
     dev = k.device
     if not (dev.type == "cuda" and dev == v.device == k_pool.device == v_pool.device
             and k.dtype == v.dtype == k_pool.dtype == v_pool.dtype and size in (1, 2, 4)
@@ -44,7 +48,8 @@ def write(k: torch.Tensor, v: torch.Tensor, slots: torch.Tensor, k_pool: torch.T
             and ks[3] == 1 == vs[3]
             and not ((ks[0] | ks[1] | ks[2] | vs[0] | vs[1] | vs[2] | d) * size
                      | kp | vp | kpp | vpp) & 15
-            and not any(pool <= p < pool + pool_bytes for p in (kp, vp) for pool in (kpp, vpp))
+            and (kp >= k_pool_end or k_end <= kpp) and (kp >= v_pool_end or k_end <= vpp)
+            and (vp >= k_pool_end or v_end <= kpp) and (vp >= v_pool_end or v_end <= vpp)
             and not (torch.is_grad_enabled() and (k.requires_grad or v.requires_grad))):
         return False
     if slots.dtype != torch.int64 or slots.shape != (b * n,) or slots.stride(0) != 1 \

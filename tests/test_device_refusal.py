@@ -152,3 +152,24 @@ def test_one_operand_on_the_cpu_is_refused(library):
         assert library.launched == [], (fn.__name__, name)
     whole()
     assert library.launched == ["ls_int8_prefill_write"]
+
+
+@pytest.mark.gpu
+@pytest.mark.skipif(not torch.cuda.is_available(), reason="needs a GPU")
+@pytest.mark.parametrize("before", [0, 3, 39, 40, -5])
+def test_paged_write_leaves_rows_that_meet_the_pool(library, before):
+    """Rows that start inside a pool, or before it and run into it, are not the
+    kernel's (it reads and stores in no defined order); rows that end where it
+    starts are.  (The recorder takes the launch's place.)"""
+    from latentserve_amd.kernels.hip import paged_write as pw
+    n = 40                                               # rows of k; `before` of them before the pool
+    buf = torch.zeros(n + NB * 16, 1, D, dtype=torch.float16, device="cuda")
+    k = buf[n - before:2 * n - before].view(1, n, 1, D).transpose(1, 2)
+    k_pool, v_pool = buf[n:].view(NB, 16, 1, D), torch.zeros_like(buf[n:]).view(NB, 16, 1, D)
+    slots = torch.arange(n, device="cuda")
+    other = torch.zeros_like(k)
+    for args in ((k, other, slots, k_pool, v_pool), (other, k, slots, k_pool, v_pool),
+                 (k, other, slots, v_pool, k_pool), (other, k, slots, v_pool, k_pool)):
+        library.launched.clear()
+        assert pw.write(*args) is (before == n)
+        assert library.launched == (["ls_paged_write"] if before == n else [])
