@@ -17,6 +17,7 @@ stores when it runs on a GPU and what its int8_write.cu computes.
 
 from __future__ import annotations
 
+import ctypes
 from typing import Optional
 
 import torch
@@ -25,6 +26,7 @@ from latentserve_amd import _lib
 
 HEAD_DIM = 128
 PAGE = 16
+_I64x3 = ctypes.c_int64 * 3
 
 
 def eligible(k: torch.Tensor, v: torch.Tensor) -> bool:
@@ -150,26 +152,33 @@ def prefill_write(k, v, slots, rows, k_pool, k_scale, k_zero, v_pool, v_scale, v
         if k_zero is None or v_zero is None:
             raise ValueError("asymmetric quantization needs k_zero and v_zero")
         pools += [(k_zero, "k_zero", f32, (nb, h, d)), (v_zero, "v_zero", f32, (nb, PAGE, h))]
-    for t, name, dt, shape in pools:
-        if t.dtype != dt or t.shape != shape or not t.is_contiguous() or t.get_device() != dev:
-            raise ValueError(f"{name} must be contiguous {dt} {shape} on k's device")
-    k, v = _loadable(k, 4), _loadable(v, 16)
-    S = _lib.strides
+    for t, name, dt, like in pools:
+        if t.dtype != dt or t.shape != like or not t.is_contiguous() or t.get_device() != dev:
+            raise ValueError(f"{name} must be contiguous {dt} {like} on k's device")
+    res = k_res.data_ptr()
+    res_end = res + 2 * nr * PAGE * h * d
+    k, ks = _loadable(k, shape, 4, res, res_end)
+    v, vs = _loadable(v, shape, 16, res, res_end)
     eps, qmax, levels, offset = k_quant
     v_eps, v_qmax, v_levels, v_offset = v_quant
     rc = _lib.lib().ls_int8_prefill_write(
-        k.data_ptr(), S(k, 3), v.data_ptr(), S(v, 3), slots.data_ptr(), rows.data_ptr(),
+        k.data_ptr(), ks, v.data_ptr(), vs, slots.data_ptr(), rows.data_ptr(),
         k_pool.data_ptr(), k_scale.data_ptr(), k_zero.data_ptr() if asym else None,
         v_pool.data_ptr(), v_scale.data_ptr(), v_zero.data_ptr() if asym else None,
-        k_res.data_ptr(),
-        nb, nr, b, h, n, d, PAGE, int(bool(asym)), eps, qmax, levels, offset,
+        res, nb, nr, b, h, n, d, PAGE, int(bool(asym)), eps, qmax, levels, offset,
         0 if exact_division else 1, v_eps, v_qmax, v_levels, v_offset, _lib.stream_of(k.device))
     _lib.check(rc, "ls_int8_prefill_write")
 
 
-def _loadable(t: torch.Tensor, nbytes: int) -> torch.Tensor:
-    """t, or a contiguous copy where its rows are not unit-stride and aligned
-    to the kernel's loads."""
+def _loadable(t: torch.Tensor, shape, nbytes: int, lo: int, hi: int):
+    """t, or a contiguous copy where its rows are not unit-stride and aligned to
+    the kernel's loads or its span meets the bytes [lo, hi) that the launch
+    stores to; and its first three strides."""
     sb, sh, st, sd = t.stride()
-    ok = sd == 1 and not (t.data_ptr() | 2 * (sb | sh | st)) % nbytes
-    return t if ok else t.clone(memory_format=torch.contiguous_format)
+    p = t.data_ptr()
+    b, h, n, d = shape
+    if sd != 1 or (p | 2 * (sb | sh | st)) % nbytes \
+            or p < hi and lo < p + 2 * ((b - 1) * sb + (h - 1) * sh + (n - 1) * st + d):
+        t = t.clone(memory_format=torch.contiguous_format)
+        sb, sh, st, _ = t.stride()
+    return t, _I64x3(sb, sh, st)

@@ -154,3 +154,48 @@ def test_int8_chunk_takes_ks_and_vs_own_eps(asym):
         if asym:
             assert np.array_equal(vz.view(-1, h)[:n].cpu().numpy(), zero)
             assert np.array_equal(kz[:2].cpu().numpy(), kzero)
+
+
+@pytest.mark.parametrize("which", ["k", "v"])
+@pytest.mark.parametrize("first", [0, 16, 24])
+def test_int8_chunk_read_from_the_residual(monkeypatch, which, first):
+    """k or v that lies in the residual pool the launch stores to: a copy of it
+    is what the kernel reads (the pointers that reach the library say so), and
+    the result is that of the values as they were."""
+    from latentserve_amd import _lib
+    from latentserve_amd.kernels.hip import int8_write as iw
+    h, n, nb, nr = 2, 37, 4, 4
+    g = torch.Generator(device="cuda").manual_seed(first)
+    # (the buffer: 16 rows, then the residual pool; the chunk starts at row `first`)
+    buf = torch.randn((nr + 1) * BS, h, 128, generator=g, device="cuda").half()
+    other = torch.randn(1, h, n, 128, generator=g, device="cuda").half()
+    real, seen = _lib.lib(), []
+
+    class Library:
+        def __getattr__(self, name):
+            def call(*args):
+                seen.append((args[0], args[2]))
+                return getattr(real, name)(*args)
+            return call
+
+    def run(apart):
+        buf_ = buf.clone()
+        chunk, res = buf_[first:first + n].transpose(0, 1)[None], buf_[BS:].view(nr, BS, h, 128)
+        if apart:
+            chunk = chunk.clone()
+        k, v = (chunk, other) if which == "k" else (other, chunk)
+        pool = lambda *shape, dtype=torch.float32: torch.zeros(*shape, dtype=dtype, device="cuda")
+        out = [pool(nb, BS, h, 128, dtype=torch.int8), pool(nb, h, 128), None,
+               pool(nb, BS, h, 128, dtype=torch.int8), pool(nb, BS, h), None, res]
+        quant = (1e-8, 127.0, 255.0, 128.0)
+        iw.prefill_write(k, v, torch.arange(5, 5 + n, device="cuda").view(1, n),
+                         torch.ones(1, dtype=torch.long, device="cuda"), *out, asym=False,
+                         k_quant=quant, v_quant=quant)
+        lo, hi = res.data_ptr(), res.data_ptr() + res.numel() * 2
+        return [t for t in out if t is not None], lo, hi
+
+    want, _, _ = run(True)
+    monkeypatch.setattr(_lib, "lib", lambda: Library())
+    got, lo, hi = run(False)
+    assert all(p >= hi or p + n * h * 256 <= lo for p in seen[-1]), "read where it stores"
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
